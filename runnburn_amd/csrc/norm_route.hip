@@ -18,100 +18,184 @@ namespace rnb {
 
 namespace {
 
-constexpr int kNormWaves = 4;
-constexpr int kNormThreads = kWave * kNormWaves;
+constexpr int kNormMaxWaves = 16;
 
-// sum over the workgroup, every thread gets the total; partial sums meet in wave order
+// sum over the wave on the DPP data path, in lane 63 (f64: its two halves move separately)
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ double dpp_add(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), kCtrl, kRowMask, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), kCtrl, kRowMask, 0xf, false);
+    const unsigned long long t = static_cast<unsigned long long>(static_cast<uint32_t>(hi)) << 32 | static_cast<uint32_t>(lo);
+    return v + __builtin_bit_cast(double, t);
+}
+__device__ __forceinline__ double row16_sum(double v) {  // every lane of an aligned 16 gets the sum
+    v = dpp_add<0xB1, 0xf>(v);
+    v = dpp_add<0x4E, 0xf>(v);
+    v = dpp_add<0x141, 0xf>(v);
+    return dpp_add<0x140, 0xf>(v);
+}
+__device__ __forceinline__ float row16_sum(float v) { return seg_sum<16>(v); }
+__device__ __forceinline__ double wave_sum63(double v) { return dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(row16_sum(v))); }
+__device__ __forceinline__ float wave_sum63(float v) { return seg_sum<64>(v); }
+
+// sum over the workgroup's `waves` waves, every thread gets the total; s_part holds kNormMaxWaves zeros before its first
+// use (slots of absent waves stay zero) and one slot array serves one call
 template <typename T>
 __device__ __forceinline__ T wg_sum(T v, T *s_part) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-    const int wave = threadIdx.x >> 6;
-    __syncthreads();  // s_part may still be read from an earlier call
-    if ((threadIdx.x & 63) == 0) s_part[wave] = v;
+    const T total = wave_sum63(v);
+    if ((threadIdx.x & 63) == 63) s_part[threadIdx.x >> 6] = total;
     __syncthreads();
-    T total = s_part[0];
-#pragma unroll
-    for (int w = 1; w < kNormWaves; w++) total += s_part[w];
-    return total;
+    return row16_sum(s_part[threadIdx.x & 15]);
 }
 
-// rms of one row of `nb` 256-element blocks: wave w of the workgroup owns blocks w, w + 4, ..., lane l the elements
-// 4l .. 4l+3 of a block
+// what the mean square is summed in: f64, or f32 for the unit-offset form
 template <bool kUnit>
-__device__ __forceinline__ float row_rms(const float *__restrict__ x, uint32_t nb, float eps, double *s_d, float *s_f) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+struct NormSum {
+    typedef double type;
+};
+template <>
+struct NormSum<true> {
+    typedef float type;
+};
+template <bool kUnit>
+__device__ __forceinline__ void add_squares(typename NormSum<kUnit>::type &acc, const float4 v) {
+    typedef typename NormSum<kUnit>::type T;
+    acc += static_cast<T>(v.x) * static_cast<T>(v.x);
+    acc += static_cast<T>(v.y) * static_cast<T>(v.y);
+    acc += static_cast<T>(v.z) * static_cast<T>(v.z);
+    acc += static_cast<T>(v.w) * static_cast<T>(v.w);
+}
+template <bool kUnit>
+__device__ __forceinline__ float rms_of(typename NormSum<kUnit>::type acc, uint32_t nb, float eps, typename NormSum<kUnit>::type *s_part) {
     const float n = static_cast<float>(nb) * 256.0f;
-    if constexpr (kUnit) {
-        float acc = 0.0f;
-        for (uint32_t b = wave; b < nb; b += kNormWaves) {
-            const float4 v = reinterpret_cast<const float4 *>(x + static_cast<size_t>(b) * 256)[lane];
-            acc += v.x * v.x;
-            acc += v.y * v.y;
-            acc += v.z * v.z;
-            acc += v.w * v.w;
-        }
-        const float mean = wg_sum<float>(acc, s_f) / n;
-        return sqrtf(mean + eps);
-    } else {
-        double acc = 0.0;
-        for (uint32_t b = wave; b < nb; b += kNormWaves) {
-            const float4 v = reinterpret_cast<const float4 *>(x + static_cast<size_t>(b) * 256)[lane];
-            acc += static_cast<double>(v.x) * static_cast<double>(v.x);
-            acc += static_cast<double>(v.y) * static_cast<double>(v.y);
-            acc += static_cast<double>(v.z) * static_cast<double>(v.z);
-            acc += static_cast<double>(v.w) * static_cast<double>(v.w);
-        }
-        const double mean = wg_sum<double>(acc, s_d) / static_cast<double>(n);
-        return static_cast<float>(sqrt(mean + static_cast<double>(eps)));
-    }
+    if constexpr (kUnit)
+        return sqrtf(wg_sum<float>(acc, s_part) / n + eps);
+    else
+        return static_cast<float>(sqrt(wg_sum<double>(acc, s_part) / static_cast<double>(n) + static_cast<double>(eps)));
 }
 
 template <bool kUnit>
-__device__ __forceinline__ float4 scale_of(const float *__restrict__ weight, uint32_t b, int lane) {
-    float4 w = reinterpret_cast<const float4 *>(weight + static_cast<size_t>(b) * 256)[lane];
+__device__ __forceinline__ float4 unit_scale(float4 w) {
     if constexpr (kUnit) w = make_float4(1.0f + w.x, 1.0f + w.y, 1.0f + w.z, 1.0f + w.w);
     return w;
 }
 
-// One workgroup per token row.  kAdd: residual += norm(input, post_weight) first, then the row that is normalised with
-// `weight` is the new residual; else it is `input`.  out_f32 and the Q8_K outputs are optional (null).
-template <bool kAdd, bool kUnitPost, bool kUnit>
-__global__ void __launch_bounds__(kNormThreads)
+// One workgroup per token row; wave w owns the 256-element blocks w, w + waves, ... of the row, lane l the elements
+// 4l .. 4l+3 of a block.  kAdd: residual += norm(input, post_weight) first, then the row that is normalised with `weight`
+// is the new residual; else it is `input`.  out_f32 and the Q8_K outputs are optional (null).
+//
+// A row is a few KB, so the kernel is a chain of latencies: one round trip for everything it reads, a sum across the
+// workgroup per norm, the quantiser.  Hence up to sixteen waves, so that the blocks of a row of up to 4096 elements run side
+// by side, and kPer > 0: a wave's kPer blocks of the input, the residual and both weights are requested together in front
+// of the first sum and stay in registers (rows of up to kPer * 16 blocks).  One row of 4096 with the residual add: 9.4 ->
+// 5.2 us (6.1 -> 3.8 us without it, twelve rows 10.0 -> 5.8); with four waves that read the row again for every step each
+// wave went through four blocks and four dependent round trips, and with loads behind `b < nb` (four dword loads and a
+// branch each) sixteen waves took 7.6.  kPer == 0 is the form for longer rows: blocks are read again in each step.
+template <bool kAdd, bool kUnitPost, bool kUnit, int kPer>
+__global__ void __launch_bounds__(kWave * kNormMaxWaves)
     rms_norm_kernel(const float *__restrict__ input, const float *__restrict__ post_weight, float post_eps,
                     float *__restrict__ residual, const float *__restrict__ weight, float eps, uint32_t nb,
                     float *__restrict__ out_f32, int8_t *__restrict__ qs, float *__restrict__ d_out,
                     int16_t *__restrict__ bsums, uint8_t *__restrict__ digits) {
-    __shared__ double s_d[kNormWaves];
-    __shared__ float s_f[kNormWaves];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int kHeld = kPer > 0 ? kPer : 1;
+    __shared__ typename NormSum<kUnitPost>::type s_post[kNormMaxWaves];
+    __shared__ typename NormSum<kUnit>::type s_sum[kNormMaxWaves];
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const size_t row = blockIdx.x, hidden = static_cast<size_t>(nb) * 256;
-    const float *x = input + row * hidden;
-    if constexpr (kAdd) {
-        float *res = residual + row * hidden;
-        const float post_rms = row_rms<kUnitPost>(x, nb, post_eps, s_d, s_f);
-        for (uint32_t b = wave; b < nb; b += kNormWaves) {
-            const float4 v = reinterpret_cast<const float4 *>(x + static_cast<size_t>(b) * 256)[lane];
-            const float4 w = scale_of<kUnitPost>(post_weight, b, lane);
-            float4 r = reinterpret_cast<float4 *>(res + static_cast<size_t>(b) * 256)[lane];
-            r.x += (v.x / post_rms) * w.x;
-            r.y += (v.y / post_rms) * w.y;
-            r.z += (v.z / post_rms) * w.z;
-            r.w += (v.w / post_rms) * w.w;
-            reinterpret_cast<float4 *>(res + static_cast<size_t>(b) * 256)[lane] = r;  // re-read below by the same thread
+    const float4 *x = reinterpret_cast<const float4 *>(input + row * hidden) + lane;
+    const float4 *pw = reinterpret_cast<const float4 *>(post_weight) + lane, *nw = reinterpret_cast<const float4 *>(weight) + lane;
+    float4 *res = kAdd ? reinterpret_cast<float4 *>(residual + row * hidden) + lane : nullptr;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+
+    float4 v[kHeld], w[kHeld];
+    [[maybe_unused]] float4 r[kHeld], p[kHeld];
+    if constexpr (kPer > 0) {
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            const uint32_t b = wave + i * waves;
+            const size_t at = static_cast<size_t>(min(b, nb - 1)) * 64;  // a load in a branch would be four of one dword
+            v[i] = x[at];
+            if constexpr (kAdd) {
+                r[i] = res[at];
+                p[i] = pw[at];
+            }
+            w[i] = nw[at];
         }
-        x = res;
+#pragma unroll
+        for (int i = 1; i < kPer; i++)
+            if (wave + i * waves >= nb) v[i] = zero;  // not in the sums (kPer == 1: a wave per block)
     }
-    const float rms = row_rms<kUnit>(x, nb, eps, s_d, s_f);
-    for (uint32_t b = wave; b < nb; b += kNormWaves) {
-        const float4 v = reinterpret_cast<const float4 *>(x + static_cast<size_t>(b) * 256)[lane];
-        const float4 w = scale_of<kUnit>(weight, b, lane);
-        const float4 o = make_float4((v.x / rms) * w.x, (v.y / rms) * w.y, (v.z / rms) * w.z, (v.w / rms) * w.w);
+    if (threadIdx.x < kNormMaxWaves) {
+        if constexpr (kAdd) s_post[threadIdx.x] = 0;
+        s_sum[threadIdx.x] = 0;
+    }
+    __syncthreads();
+
+    typename NormSum<kUnit>::type acc = 0;
+    if constexpr (kAdd) {
+        typename NormSum<kUnitPost>::type pacc = 0;
+        if constexpr (kPer > 0) {
+#pragma unroll
+            for (int i = 0; i < kPer; i++) add_squares<kUnitPost>(pacc, v[i]);
+        } else {
+            for (uint32_t b = wave; b < nb; b += waves) add_squares<kUnitPost>(pacc, x[static_cast<size_t>(b) * 64]);
+        }
+        const float post_rms = rms_of<kUnitPost>(pacc, nb, post_eps, s_post);
+        auto add = [&](float4 q, const float4 a, const float4 raw) {
+            const float4 s = unit_scale<kUnitPost>(raw);
+            q.x += (a.x / post_rms) * s.x;
+            q.y += (a.y / post_rms) * s.y;
+            q.z += (a.z / post_rms) * s.z;
+            q.w += (a.w / post_rms) * s.w;
+            return q;
+        };
+        if constexpr (kPer > 0) {
+#pragma unroll
+            for (int i = 0; i < kPer; i++) {
+                const uint32_t b = wave + i * waves;
+                v[i] = add(r[i], v[i], p[i]);
+                if (b < nb) {
+                    res[static_cast<size_t>(b) * 64] = v[i];
+                    add_squares<kUnit>(acc, v[i]);
+                }
+            }
+        } else {
+            for (uint32_t b = wave; b < nb; b += waves) {
+                const size_t at = static_cast<size_t>(b) * 64;
+                const float4 q = add(res[at], x[at], pw[at]);
+                res[at] = q;  // read again below by the same thread
+                add_squares<kUnit>(acc, q);
+            }
+            x = res;
+        }
+    } else {
+        if constexpr (kPer > 0) {
+#pragma unroll
+            for (int i = 0; i < kPer; i++) add_squares<kUnit>(acc, v[i]);
+        } else {
+            for (uint32_t b = wave; b < nb; b += waves) add_squares<kUnit>(acc, x[static_cast<size_t>(b) * 64]);
+        }
+    }
+    const float rms = rms_of<kUnit>(acc, nb, eps, s_sum);
+    auto finish = [&](uint32_t b, const float4 a, const float4 raw) {
+        const float4 s = unit_scale<kUnit>(raw);
+        const float4 o = make_float4((a.x / rms) * s.x, (a.y / rms) * s.y, (a.z / rms) * s.z, (a.w / rms) * s.w);
         if (out_f32 != nullptr) reinterpret_cast<float4 *>(out_f32 + row * hidden + static_cast<size_t>(b) * 256)[lane] = o;
         if (qs != nullptr) {
             const size_t blk = row * nb + b;
             q8k_quantize_vals(o, lane, qs + blk * 256, d_out + blk, bsums + blk * 16, digits != nullptr ? digits + blk * 16 : nullptr);
         }
+    };
+    if constexpr (kPer > 0) {
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            const uint32_t b = wave + i * waves;
+            if (b < nb) finish(b, v[i], w[i]);
+        }
+    } else {
+        for (uint32_t b = wave; b < nb; b += waves) finish(b, x[static_cast<size_t>(b) * 64], nw[static_cast<size_t>(b) * 64]);
     }
 }
 
@@ -186,10 +270,23 @@ void launch_rms_norm(const float *input, const float *post_weight, float post_ep
                      const float *weight, float eps, bool unit, uint32_t seq, uint32_t nb, float *out_f32, int8_t *qs,
                      float *d, int16_t *bsums, uint8_t *digits, hipStream_t stream) {
     if (seq == 0 || nb == 0) return;
-    const dim3 grid(seq), block(kNormThreads);
-#define RNB_NORM(ADD, UP, U)                                                                                          \
-    hipLaunchKernelGGL((rms_norm_kernel<ADD, UP, U>), grid, block, 0, stream, input, post_weight, post_eps, residual, \
+    // rows of up to 16 blocks: a wave per block; up to 64 blocks: sixteen waves with their two or four blocks in registers
+    const uint32_t waves = nb < kNormMaxWaves ? nb : kNormMaxWaves, per = (nb + waves - 1) / waves;
+    const dim3 grid(seq), block(kWave * waves);
+#define RNB_NORM_PER(ADD, UP, U, PER)                                                                                      \
+    hipLaunchKernelGGL((rms_norm_kernel<ADD, UP, U, PER>), grid, block, 0, stream, input, post_weight, post_eps, residual, \
                        weight, eps, nb, out_f32, qs, d, bsums, digits)
+#define RNB_NORM(ADD, UP, U)                  \
+    do {                                      \
+        if (per == 1)                         \
+            RNB_NORM_PER(ADD, UP, U, 1);      \
+        else if (per == 2)                    \
+            RNB_NORM_PER(ADD, UP, U, 2);      \
+        else if (per <= 4)                    \
+            RNB_NORM_PER(ADD, UP, U, 4);      \
+        else                                  \
+            RNB_NORM_PER(ADD, UP, U, 0);      \
+    } while (0)
     if (residual == nullptr) {
         if (unit)
             RNB_NORM(false, false, true);
@@ -206,6 +303,7 @@ void launch_rms_norm(const float *input, const float *post_weight, float post_ep
         else
             RNB_NORM(true, false, false);
     }
+#undef RNB_NORM_PER
 #undef RNB_NORM
 }
 

@@ -95,6 +95,37 @@ def test_rms_norm_add_then_rms_norm_quantize(rnb, oracle, seq, hidden, post_unit
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("seq,blocks", [(1, 1), (2, 15), (1, 16), (3, 17), (1, 32), (2, 33), (1, 64), (2, 65)])
+@pytest.mark.parametrize("unit", [False, True])
+def test_rms_norm_rows_around_the_wave_and_register_limits(rnb, oracle, seq, blocks, unit):
+    """Rows of one block per wave, two, four and beyond (16, 32, 64 blocks are the last of their form), with the residual
+    add.  Bounds: the sum of squares is in another order than the oracle's, f64 moves rms by its last f32 bit at most, f32
+    over n terms by about sqrt(n) * 2^-24 (n = 16640: 8e-6)."""
+    hidden = 256 * blocks
+    rng = np.random.default_rng(40 + blocks)
+    inp, res = rng.standard_normal((2, seq * hidden)).astype(np.float32)
+    pw, qw = (rng.standard_normal((2, hidden)) * 0.3 + 1.0).astype(np.float32)
+    bufs = [rnb.DeviceBuffer.from_host(a) for a in (inp, pw, res, qw)]
+    out, quantised = rnb.DeviceBuffer(seq * hidden * 4), rnb.DeviceBuffer(seq * 64 * 4)
+    rel = 8e-6 if unit else 3e-7
+    rnb.rms_norm_add_rms_norm_quantize_dev(bufs[0], bufs[1], 1e-6, bufs[2], bufs[3], 1e-5, seq, hidden, out,
+                                           post_unit_offset=unit, pre_unit_offset=unit)
+    wq = rnb.DeviceBuffer.from_host(oracle.make_weights(Q4_K, 64, hidden, 9))
+    rnb.gemv_quantized_dev(Q4_K, wq, 64, hidden, seq, quantised)
+    rnb.sync()
+    got_res, got_out, got_q = bufs[2].to_host(np.float32), out.to_host(np.float32), quantised.to_host(np.float32)
+    normed = oracle.rms_norm(inp, pw, 1e-6, unit_offset=unit).ravel()
+    assert np.all(np.abs(got_res.astype(np.float64) - (res + normed)) <= 4 * rel * (np.abs(res) + np.abs(normed)) + 1e-12)
+    assert _close(got_out, oracle.rms_norm(got_res, qw, 1e-5, unit_offset=unit), rel)
+    rnb.quantize_dev(Q4_K, out, seq, hidden)
+    rnb.gemv_quantized_dev(Q4_K, wq, 64, hidden, seq, quantised)
+    rnb.sync()
+    assert np.array_equal(quantised.to_host(np.float32).view(np.uint32), got_q.view(np.uint32))
+    for buf in bufs + [out, quantised, wq]:
+        buf.free()
+
+
+@pytest.mark.gpu
 def test_rms_norm_rejects_bad_shapes(rnb):
     x = rnb.DeviceBuffer(4096)
     with pytest.raises(rnb.BackendError) as err:
