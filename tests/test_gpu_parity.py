@@ -560,6 +560,39 @@ def test_gemm_k_slices(rnb, oracle, quant, rows, nblk, seq):
     assert np.array_equal(rev[::-1], got)
 
 
+@pytest.mark.parametrize("quant,rows,nblk,seq", [(Q6_K, 8451, 11, 97), (Q6_K, 2111, 56, 75), (Q6_K, 40000, 7, 33),
+                                                 (Q5_K, 16385, 17, 71), (Q5_K, 4071, 40, 130), (Q4_K, 16500, 16, 273),
+                                                 (Q4_K, 8500, 25, 333), (Q4_K, 16385, 9, 491)])
+def test_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
+    """Enough work for the GEMM that makes a super-block's operands once for up to 128 tokens: two, three and four token tiles
+    per workgroup, a last wave of one row, a last group of one token, K slices of unequal length, Q6_K rows of an odd
+    number of blocks (every other one off a 4-byte boundary).  Rows at both ends, around the 32- and 256-row tile edges and
+    spread between against the oracle, the tight bound of the module; extreme scales and codes in three of them; a token's
+    row has the same bits in the reversed batch."""
+    cols = nblk * 256
+    w = oracle.make_weights(quant, rows, cols, 70 + rows).copy()
+    per_row = w.size // rows
+    rng = np.random.default_rng(rows)
+    for row, fill in ((5, 255), (rows - 2, 0), (rows // 2, 127)):  # scales, codes and mins at an end; the f16 scales as they were
+        b = w[row * per_row:(row + 1) * per_row].reshape(nblk, -1)
+        if quant == Q6_K:
+            b[:, :208] = fill
+        else:
+            b[:, 4:] = fill
+    x = oracle.fill_normal(seq * cols, 80 + seq, 1.0).reshape(seq, cols)
+    x[3, 256:512] = 0.0
+    x[7] = 3.0  # every code at an end of its range
+    got = gemv_fn(rnb, quant, True)(w, rows, cols, x)
+    pick = sorted({0, 1, 5, 31, 32, 255, 256, rows // 2, rows - 33, rows - 2, rows - 1, *rng.integers(0, rows, 20).tolist()})
+    ws = np.concatenate([w[r * per_row:(r + 1) * per_row] for r in pick])
+    ref, gold = (oracle.gemv(quant, ws, len(pick), cols, x, gold=g).reshape(seq, len(pick)) for g in (False, True))
+    for i, r in enumerate(pick):
+        check_close(got[:, r], ref[:, i], gold[:, i], f"quant {quant} rows {rows} nblk {nblk} seq {seq} row {r}")
+    rev = gemv_fn(rnb, quant, True)(w, rows, cols, x[::-1].copy())
+    assert np.array_equal(rev[::-1], got)
+    rnb.release(w)
+
+
 @pytest.mark.parametrize("quant", [Q2_K, Q3_K])
 @pytest.mark.parametrize("rows,nblk,seq", [(32, 1, 32), (31, 2, 17), (33, 3, 17), (64, 4, 129), (100, 2, 33), (1, 1, 17),
                                            (257, 5, 40), (129, 1, 65), (640, 3, 600)])
