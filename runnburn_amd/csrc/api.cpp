@@ -256,7 +256,10 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
     float *ws = nullptr;
     if (is_iq_quant(quant)) {
         // importance quants: the matrix-core GEMM for batches, else the GEMV (a pass per group of up to four tokens)
-        if (seq >= kIqGemmMinSeq) {
+        if (gemm_iq_digits_pays(quant, w_dev, rows, cols, seq) && fits(gemm_digits_slice_floats(r, nb, q))) {
+            if (int st = slice_floats(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
+            launch_gemm_iq_digits(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
+        } else if (seq >= kIqGemmMinSeq) {
             if (int st = slice_floats(gemm_iq_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
             launch_gemm_iq_mfma(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
         } else {

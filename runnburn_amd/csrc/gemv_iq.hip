@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "embed_gather.h"
+#include "gemm_digits.h"
 #include "kernels.h"
 #include "mfma_blocks.h"
 
@@ -623,6 +624,143 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same formats in the GEMM of gemm_digits.h (operands made once for up to 128 tokens, scale times code as two int8
+// digits): the lane of K-half k takes elements 16 k .. + 16 of group s.  The signed codes go in as code + 128, `off` takes
+// 128 sc off again.  IQ2_XXS, IQ2_S and IQ3_XXS blocks sit at any even address: their lanes read their own bytes; IQ4_XS
+// rows (136 bytes, a multiple of 8) come through the strip, piece 8 being the block's last sixteen bytes.
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ void iq_digits(const uint32_t (&codes)[4], int scale, v4i &lo, v4i &hi) {
+    const u16x2 sc = splat(static_cast<unsigned short>(scale)), off = splat(static_cast<unsigned short>(128 - 128 * scale));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        int l, h;
+        digits256(codes[i] ^ 0x80808080u, sc, off, l, h);
+        lo[i] = l;
+        hi[i] = h;
+    }
+}
+
+struct IqDirect {
+    static constexpr int kPieces = 1, kInv = 0, kRows = 1, kShift = 8, kDOff = 0;
+    static constexpr bool kMins = false, kDirect = true;
+    __device__ __forceinline__ static uint32_t piece(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) { return 0; }
+    __device__ __forceinline__ static uint32_t block_off(uint32_t) { return 0; }
+    __device__ __forceinline__ void head(const uint8_t *, int, uint32_t) {}
+    __device__ __forceinline__ void fetch(int, const uint8_t *, int) {}
+};
+
+template <>
+struct Rows<kIQ2XXS> : IqDirect {
+    static constexpr int kBytes = kIQ2XXSBytes, kTableBytes = Iq<kIQ2XXS>::kTableBytes;
+    static constexpr float kD = 0.125f;
+    static __device__ __forceinline__ const void *table() { return Iq<kIQ2XXS>::table(); }
+    uint32_t w[16];
+    __device__ __forceinline__ void load(const uint8_t *blk, int) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint4 v = ld_u4_a2(blk + 2 + 16 * i);
+            w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
+        }
+    }
+    __device__ __forceinline__ void operand(int s, int khalf, const void *tab, v4i &lo, v4i &hi) {
+        const uint32_t idx = w[2 * s] >> (16 * khalf), ss = w[2 * s + 1], seven = ss >> (14 * khalf);
+        uint32_t codes[4];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const uint64_t grid = static_cast<const uint64_t *>(tab)[(idx >> (8 * e)) & 0xffu];
+            const uint32_t sg = sign_byte(seven >> (7 * e));
+            codes[2 * e] = apply_signs4(static_cast<uint32_t>(grid), sg);
+            codes[2 * e + 1] = apply_signs4(static_cast<uint32_t>(grid >> 32), sg >> 4);
+        }
+        iq_digits(codes, static_cast<int>(2 * (ss >> 28) + 1), lo, hi);
+    }
+};
+
+template <>
+struct Rows<kIQ2S> : IqDirect {
+    static constexpr int kBytes = kIQ2SBytes, kTableBytes = Iq<kIQ2S>::kTableBytes;
+    static constexpr float kD = 0.125f;
+    static __device__ __forceinline__ const void *table() { return Iq<kIQ2S>::table(); }
+    uint32_t w[20];
+    __device__ __forceinline__ void load(const uint8_t *blk, int) {
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            const uint4 v = ld_u4_a2(blk + 2 + 16 * i);
+            w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
+        }
+    }
+    __device__ __forceinline__ void operand(int s, int khalf, const void *tab, v4i &lo, v4i &hi) {
+        const uint32_t idx = w[s] >> (16 * khalf), signs = w[8 + s] >> (16 * khalf);
+        const uint32_t qh = (w[16 + (s >> 2)] >> (8 * (s & 3) + 4 * khalf)) & 15u;
+        const uint32_t sc = (w[18 + (s >> 2)] >> (8 * (s & 3) + 4 * khalf)) & 15u;
+        uint32_t codes[4];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const uint64_t grid = static_cast<const uint64_t *>(tab)[((idx >> (8 * e)) & 0xffu) | ((qh << (8 - 2 * e)) & 0x300u)];
+            const uint32_t sg = (signs >> (8 * e)) & 0xffu;
+            codes[2 * e] = apply_signs4(static_cast<uint32_t>(grid), sg);
+            codes[2 * e + 1] = apply_signs4(static_cast<uint32_t>(grid >> 32), sg >> 4);
+        }
+        iq_digits(codes, static_cast<int>(2 * sc + 1), lo, hi);
+    }
+};
+
+template <>
+struct Rows<kIQ3XXS> : IqDirect {
+    static constexpr int kBytes = kIQ3XXSBytes, kTableBytes = Iq<kIQ3XXS>::kTableBytes;
+    static constexpr float kD = 0.25f;
+    static __device__ __forceinline__ const void *table() { return Iq<kIQ3XXS>::table(); }
+    uint32_t idx[8], ss[8];  // the K-half's four indices of every group; signs and scale
+    __device__ __forceinline__ void load(const uint8_t *blk, int khalf) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) idx[i] = ld_u32_a2(blk + 2 + 8 * i + 4 * khalf);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint4 v = ld_u4_a2(blk + 66 + 16 * i);
+            ss[4 * i] = v.x, ss[4 * i + 1] = v.y, ss[4 * i + 2] = v.z, ss[4 * i + 3] = v.w;
+        }
+    }
+    __device__ __forceinline__ void operand(int s, int khalf, const void *tab, v4i &lo, v4i &hi) {
+        const uint32_t *grid = static_cast<const uint32_t *>(tab);
+        const uint32_t seven = ss[s] >> (14 * khalf);
+        uint32_t codes[4];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const uint32_t sg = sign_byte(seven >> (7 * e));
+            codes[2 * e] = apply_signs4(grid[(idx[s] >> (16 * e)) & 0xffu], sg);
+            codes[2 * e + 1] = apply_signs4(grid[(idx[s] >> (16 * e + 8)) & 0xffu], sg >> 4);
+        }
+        iq_digits(codes, static_cast<int>(2 * (ss[s] >> 28) + 1), lo, hi);
+    }
+};
+
+template <>
+struct Rows<kIQ4XS> {
+    static constexpr int kBytes = kIQ4XSBytes, kPieces = 9, kInv = 7282, kRows = 7, kShift = 8, kTableBytes = 0, kDOff = 0;
+    static constexpr float kD = 1.0f;
+    static constexpr bool kMins = false, kDirect = false;
+    uint2 hdr, raw[2];
+    __device__ __forceinline__ static uint32_t piece(uint32_t r, uint32_t j, uint32_t row_bytes, uint32_t, uint32_t) {
+        return r * row_bytes + (j < 8 ? 16 * j : 120);
+    }
+    __device__ __forceinline__ static uint32_t block_off(uint32_t b) { return b * kBytes; }
+    __device__ __forceinline__ void head(const uint8_t *row, int, uint32_t) { hdr = *reinterpret_cast<const uint2 *>(row); }
+    __device__ __forceinline__ void fetch(int s, const uint8_t *row, int) {
+        const uint8_t *p = row + (s < 7 ? 8 + 16 * s : 128);
+        raw[0] = *reinterpret_cast<const uint2 *>(p);
+        raw[1] = *reinterpret_cast<const uint2 *>(p + 8);
+    }
+    __device__ __forceinline__ void operand(int s, int khalf, const void *, v4i &lo, v4i &hi) {
+        const int scale = static_cast<int>(((hdr.y >> (4 * s)) & 15u) | (((hdr.x >> (16 + 2 * s)) & 3u) << 4)) - 32;
+        const uint32_t q[4] = {raw[0].x, raw[0].y, raw[1].x, raw[1].y};
+        uint32_t codes[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) codes[i] = iq4nl_lookup((q[i] >> (4 * khalf)) & 0x0f0f0f0fu);
+        iq_digits(codes, scale, lo, hi);
+    }
+};
+
 // the tiling and slicing choices, shared by the launcher and the workspace size
 struct IqGemmPlan {
     bool wide;  // 64-token workgroups
@@ -668,6 +806,26 @@ void launch_gemv_iq(const uint8_t *w, uint32_t quant, ActView act, float *out, u
     case kIQ2S: launch_iq<kIQ2S>(w, act, out, rows, nb, seq, stream); break;
     case kIQ3XXS: launch_iq<kIQ3XXS>(w, act, out, rows, nb, seq, stream); break;
     default: launch_iq<kIQ4XS>(w, act, out, rows, nb, seq, stream); break;
+    }
+}
+
+// Measured over rows 1111 - 14336, columns 3072 - 14336, 40 - 1322 tokens, us per step: ahead of the 32- / 64-token kernel from
+// 2.2e9 multiply-adds (IQ2_S 14336 x 4096 x 40 tokens 38 -> 33, x 160 83 -> 62, x 512 179 -> 110; 4096 x 14336 x 300 213 ->
+// 102; IQ4_XS 14336 x 4096 x 160 78 -> 57) where its workgroups fill the chip.
+bool gemm_iq_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq) {
+    const double macs = static_cast<double>(rows) * static_cast<double>(cols) * static_cast<double>(seq);
+    return seq > 32 && macs >= 2.2e9 && (quant != kIQ4XS || reinterpret_cast<uintptr_t>(w) % 8 == 0) &&
+           digits_fill_the_chip(static_cast<uint32_t>(rows), static_cast<uint32_t>(cols / 256), static_cast<uint32_t>(seq));
+}
+
+void launch_gemm_iq_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows,
+                           uint32_t nb, uint32_t seq, hipStream_t stream) {
+    if (rows == 0 || seq == 0 || nb == 0) return;
+    switch (quant) {
+    case kIQ2XXS: launch_digits_plan<kIQ2XXS>(w, act, out, slice_out, rows, nb, seq, stream); break;
+    case kIQ2S: launch_digits_plan<kIQ2S>(w, act, out, slice_out, rows, nb, seq, stream); break;
+    case kIQ3XXS: launch_digits_plan<kIQ3XXS>(w, act, out, slice_out, rows, nb, seq, stream); break;
+    default: launch_digits_plan<kIQ4XS>(w, act, out, slice_out, rows, nb, seq, stream); break;
     }
 }
 

@@ -141,6 +141,11 @@ void launch_gemm_q8_mfma(const uint8_t *w, uint32_t quant, ActView act, float *o
 size_t gemm_q4k_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq);
 void launch_gemm_q4k_mfma(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
                           uint32_t seq, hipStream_t stream);
+// the importance quants in the same kernel as launch_gemm_digits (workspace: gemm_digits_slice_floats)
+bool gemm_iq_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq);
+void launch_gemm_iq_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows,
+                           uint32_t nb, uint32_t seq, hipStream_t stream);
+
 // Q4_K, Q5_K and Q6_K batches of more than 32 tokens with the operands made once for up to 128 tokens (act needs digits for
 // Q4_K / Q5_K); workspace for K slices as for the kernels above.  _pays: weights aligned for it and enough work.
 bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq);

@@ -74,6 +74,33 @@ def test_iq_gemm_matrix_cores(rnb, oracle, quant, rows, cols, seq):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("quant", [IQ2_XXS, IQ2_S, IQ3_XXS, IQ4_XS])
+@pytest.mark.parametrize("rows,nblk,seq", [(2111, 56, 75), (49153, 6, 33), (16385, 13, 75), (12545, 3, 510)])
+def test_iq_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
+    """Enough work for the GEMM that makes a block's operands once for up to 128 tokens: two, three and four token tiles per
+    workgroup, K slices, a last wave of one row.  Blocks of random bytes in a third of the rows (every grid index, sign
+    pattern and scale), rows at the tile edges and spread between against the oracle; a token's row has the same bits in
+    the reversed batch."""
+    cols = nblk * 256
+    w = oracle.make_weights(quant, rows, cols, 1700 + quant + rows).copy().reshape(rows, nblk, -1)
+    rng = np.random.default_rng(rows)
+    w[::3, :, 2:] = rng.integers(0, 256, size=w[::3, :, 2:].shape, dtype=np.uint8)
+    w = w.reshape(-1)
+    per_row = w.size // rows
+    x = oracle.fill_normal(seq * cols, 1300 + seq, 1.0).reshape(seq, cols)
+    x[7] = 3.0  # every code at an end of its range
+    got = _fns(rnb, quant)[1](w, rows, cols, x).reshape(seq, rows)
+    pick = sorted({0, 1, 3, 31, 32, 255, 256, rows - 33, rows - 2, rows - 1, *rng.integers(0, rows, 20).tolist()})
+    ws = np.concatenate([w[r * per_row:(r + 1) * per_row] for r in pick])
+    ref, gold = (np.asarray(oracle.gemv(quant, ws, len(pick), cols, x, gold=g)).reshape(seq, len(pick)) for g in (False, True))
+    for i, r in enumerate(pick):
+        _check(got[:, r], ref[:, i], gold[:, i], f"{LABEL[quant]} {rows}x{cols}x{seq} row {r}")
+    rev = _fns(rnb, quant)[1](w, rows, cols, x[::-1].copy()).reshape(seq, rows)
+    assert np.array_equal(rev[::-1], got)
+    rnb.release(w)
+
+
+@pytest.mark.gpu
 def test_iq_gemm_every_code_and_scale(rnb, oracle):
     """Blocks of random bytes (every grid index, sign pattern and scale value) with a finite d, eight tokens."""
     rng = np.random.default_rng(99)
