@@ -718,7 +718,7 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     uint32_t max_group = 0;
     for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
     const MoeGroups groups{d_list + 3 * n_slots, d_list + 3 * n_slots + n_groups, d_list + n_slots, d_list + 2 * n_slots,
-                           static_cast<uint32_t>(n_groups), max_group};
+                           static_cast<uint32_t>(n_groups), max_group, grp_start.data()};
 
     ActView act;
     if (inline_tables) {

@@ -166,6 +166,12 @@ struct MoeGroups {
     const uint32_t *sorted_token;  // [n_slots]
     uint32_t n_groups;
     uint32_t max_group = 32;       // slots of the largest group (host-side knowledge: sizes the matrix-core kernels' LDS)
+    const uint32_t *host_start = nullptr;  // `start` in host memory, for the length of the call
+    uint32_t tiles_of(uint32_t slots) const {  // the groups' slots in tiles of `slots`
+        uint32_t n = 0;
+        for (uint32_t g = 0; g < n_groups; g++) n += (host_start[g + 1] - host_start[g] + slots - 1) / slots;
+        return n;
+    }
 };
 // Q8_K of act(gate[i]) * up[i] (SiLU, or the tanh form of GELU): the gated FFN's intermediate quantised as it is made
 void launch_quantize_q8k_gated(const float *gate, const float *up, size_t n_blocks, bool gelu, int8_t *qs, float *d,

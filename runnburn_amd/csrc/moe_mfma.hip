@@ -48,6 +48,33 @@ __device__ __forceinline__ void tile_map_fill(TileMap &m, const uint32_t *__rest
     }
 }
 
+// Token tile `unit` of the call: the tiles of `toks` slots of group 0, then those of group 1, ...  A call whose groups are one
+// tile each (n_units == n_groups) skips the search; else every wave walks the groups 64 at a time, a group per lane.
+struct TileUnit {
+    uint32_t grp, first;  // group, first slot of the tile in it
+};
+__device__ __forceinline__ TileUnit find_unit(uint32_t unit, uint32_t n_units, const uint32_t *__restrict__ grp_start, uint32_t n_groups,
+                                              uint32_t toks, int lane) {
+    if (n_units == n_groups) return {unit, 0};
+    for (uint32_t g0 = 0;; g0 += kWave) {
+        const uint32_t g = min(g0 + lane, n_groups - 1);
+        const uint32_t mine = g0 + lane < n_groups ? (grp_start[g + 1] - grp_start[g] + toks - 1) / toks : 0;
+        uint32_t end = mine;  // tiles up to and with the lane's group
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const uint32_t below = __shfl_up(end, off, kWave);
+            if (lane >= off) end += below;
+        }
+        const uint64_t past = __ballot(end > unit);
+        if (past != 0) {
+            const int at = __builtin_ctzll(past);
+            return {g0 + at, (unit - __shfl(end - mine, at, kWave)) * toks};
+        }
+        unit -= __shfl(end, kWave - 1, kWave);
+        if (g0 + kWave >= n_groups) return {n_groups - 1, 0xffffffffu};  // not reached: the grid has n_units rows
+    }
+}
+
 // the tile's quantised activations of block b (256 int8 per token, 8-byte chunks), scale and digits
 template <int kThreads>
 struct TileStage {
@@ -316,18 +343,21 @@ __device__ __forceinline__ void tile_image_fill(const TileImage<kStride, kDigits
 }
 
 // ---------------------------------------------------------------------------------------------
-// gate + up + SiLU * up.  Grid (row tiles of 128, expert groups).  The tile's activations are staged once, all blocks;
-// after that the waves run without barriers, each streaming its 32 rows of both matrices one block ahead.  The rows
-// come in by whole cache lines as LDS-direct loads into the wave's two strips (consecutive lanes take consecutive
-// 16-byte pieces of a row, see RowRoute for why; no vector registers hold the data in flight), and each lane reads its
-// row's share back from there.  Dynamic LDS: the four waves' strips, then the tile image.
+// gate + up + SiLU * up.  Grid (row tiles of 32 kW, token tiles of all groups, see find_unit).  A router's groups differ
+// severalfold in size: with one workgroup walking all token tiles of its group the largest group set the time (128 experts x
+// top-8 at 512 tokens, groups of 2 to 172: gate/up 282 -> 92 us, down 218 -> 94; a grid with empty workgroups for the tiles
+// that smaller groups have not: 153; 8 experts x top-2 at 300 tokens, the whole call: 917 -> 190).
+// The tile's activations are staged once, all blocks; after that the waves run without barriers, each streaming its 32 rows
+// of both matrices one block ahead.  The rows come in by whole cache lines as LDS-direct loads into the wave's two strips
+// (consecutive lanes take consecutive 16-byte pieces of a row, see RowRoute for why; no vector registers hold the data in
+// flight), and each lane reads its row's share back from there.  Dynamic LDS: the waves' strips, then the tile image.
 // ---------------------------------------------------------------------------------------------
 template <int kJ, int kW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * kW), amdgpu_waves_per_eu(2)))
     moe_gate_up_mfma_kernel(const uint8_t *__restrict__ gate_all, const uint8_t *__restrict__ up_all,
                             const uint8_t *__restrict__ gate_shared, const uint8_t *__restrict__ up_shared, uint32_t n_routed,
                             const int8_t *__restrict__ aq, const float *__restrict__ ad, const uint8_t *__restrict__ adig,
-                            const uint32_t *__restrict__ grp_expert, const uint32_t *__restrict__ grp_start,
+                            const uint32_t *__restrict__ grp_expert, const uint32_t *__restrict__ grp_start, uint32_t n_groups,
                             const uint32_t *__restrict__ sorted_slot, const uint32_t *__restrict__ sorted_token,
                             float *__restrict__ mid, uint32_t n_ff, uint32_t nb, uint32_t img_toks, uint32_t tiles_per_wg) {
     constexpr bool kFifth = false;
@@ -341,8 +371,10 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
     const int lrow = lane & 31, khalf = lane >> 5;
     uint8_t *strips = s_dyn + wave * kPair;
     const uint32_t lds_strips = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)strips));
-    const uint32_t grp = blockIdx.y;
+    const TileUnit unit = find_unit(blockIdx.y, gridDim.y, grp_start, n_groups, img_toks, lane);
+    const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
     const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
+    if (tile0 >= count) return;
     const uint32_t row_bytes = nb * static_cast<uint32_t>(kQ4KBytes);
     const size_t per_expert = static_cast<size_t>(n_ff) * row_bytes;
     const uint8_t *gate_e = expert_base(gate_all, gate_shared, n_routed, expert, per_expert),
@@ -396,70 +428,67 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
         q4_row_from_strip(u, strips + kQ4FillBytes + lrow * kQ4StripStride, khalf);
     };
 
-    for (uint32_t tile0 = 0; tile0 < count; tile0 += img_toks) {
-        // the first weight blocks do not depend on the token lists: requested before them
-        req_b = req_rt = 0;
-        set_tile(0);
-        request();
-        const uint32_t live = min(count - tile0, img_toks);
-        const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);  // padding lanes read the last live row
-        if (tile0) __syncthreads();  // the previous tile's readers of the map and the image are done
-        tile_map_fill(s_map, sorted_token, sorted_slot, nullptr, start + tile0, live, tid);
-        __syncthreads();
-        tile_image_fill<kWave * kW>(img, s_map, aq, ad, adig, tid, live);
-        Q5Row cg, cu;
-        take(cg, cu);
-        __syncthreads();
-        // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
-        auto walk = [&](auto jtag) {
-            constexpr int kJl = decltype(jtag)::value;
-            for (uint32_t rt = 0; rt < rt_n; rt++) {
-                const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
-                float accg[4 * kJl], accu[4 * kJl];
+    // the first weight blocks do not depend on the token lists: requested before them
+    set_tile(0);
+    request();
+    const uint32_t live = min(count - tile0, img_toks);
+    const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);  // padding lanes read the last live row
+    tile_map_fill(s_map, sorted_token, sorted_slot, nullptr, start + tile0, live, tid);
+    __syncthreads();
+    tile_image_fill<kWave * kW>(img, s_map, aq, ad, adig, tid, live);
+    Q5Row cg, cu;
+    take(cg, cu);
+    __syncthreads();
+    // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
+    auto walk = [&](auto jtag) {
+        constexpr int kJl = decltype(jtag)::value;
+        for (uint32_t rt = 0; rt < rt_n; rt++) {
+            const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
+            float accg[4 * kJl], accu[4 * kJl];
 #pragma unroll
-                for (int i = 0; i < 4 * kJl; i++) accg[i] = accu[i] = 0.0f;
-                for (uint32_t b = 0; b < nb; b++) {
-                    request();  // the step after this one
-                    const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
-                    const uint4 dig = img.dig(b)[lrow];
-                    float val[4 * kJl];
-                    TileOps128 aops;
-                    tile_ops_load(aops, abase);
-                    q45_block_tile<kFifth, kJl>(cg, aops, dig, khalf, val);
-                    tile_scale_add<kJl>(img.dx(b), khalf, val, accg);
-                    q45_block_tile<kFifth, kJl>(cu, aops, dig, khalf, val);
-                    tile_scale_add<kJl>(img.dx(b), khalf, val, accu);
-                    take(cg, cu);  // (after the last step: a repeat of it, unused)
-                }
-                if (row < n_ff) {
+            for (int i = 0; i < 4 * kJl; i++) accg[i] = accu[i] = 0.0f;
+            for (uint32_t b = 0; b < nb; b++) {
+                request();  // the step after this one
+                const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
+                const uint4 dig = img.dig(b)[lrow];
+                float val[4 * kJl];
+                TileOps128 aops;
+                tile_ops_load(aops, abase);
+                q45_block_tile<kFifth, kJl>(cg, aops, dig, khalf, val);
+                tile_scale_add<kJl>(img.dx(b), khalf, val, accg);
+                q45_block_tile<kFifth, kJl>(cu, aops, dig, khalf, val);
+                tile_scale_add<kJl>(img.dx(b), khalf, val, accu);
+                take(cg, cu);  // (after the last step: a repeat of it, unused)
+            }
+            if (row < n_ff) {
 #pragma unroll
-                    for (int r = 0; r < 4 * kJl; r++) {
-                        const uint32_t slot = s_map.out_row[8 * (r >> 2) + 4 * khalf + (r & 3)];
-                        if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
-                    }
+                for (int r = 0; r < 4 * kJl; r++) {
+                    const uint32_t slot = s_map.out_row[8 * (r >> 2) + 4 * khalf + (r & 3)];
+                    if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
                 }
             }
-        };
-        if constexpr (kJ == 2) {  // (the 32-token kernel keeps its one form: its groups are large)
-            if (live <= 8)  // workgroup-uniform
-                walk(std::integral_constant<int, 1>{});
-            else
-                walk(std::integral_constant<int, 2>{});
-        } else {
-            walk(std::integral_constant<int, kJ>{});
         }
+    };
+    if constexpr (kJ == 2) {  // (the 32-token kernel keeps its one form: its groups are large)
+        if (live <= 8)  // workgroup-uniform
+            walk(std::integral_constant<int, 1>{});
+        else
+            walk(std::integral_constant<int, 2>{});
+    } else {
+        walk(std::integral_constant<int, kJ>{});
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// down projection of the re-quantised intermediate, scaled by the route weight.  Grid (row tiles of 128, expert groups).
+// down projection of the re-quantised intermediate, scaled by the route weight.  Grid (row tiles of 128, token tiles of all
+// groups).
 // ---------------------------------------------------------------------------------------------
 template <uint32_t kQuant, int kJ>
 __global__ void __launch_bounds__(kGbThreads, 2)
     moe_down_mfma_kernel(const uint8_t *__restrict__ down_all, const uint8_t *__restrict__ down_shared, uint32_t n_routed,
                          const float *__restrict__ mid,
                          const uint32_t *__restrict__ grp_expert,
-                         const uint32_t *__restrict__ grp_start, const uint32_t *__restrict__ sorted_slot,
+                         const uint32_t *__restrict__ grp_start, uint32_t n_groups, const uint32_t *__restrict__ sorted_slot,
                          const float *__restrict__ slot_route, float *__restrict__ slot_out, uint32_t n_embd, uint32_t nb,
                          uint32_t tiles_per_wg, uint32_t img_toks) {
     constexpr bool kSix = kQuant == kQ6K;
@@ -473,8 +502,10 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: the wave's row addresses are scalar bases plus lane offsets
     const int lrow = lane & 31, khalf = lane >> 5;
-    const uint32_t grp = blockIdx.y;
+    const TileUnit unit = find_unit(blockIdx.y, gridDim.y, grp_start, n_groups, img_toks, lane);
+    const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
     const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
+    if (tile0 >= count) return;
     const size_t row_bytes = static_cast<size_t>(nb) * kBlockBytes;
     const uint8_t *down_e = expert_base(down_all, down_shared, n_routed, expert, n_embd * row_bytes);
     // The workgroup walks tiles_per_wg row tiles of 128 against one staged token tile: map and image are made once,
@@ -508,108 +539,105 @@ __global__ void __launch_bounds__(kGbThreads, 2)
         r.d = d_next;
     };
 
-    for (uint32_t tile0 = 0; tile0 < count; tile0 += img_toks) {
-        Q6Row c6{};
-        Q5Row c5{};
-        // the first weight block does not depend on the token lists: requested before them
-        if constexpr (kSix)
-            q6_request(0, 0);
-        else
-            c5 = q45_load_row<kFifth>(block_ptr(0, 0), khalf);
-        if (tile0) __syncthreads();
-        const uint32_t live = min(count - tile0, img_toks);
-        const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);
-        tile_map_fill(s_map, sorted_slot, sorted_slot, slot_route, start + tile0, live, tid);
-        __syncthreads();
-        // the tile's slots' intermediates (f32, [slot][nb * 256]) are quantised to Q8_K as they are staged, with the
-        // stand-alone quantiser's wave-level routine (the same bits): wave w takes (token, block) pairs w, w + 4, ...,
-        // four loads in flight.  The workgroups of a group's other row tiles repeat this; it is a few blocks each.
-        {
-            const uint32_t pairs = live * nb;
-            for (uint32_t p0 = wave; p0 < pairs; p0 += 4 * kGbWaves) {
-                float4 v[4];
+    Q6Row c6{};
+    Q5Row c5{};
+    // the first weight block does not depend on the token lists: requested before them
+    if constexpr (kSix)
+        q6_request(0, 0);
+    else
+        c5 = q45_load_row<kFifth>(block_ptr(0, 0), khalf);
+    const uint32_t live = min(count - tile0, img_toks);
+    const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);
+    tile_map_fill(s_map, sorted_slot, sorted_slot, slot_route, start + tile0, live, tid);
+    __syncthreads();
+    // the tile's slots' intermediates (f32, [slot][nb * 256]) are quantised to Q8_K as they are staged, with the
+    // stand-alone quantiser's wave-level routine (the same bits): wave w takes (token, block) pairs w, w + 4, ...,
+    // four loads in flight.  The workgroups of a group's other row tiles repeat this; it is a few blocks each.
+    {
+        const uint32_t pairs = live * nb;
+        for (uint32_t p0 = wave; p0 < pairs; p0 += 4 * kGbWaves) {
+            float4 v[4];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const uint32_t p = p0 + k * kGbWaves;
-                    v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (p < pairs) {
-                        const uint32_t t = p / nb, b = p - t * nb;
-                        v[k] = reinterpret_cast<const float4 *>(mid + (static_cast<size_t>(s_map.act_row[t]) * nb + b) * 256)[lane];
-                    }
+            for (int k = 0; k < 4; k++) {
+                const uint32_t p = p0 + k * kGbWaves;
+                v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (p < pairs) {
+                    const uint32_t t = p / nb, b = p - t * nb;
+                    v[k] = reinterpret_cast<const float4 *>(mid + (static_cast<size_t>(s_map.act_row[t]) * nb + b) * 256)[lane];
                 }
+            }
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const uint32_t p = p0 + k * kGbWaves;
-                    if (p < pairs) {  // wave-uniform
-                        const uint32_t t = p / nb, b = p - t * nb;
-                        q8k_quantize_vals(v[k], lane, reinterpret_cast<int8_t *>(img.act(b) + t * kStride), &img.dx(b)[t], s_bsums[wave],
-                                          kSix ? nullptr : reinterpret_cast<uint8_t *>(&img.dig(b)[t]));
-                    }
+            for (int k = 0; k < 4; k++) {
+                const uint32_t p = p0 + k * kGbWaves;
+                if (p < pairs) {  // wave-uniform
+                    const uint32_t t = p / nb, b = p - t * nb;
+                    q8k_quantize_vals(v[k], lane, reinterpret_cast<int8_t *>(img.act(b) + t * kStride), &img.dx(b)[t], s_bsums[wave],
+                                      kSix ? nullptr : reinterpret_cast<uint8_t *>(&img.dig(b)[t]));
                 }
             }
         }
-        if constexpr (kSix) q6_take(c6);
-        __syncthreads();
-        // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
-        auto walk = [&](auto jtag) {
-        constexpr int kJl = decltype(jtag)::value;
-        float accf[4 * kJl];
+    }
+    if constexpr (kSix) q6_take(c6);
+    __syncthreads();
+    // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
+    auto walk = [&](auto jtag) {
+    constexpr int kJl = decltype(jtag)::value;
+    float accf[4 * kJl];
 #pragma unroll
-        for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
-        uint32_t rt = 0, b = 0;
-        for (uint32_t s = 0; s < steps; s++) {
-            uint32_t rtn = rt, bn = b + 1;  // the step after this one; the last step reloads its own block, unused
-            if (bn == nb) {
-                bn = 0;
-                rtn = rt + 1;
-            }
-            if (s + 1 == steps) {
-                rtn = rt;
-                bn = b;
-            }
-            Q5Row n5{};
-            float val[4 * kJl];
-            if constexpr (kSix) {
-                q6_request(rtn, bn);
-                TileOps64 aops;
-                tile_ops_load(aops, img.act(b) + arow * kStride + 8 * khalf);
-                q6_block_tile<kJl>(c6, aops, val);
-            } else {
-                n5 = q45_load_row<kFifth>(block_ptr(rtn, bn), khalf);
-                TileOps128 aops;
-                tile_ops_load(aops, img.act(b) + arow * kStride + 16 * khalf);
-                q45_block_tile<kFifth, kJl>(c5, aops, img.dig(b)[lrow], khalf, val);
-            }
-            tile_scale_add<kJl>(img.dx(b), khalf, val, accf);
-            if constexpr (kSix) q6_take(c6);
-            c5 = n5;
-            if (b + 1 == nb) {  // the row tile is complete
-                const uint32_t row = row_of(rt);
-                if (row < n_embd) {
-#pragma unroll
-                    for (int r = 0; r < 4 * kJl; r++) {
-                        const int t = 8 * (r >> 2) + 4 * khalf + (r & 3);
-                        const uint32_t slot = s_map.out_row[t];
-                        // fanout.rs:306-308: the expert's output times the slot's route weight
-                        if (slot != 0xffffffffu)
-                            slot_out[static_cast<size_t>(slot) * n_embd + row] = accf[r] * s_map.scale[t];
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
-            }
-            rt = rtn;
-            b = bn;
+    for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
+    uint32_t rt = 0, b = 0;
+    for (uint32_t s = 0; s < steps; s++) {
+        uint32_t rtn = rt, bn = b + 1;  // the step after this one; the last step reloads its own block, unused
+        if (bn == nb) {
+            bn = 0;
+            rtn = rt + 1;
         }
-        };
-        if constexpr (kJ == 2) {
-            if (live <= 8)  // workgroup-uniform
-                walk(std::integral_constant<int, 1>{});
-            else
-                walk(std::integral_constant<int, 2>{});
+        if (s + 1 == steps) {
+            rtn = rt;
+            bn = b;
+        }
+        Q5Row n5{};
+        float val[4 * kJl];
+        if constexpr (kSix) {
+            q6_request(rtn, bn);
+            TileOps64 aops;
+            tile_ops_load(aops, img.act(b) + arow * kStride + 8 * khalf);
+            q6_block_tile<kJl>(c6, aops, val);
         } else {
-            walk(std::integral_constant<int, kJ>{});
+            n5 = q45_load_row<kFifth>(block_ptr(rtn, bn), khalf);
+            TileOps128 aops;
+            tile_ops_load(aops, img.act(b) + arow * kStride + 16 * khalf);
+            q45_block_tile<kFifth, kJl>(c5, aops, img.dig(b)[lrow], khalf, val);
         }
+        tile_scale_add<kJl>(img.dx(b), khalf, val, accf);
+        if constexpr (kSix) q6_take(c6);
+        c5 = n5;
+        if (b + 1 == nb) {  // the row tile is complete
+            const uint32_t row = row_of(rt);
+            if (row < n_embd) {
+#pragma unroll
+                for (int r = 0; r < 4 * kJl; r++) {
+                    const int t = 8 * (r >> 2) + 4 * khalf + (r & 3);
+                    const uint32_t slot = s_map.out_row[t];
+                    // fanout.rs:306-308: the expert's output times the slot's route weight
+                    if (slot != 0xffffffffu)
+                        slot_out[static_cast<size_t>(slot) * n_embd + row] = accf[r] * s_map.scale[t];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
+        }
+        rt = rtn;
+        b = bn;
+    }
+    };
+    if constexpr (kJ == 2) {
+        if (live <= 8)  // workgroup-uniform
+            walk(std::integral_constant<int, 1>{});
+        else
+            walk(std::integral_constant<int, 2>{});
+    } else {
+        walk(std::integral_constant<int, kJ>{});
     }
 }
 
@@ -626,6 +654,7 @@ bool allow_lds(K kernel, size_t bytes) {
 // the tile image (all blocks of the tile's tokens) must fit the LDS of a compute unit beside the waves' strips and the
 // small static arrays; a tile holds as many tokens as fit, at most 32
 constexpr size_t kMmLdsLimit = 150 * 1024;
+constexpr size_t kMmLdsWide = 158 * 1024;  // for the eight-wave gate/up kernel (the token map is all it has besides)
 constexpr size_t kMmGateUpImageLimit = kMmLdsLimit - kMmGateUpStripBytes;
 constexpr size_t kMmQ6DownLdsLimit = kMmLdsLimit - kGbWaves * 32 * kQ6StripStride;
 constexpr uint32_t kMmMinToks = 16;  // below this the matrix-core path re-reads the weights too often to pay
@@ -659,9 +688,28 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     // one workgroup per compute unit, map and image made once per walk.  128 experts x top-8 at 64 tokens (126 groups):
     // four waves 1 / 2 / 3 tiles per workgroup 55.4 / 58.4 / 50.6 us (2 leaves half the units with two workgroups and
     // half with one), six waves x 2 tiles 48.8 us, eight waves x 1 (two rounds) 61.6, twelve waves 67-74.
+    const uint32_t units = groups.tiles_of(toks);
     int waves = kGbWaves;
     uint32_t tiles_per_wg = 1;
+    const bool many = units > groups.n_groups;  // groups of more than a tile
+    if (many) {
+        // Whole tiles: the image and a strip pair per wave leave one workgroup per compute unit; eight waves (two per SIMD)
+        // where they fit.  Row tiles are merged for the least of rounds * (steps + about two for the setup); a step of eight
+        // waves takes a little longer than one of four.  (Four waves at 512 tokens 220 us a call against 198; with one tile a
+        // group the rule below is ahead, 64 tokens 114 against 120.)
+        uint64_t best = ~0ull;
+        for (const int w : {8, 4}) {
+            if (w == 8 && 8 * 2 * kQ4FillBytes + image > kMmLdsWide) continue;
+            const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
+            for (uint32_t t = 1; t <= tiles && t <= 8; t++) {
+                const uint64_t wgs = static_cast<uint64_t>(units) * ((tiles + t - 1) / t);
+                const uint64_t cost = (wgs + 255) / 256 * (t * nb_in + 2) * (w == 8 ? 9 : 8);
+                if (cost < best) best = cost, waves = w, tiles_per_wg = t;
+            }
+        }
+    }
     for (const int w : {6, 4}) {
+        if (many) break;
         if (w != kGbWaves && (toks > 16 || static_cast<size_t>(w) * 2 * kQ4FillBytes + image > kMmLdsLimit)) continue;
         const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
         const uint32_t t = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * groups.n_groups + 255) / 256);
@@ -674,14 +722,16 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     }
     const size_t lds = static_cast<size_t>(waves) * 2 * kQ4FillBytes + image;
     const uint32_t rows_per_wg = 32 * waves, row_tiles = (n_ff + rows_per_wg - 1) / rows_per_wg;
-    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, groups.n_groups, 1);
+    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, units, 1);
     // tiles of at most 8 / 16 / 32 tokens: the kernel finishes only that many results per lane
 #define RNB_LAUNCH_GUW(J, W)                                                                                          \
-    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, kMmLdsLimit)) return;                                   \
+    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, W == 8 ? kMmLdsWide : kMmLdsLimit)) return;                                   \
     hipLaunchKernelGGL((moe_gate_up_mfma_kernel<J, W>), grid, dim3(kWave * W), lds, stream, gate_all, up_all, shared.gate, \
                        shared.up, shared.n_routed, act.qs, act.d, act.digits, groups.expert, groups.start,            \
-                       groups.sorted_slot, groups.sorted_token, mid, n_ff, nb_in, toks, tiles_per_wg)
-    if (toks > 16) {
+                       groups.n_groups, groups.sorted_slot, groups.sorted_token, mid, n_ff, nb_in, toks, tiles_per_wg)
+    if (toks > 16 && waves == 8) {
+        RNB_LAUNCH_GUW(4, 8);
+    } else if (toks > 16) {
         RNB_LAUNCH_GUW(4, kGbWaves);
     } else if (waves == 6) {
         if (toks <= 8) {
@@ -703,17 +753,28 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
     // A workgroup's setup (group, map, image: a chain of dependent loads) costs more than a row tile's few blocks, and
     // about three workgroups fit a compute unit: row tiles are merged (up to 4 per workgroup) until the grid fits them at
     // once (cfg5's shape, 16 row tiles x 126 groups, 64 tokens: 1 / 2 / 4 / 8 tiles per workgroup 72 / 62 / 59 / 62 us)
+    // With groups of more than a tile, whose workgroups fit a compute unit in twos: the least of rounds * (steps + about six for the setup, in which
+    // the tile's intermediates are quantised).
     const uint32_t row_tiles = (n_embd + kGbRows - 1) / kGbRows;
-    uint32_t tiles_per_wg = 1;
-    while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
-        tiles_per_wg *= 2;
-    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, groups.n_groups, 1), block(kGbThreads);
     const uint32_t toks = std::min<uint32_t>(std::max<uint32_t>(groups.max_group, 1), down_tile_tokens(nb_mid, down_quant));
     if (toks == 0) return;
+    const uint32_t units = groups.tiles_of(toks);
+    uint32_t tiles_per_wg = 1;
+    if (units > groups.n_groups) {
+        uint64_t best = ~0ull;
+        for (uint32_t t = 1; t <= row_tiles && t <= 16; t++) {
+            const uint64_t cost = (static_cast<uint64_t>(units) * ((row_tiles + t - 1) / t) + 511) / 512 * (t * nb_mid + 6);
+            if (cost < best) best = cost, tiles_per_wg = t;
+        }
+    } else {
+        while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
+            tiles_per_wg *= 2;
+    }
+    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, units, 1), block(kGbThreads);
 #define RNB_LAUNCH_DMJ(Q, J, LDS)                                                                                     \
     if (!allow_lds<static_cast<int>(Q) * 8 + J>(moe_down_mfma_kernel<Q, J>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
     hipLaunchKernelGGL((moe_down_mfma_kernel<Q, J>), grid, block, LDS, stream, down_all, shared.down, shared.n_routed, mid, \
-                       groups.expert, groups.start, groups.sorted_slot, slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks)
+                       groups.expert, groups.start, groups.n_groups, groups.sorted_slot, slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks)
 #define RNB_LAUNCH_DM(Q, LDS)                                                                                         \
     if (toks <= 8) {                                                                                                  \
         RNB_LAUNCH_DMJ(Q, 1, LDS);                                                                                    \

@@ -1375,6 +1375,33 @@ def test_moe_shared_expert_slot_on_the_matrix_cores_dev(rnb, oracle):
     assert v["ok"] or v["flip_aware_ok"], v
 
 
+@pytest.mark.parametrize("tokens,n_ff,n_embd,down_quant", [(100, 512, 256, Q6_K), (97, 256, 768, Q4_K), (64, 1280, 256, Q5_K)])
+def test_moe_few_experts_take_most_tokens(rnb, oracle, tokens, n_ff, n_embd, down_quant):
+    """Two experts that every token is routed to (two to four token tiles each, the last of one to thirty-two slots) among a
+    hundred with a slot or two: workgroups find their group and token tile across three 64-group steps of the search.
+    Against the oracle, and the same bits with the tokens in reverse order."""
+    n_expert = 140
+    gate, up, down, x, *_ = _moe_case(oracle, n_expert, n_ff, n_embd, tokens, 1, 1500 + tokens, down_quant)
+    rng = np.random.default_rng(tokens)
+    third = (np.arange(tokens) * 7 % 67 + 71).astype(np.uint32)  # 71 .. 137
+    e = np.stack([np.full(tokens, 3, np.uint32), np.full(tokens, 69, np.uint32), third], axis=1).reshape(-1)
+    t = np.repeat(np.arange(tokens, dtype=np.uint32), 3)
+    r = rng.uniform(0.1, 0.6, e.size).astype(np.float32)
+    extra = np.arange(4, 68, 2, dtype=np.uint32)  # experts with one slot each between the two
+    e, t = np.concatenate([e, extra]), np.concatenate([t, extra % tokens])
+    r = np.concatenate([r, rng.uniform(0.1, 0.6, extra.size).astype(np.float32)])
+    got = rnb.qwen35_sparse_experts_selected_base_by_token(gate, up, down, e, r, t, tokens, down_quant, n_ff, n_embd, x)
+    ref = oracle.moe_sparse_experts_by_token(gate, up, down, n_expert, e, r, t, tokens, down_quant, n_ff, n_embd, x)
+    from oracle import flips
+    v = flips.moe_verdict(got, ref, gate, up, down, n_expert, e, r, t, tokens, down_quant, n_ff, n_embd, x)
+    assert v["ok"] or v["flip_aware_ok"], {key: v[key] for key in v if key != "flips"}
+    xr = x.reshape(tokens, n_embd)[::-1].copy()
+    rev = rnb.qwen35_sparse_experts_selected_base_by_token(gate, up, down, e, r, tokens - 1 - t, tokens, down_quant, n_ff, n_embd, xr)
+    assert np.array_equal(rev.reshape(tokens, n_embd)[::-1], got.reshape(tokens, n_embd))
+    for w in (gate, up, down):
+        rnb.release(w)
+
+
 @pytest.mark.parametrize("tokens,n_expert,k,n_ff,n_embd,down_quant,shared", [(64, 128, 8, 1024, 512, Q6_K, False),
                                                                             (48, 60, 8, 1280, 768, Q5_K, False),
                                                                             (100, 128, 2, 512, 256, Q4_K, False),
