@@ -806,6 +806,8 @@ constexpr size_t q8_lds_bytes(bool routed) {
     return 2 * (32 * kTT) * kGbStride128 + 2 * 8 * (32 * kTT) * sizeof(float) + (routed ? kGbWaves * kQ8StripBytes : 0);
 }
 
+typedef float v32f __attribute__((ext_vector_type(32)));
+
 template <int kTT, uint32_t kFmt, bool kRouted, int kLive>
 __global__ void __launch_bounds__(kGbThreads, 2)
     gemm_q8_mfma_kernel(const uint8_t *__restrict__ w, const int8_t *__restrict__ aq, const float *__restrict__ ad,
@@ -833,6 +835,7 @@ __global__ void __launch_bounds__(kGbThreads, 2)
 #pragma unroll
         for (int i = 0; i < 16; i++) accf[t][i] = 0.0f;
     const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    [[maybe_unused]] const v32f zero32 = {};
 
     uint2 sv[kToks * 32 / kGbThreads];
     float sdx[kDxPerThread];
@@ -904,28 +907,69 @@ __global__ void __launch_bounds__(kGbThreads, 2)
             nxt = q8_load_blocks<kFmt>(wrow, sn * 8, nb32, khalf);
         const uint8_t *abase = s_a[buf] + lrow * kGbStride128 + 16 * khalf;
         const uint32_t live = min(8u, nb32 - step * 8);  // blocks of this step that exist (workgroup-uniform)
+        if constexpr (kLive == 16) {
+            // Blocks in pairs: one K=1 matrix instruction over two blocks makes every result's d * d_x of both, which leaves a
+            // conversion and a multiply-add per result and block to the vector port (four instructions before: 4096 x 4096 x
+            // 333 tokens 63 -> 57 us, 9289 x 6400 x 200 133 -> 120).  Its rounding is the multiply's.
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            if (static_cast<uint32_t>(k) < live) {
-                const v4i bop = b32_operand<kFmt>(cur.q[k], cur.qh[k], khalf);
+            for (int k = 0; k < 8; k += 2) {
+                if (static_cast<uint32_t>(k) < live) {
+                    const bool both = static_cast<uint32_t>(k + 1) < live;
+                    const v4i bop0 = b32_operand<kFmt>(cur.q[k], cur.qh[k], khalf), bop1 = b32_operand<kFmt>(cur.q[k + 1], cur.qh[k + 1], khalf);
+                    const float dk = khalf ? cur.d[k + 1] : cur.d[k];
+                    [[maybe_unused]] float mk = 0.0f;
+                    if constexpr (B32<kFmt>::kMin) mk = khalf ? cur.m[k + 1] : cur.m[k];
 #pragma unroll
-                for (int t = 0; t < kTT; t++) {
-                    const v4i aop = *reinterpret_cast<const v4i *>(abase + 32 * t * kGbStride128 + 32 * k);
-                    const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, bop, zero16, 0, 0, 0);
-                    v16i sum = zero16;  // d n + m formats: the block's sum of activations, from a row of ones
-                    if constexpr (B32<kFmt>::kMin) {
-                        const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
-                        sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, ones, zero16, 0, 0, 0);
+                    for (int t = 0; t < kTT; t++) {
+                        const v4i aop0 = *reinterpret_cast<const v4i *>(abase + 32 * t * kGbStride128 + 32 * k);
+                        const v4i aop1 = *reinterpret_cast<const v4i *>(abase + 32 * t * kGbStride128 + 32 * (k + 1));
+                        const float dx = s_dx[buf][k + khalf][32 * t + lrow];
+                        const v16i acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop0, bop0, zero16, 0, 0, 0);
+                        const v16i acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop1, bop1, zero16, 0, 0, 0);
+                        const v32f dd = __builtin_amdgcn_mfma_f32_32x32x1f32(dx, dk, zero32, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 16; i++) accf[t][i] = __builtin_fmaf(dd[i], static_cast<float>(acc0[i]), accf[t][i]);
+                        if (both)
+#pragma unroll
+                            for (int i = 0; i < 16; i++) accf[t][i] = __builtin_fmaf(dd[16 + i], static_cast<float>(acc1[i]), accf[t][i]);
+                        if constexpr (B32<kFmt>::kMin) {  // d n + m formats: the blocks' sums of activations, from a row of ones
+                            const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+                            const v16i sum0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop0, ones, zero16, 0, 0, 0);
+                            const v16i sum1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop1, ones, zero16, 0, 0, 0);
+                            const v32f dm = __builtin_amdgcn_mfma_f32_32x32x1f32(dx, mk, zero32, 0, 0, 0);
+#pragma unroll
+                            for (int i = 0; i < 16; i++) accf[t][i] = __builtin_fmaf(dm[i], static_cast<float>(sum0[i]), accf[t][i]);
+                            if (both)
+#pragma unroll
+                                for (int i = 0; i < 16; i++) accf[t][i] = __builtin_fmaf(dm[16 + i], static_cast<float>(sum1[i]), accf[t][i]);
+                        }
                     }
+                }
+            }
+        } else {
 #pragma unroll
-                    for (int j = 0; j < kLive / 4; j++) {
-                        const float4 dx4 = reinterpret_cast<const float4 *>(s_dx[buf][k])[8 * t + 2 * j + khalf];
-                        const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+            for (int k = 0; k < 8; k++) {
+                if (static_cast<uint32_t>(k) < live) {
+                    const v4i bop = b32_operand<kFmt>(cur.q[k], cur.qh[k], khalf);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            accf[t][4 * j + i] += (cur.d[k] * dx[i]) * static_cast<float>(acc[4 * j + i]);
-                            if constexpr (B32<kFmt>::kMin)
-                                accf[t][4 * j + i] += (cur.m[k] * dx[i]) * static_cast<float>(sum[4 * j + i]);
+                    for (int t = 0; t < kTT; t++) {
+                        const v4i aop = *reinterpret_cast<const v4i *>(abase + 32 * t * kGbStride128 + 32 * k);
+                        const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, bop, zero16, 0, 0, 0);
+                        v16i sum = zero16;  // d n + m formats: the block's sum of activations, from a row of ones
+                        if constexpr (B32<kFmt>::kMin) {
+                            const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+                            sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop, ones, zero16, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int j = 0; j < kLive / 4; j++) {
+                            const float4 dx4 = reinterpret_cast<const float4 *>(s_dx[buf][k])[8 * t + 2 * j + khalf];
+                            const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                accf[t][4 * j + i] += (cur.d[k] * dx[i]) * static_cast<float>(acc[4 * j + i]);
+                                if constexpr (B32<kFmt>::kMin)
+                                    accf[t][4 * j + i] += (cur.m[k] * dx[i]) * static_cast<float>(sum[4 * j + i]);
+                            }
                         }
                     }
                 }
@@ -1017,13 +1061,34 @@ static bool q6_wide_tiles(uint32_t row_tiles, uint32_t seq) {
     return seq > 32 && (tiles >= 512 || (tiles > 224 && tiles <= 256));
 }
 
+// The 64-token form of the 32-element formats: two workgroups fit a compute unit, so 512 run at once and 576 take two
+// rounds.  The number of slices with the least of rounds * (steps + about one for the ends) plus the sum of the slices (about
+// one step's time and what its reads take).  4096 x 4096 x 333 tokens, 192 workgroups: 2 slices instead of 3, 8 steps in a row
+// instead of 12; 4096 x 14336 x 300 135 -> 112 us, 9289 x 6400 x 200 120 -> 108.
+static uint32_t b32_wide_slices(uint64_t wgs, uint32_t steps, uint32_t rows, uint32_t seq) {
+    uint32_t best = 1;
+    double best_cost = 1e30;
+    for (uint32_t s = 1; s <= kSliceMax && s <= std::max(1u, steps / 2); s++) {
+        const double rounds = static_cast<double>((wgs * s + 511) / 512), per = (steps + s - 1) / s;
+        const double sum = s > 1 ? 1.0 + s * static_cast<double>(rows) * seq * 4.0 / 12e6 : 0.0;  // 12 MB in a step's time
+        const double cost = rounds * (per + 1.0) + sum;
+        if (cost < best_cost) best_cost = cost, best = s;
+    }
+    return best;
+}
+static uint32_t b32_slices(uint32_t rows, uint32_t seq, uint32_t steps) {
+    const uint32_t row_tiles = (rows + kGbRows - 1) / kGbRows;
+    const bool wide = seq > 32;
+    const uint64_t wgs = tile_grid(rows, seq, wide);
+    return wide && row_tiles ? b32_wide_slices(wgs, steps, rows, seq) : k_slices(wgs, steps, true);
+}
+
 size_t gemm_blocks_slice_floats(uint32_t quant, uint32_t rows, uint32_t k_steps, uint32_t seq) {
     if (rows == 0 || seq == 0 || k_steps == 0) return 0;
     const uint32_t row_tiles = (rows + kGbRows - 1) / kGbRows;
-    const bool wide = is_b32(quant) ? seq > 32
-                      : quant == kQ6K                    ? q6_wide_tiles(row_tiles, seq)
-                                                         : wide_tiles(row_tiles, seq);
-    const uint32_t slices = k_slices(tile_grid(rows, seq, wide), k_steps, quant != kQ4K && quant != kQ5K);  // as the launchers
+    const bool wide = quant == kQ6K ? q6_wide_tiles(row_tiles, seq) : wide_tiles(row_tiles, seq);
+    const uint32_t slices = is_b32(quant) ? b32_slices(rows, seq, k_steps)
+                                          : k_slices(tile_grid(rows, seq, wide), k_steps, quant != kQ4K && quant != kQ5K);  // as the launchers
     return slices > 1 ? static_cast<size_t>(slices) * seq * rows : 0;
 }
 
@@ -1136,7 +1201,7 @@ void launch_gemm_q8_mfma(const uint8_t *w, uint32_t quant, ActView act, float *o
     const uint32_t row_tiles = (rows + kGbRows - 1) / kGbRows;
     const bool wide = seq > 32;  // measured: the 64-token tile wins here even on a small grid (4096 x 4096 x 512: 100 vs 123 us)
     const uint32_t steps = (nb32 + 7) / 8;
-    const uint32_t slices = slice_out ? k_slices(tile_grid(rows, seq, wide), steps, true) : 1;
+    const uint32_t slices = slice_out ? b32_slices(rows, seq, steps) : 1;
     const uint32_t steps_slice = (steps + slices - 1) / slices, nz = (steps + steps_slice - 1) / steps_slice;
     float *dst = nz > 1 ? slice_out : out;
     const dim3 grid(row_tiles, wide ? (seq + 63) / 64 : 1, nz), block(kGbThreads);
