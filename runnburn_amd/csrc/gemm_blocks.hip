@@ -1034,19 +1034,53 @@ static uint64_t tile_grid(uint32_t rows, uint32_t seq, bool wide) {
 }
 
 namespace {
+// A handful of loads per result and nothing else: a latency kernel on small outputs, so a result's loads are all in flight
+// before the first addition (kSlices > 0; one by one in a loop of run-time length: kSlices 0, more than sixteen slices).
+// 8 slices of 12 x 4096 results 4.0 -> 2.2 us.
+template <uint32_t kSlices>
 __global__ void __launch_bounds__(256) sum_slices_kernel(const float *__restrict__ parts, float *__restrict__ out, size_t n,
                                                          uint32_t slices) {
     const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= n) return;
-    float acc = parts[i];
-    for (uint32_t z = 1; z < slices; z++) acc += parts[z * n + i];
+    float acc;
+    if constexpr (kSlices > 0) {
+        float v[kSlices];
+#pragma unroll
+        for (uint32_t z = 0; z < kSlices; z++) v[z] = parts[z * n + i];
+        acc = v[0];
+#pragma unroll
+        for (uint32_t z = 1; z < kSlices; z++) acc += v[z];
+    } else {
+        acc = parts[i];
+        for (uint32_t z = 1; z < slices; z++) acc += parts[z * n + i];
+    }
     out[i] = acc;
 }
 }  // namespace
 
 void launch_sum_slices(const float *parts, float *out, size_t n, uint32_t slices, hipStream_t stream) {
-    hipLaunchKernelGGL(sum_slices_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, stream, parts, out, n,
-                       slices);
+    const dim3 grid(static_cast<uint32_t>((n + 255) / 256)), block(256);
+#define RNB_SUM(N) \
+    case N: hipLaunchKernelGGL((sum_slices_kernel<N>), grid, block, 0, stream, parts, out, n, slices); break
+    switch (slices) {
+        RNB_SUM(2);
+        RNB_SUM(3);
+        RNB_SUM(4);
+        RNB_SUM(5);
+        RNB_SUM(6);
+        RNB_SUM(7);
+        RNB_SUM(8);
+        RNB_SUM(9);
+        RNB_SUM(10);
+        RNB_SUM(11);
+        RNB_SUM(12);
+        RNB_SUM(13);
+        RNB_SUM(14);
+        RNB_SUM(15);
+        RNB_SUM(16);
+    default: hipLaunchKernelGGL((sum_slices_kernel<0>), grid, block, 0, stream, parts, out, n, slices);
+    }
+#undef RNB_SUM
 }
 
 static bool is_b32(uint32_t quant) {
