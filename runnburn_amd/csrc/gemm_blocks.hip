@@ -16,7 +16,7 @@
 //          d n + m formats add (m * d_x) * sum(a) from a second instruction against a row of ones.
 //   Q2_K Q3_K   Q6_K's scheme; Q2_K's mins term through two K=16 instructions over the sub-block sums' digits:
 //          crates/rnb-cpu/src/gemm/avx2_dot.rs:169-242 (Q2_K), :247-375 (Q3_K).
-// That is 16 (Q6_K) or 48 (Q8) vector instructions per matrix instruction, so these kernels are bound by the vector
+// That is 16 (Q6_K) or 32 (Q8) vector instructions per matrix instruction, so these kernels are bound by the vector
 // port, not the matrix pipe; at 512 tokens they measured 9 to 17 times faster than GEMV passes over the tokens on the
 // vector units' integer dots.
 //
