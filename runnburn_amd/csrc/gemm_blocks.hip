@@ -869,6 +869,14 @@ __global__ void __launch_bounds__(kGbThreads, 2)
         }
     };
 
+    // the value of the lane's K-half, chosen between registers: as a choice between two members the compiler made it one load
+    // at a chosen address and kept the row-load form's blocks in memory (240 bytes a lane; columns that are no multiple of
+    // 256: Q8_1 12792 x 4320 x 1202 tokens 616 us against 321, Q5_0 14014 x 3456 x 144 168 against 104)
+    [[maybe_unused]] auto of_half = [&](float lower, float upper) {
+        asm volatile("" : "+v"(lower), "+v"(upper));
+        return khalf ? upper : lower;
+    };
+
     const uint32_t wrow0 = min(blockIdx.x * kGbRows + wave * 32, rows - 1);
     const uint8_t *wbase = w + static_cast<size_t>(wrow0) * nb32 * kBlockBytes;
     uint8_t *strip = s_dyn + q8_lds_bytes<kTT>(false) + wave * kQ8StripBytes;
@@ -907,18 +915,23 @@ __global__ void __launch_bounds__(kGbThreads, 2)
             nxt = q8_load_blocks<kFmt>(wrow, sn * 8, nb32, khalf);
         const uint8_t *abase = s_a[buf] + lrow * kGbStride128 + 16 * khalf;
         const uint32_t live = min(8u, nb32 - step * 8);  // blocks of this step that exist (workgroup-uniform)
-        if constexpr (kLive == 16) {
-            // Blocks in pairs: one K=1 matrix instruction over two blocks makes every result's d * d_x of both, which leaves a
-            // conversion and a multiply-add per result and block to the vector port (four instructions before: 4096 x 4096 x
-            // 333 tokens 63 -> 57 us, 9289 x 6400 x 200 133 -> 120).  Its rounding is the multiply's.
+        // Blocks in pairs: one K=1 matrix instruction over two blocks makes every result's d * d_x of both, which leaves a
+        // conversion and a multiply-add per result and block to the vector port (four instructions before: 4096 x 4096 x
+        // 333 tokens 63 -> 57 us, 9289 x 6400 x 200 133 -> 120).  Its rounding is the multiply's.  64 tokens of rows loaded
+        // lane by lane are bound by those loads where the blocks are an odd number of 16-bit words (Q4_0, Q5_0, Q8_0) and
+        // stay with one block at a time: Q8_0 996 x 3520 x 2842 98 us against 113, Q5_0 14014 x 3456 x 144 104 against 120
+        // (ahead in pairs: Q4_0 2829 x 5920 x 3968 612 against 684; Q8_1 12792 x 4320 x 1202 321 against 345, Q5_1 2015 x
+        // 1984 x 2524 116 against 131 and all of the 4-byte blocks).
+        constexpr bool kPairs = kLive == 16 && (kRouted || kTT == 1 || kBlockBytes % 4 == 0);
+        if constexpr (kPairs) {
 #pragma unroll
             for (int k = 0; k < 8; k += 2) {
                 if (static_cast<uint32_t>(k) < live) {
                     const bool both = static_cast<uint32_t>(k + 1) < live;
                     const v4i bop0 = b32_operand<kFmt>(cur.q[k], cur.qh[k], khalf), bop1 = b32_operand<kFmt>(cur.q[k + 1], cur.qh[k + 1], khalf);
-                    const float dk = khalf ? cur.d[k + 1] : cur.d[k];
+                    const float dk = of_half(cur.d[k], cur.d[k + 1]);
                     [[maybe_unused]] float mk = 0.0f;
-                    if constexpr (B32<kFmt>::kMin) mk = khalf ? cur.m[k + 1] : cur.m[k];
+                    if constexpr (B32<kFmt>::kMin) mk = of_half(cur.m[k], cur.m[k + 1]);
 #pragma unroll
                     for (int t = 0; t < kTT; t++) {
                         const v4i aop0 = *reinterpret_cast<const v4i *>(abase + 32 * t * kGbStride128 + 32 * k);

@@ -313,3 +313,16 @@ def test_q8_0_head_batch_validation_messages_match_reference():
     e = _err(rnb.q8_0_head_gemv_batch, z(3 * 4 * 3 * 34, np.uint8), 3, 4, 96, 3, z(3 * 3 * 96 - 1, np.float32))
     assert str(e) == "Q8_0 head batch input length mismatch: got 863, expected 864"
 
+
+def test_kernels_of_the_32_element_gemm_keep_their_registers():
+    """No instantiation of the 32-element formats' GEMM keeps a weight block in scratch memory (the compiler's figure, from
+    the code objects' metadata): it walks every block of a row, so that costs a third of its time."""
+    lib = open(binding._LIB_PATH, "rb").read()
+    entry = re.compile(rb"\.name(?:[\xa0-\xbf]|\xd9.|\xda..)(_Z[\w.]+?)\xbb\.private_segment_fixed_size"
+                       rb"(\xce.{4}|\xcd..|\xcc.|[\x00-\x7f])", re.S)
+    kernels = {}
+    for name, v in entry.findall(lib):
+        kernels[name.decode()] = v[0] if len(v) == 1 else int.from_bytes(v[1:], "big")
+    found = {name: size for name, size in kernels.items() if "gemm_q8_mfma_kernel" in name}
+    assert len(found) == 48  # six formats, strip and row loads, four forms
+    assert not any(found.values()), {name: size for name, size in found.items() if size}
