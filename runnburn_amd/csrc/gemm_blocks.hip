@@ -1111,11 +1111,13 @@ static bool q6_wide_tiles(uint32_t row_tiles, uint32_t seq) {
 // The 64-token form of the 32-element formats: two workgroups fit a compute unit, so 512 run at once and 576 take two
 // rounds.  The number of slices with the least of rounds * (steps + about one for the ends) plus the sum of the slices (about
 // one step's time and what its reads take).  4096 x 4096 x 333 tokens, 192 workgroups: 2 slices instead of 3, 8 steps in a row
-// instead of 12; 4096 x 14336 x 300 135 -> 112 us, 9289 x 6400 x 200 120 -> 108.
+// instead of 12; 4096 x 14336 x 300 135 -> 112 us, 9289 x 6400 x 200 120 -> 108.  The partial sums stay within
+// kSliceScratchBytes: the workspace is kept for the next call.
 static uint32_t b32_wide_slices(uint64_t wgs, uint32_t steps, uint32_t rows, uint32_t seq) {
     uint32_t best = 1;
     double best_cost = 1e30;
     for (uint32_t s = 1; s <= kSliceMax && s <= std::max(1u, steps / 2); s++) {
+        if (s > 1 && static_cast<uint64_t>(s) * rows * seq * sizeof(float) > kSliceScratchBytes) break;
         const double rounds = static_cast<double>((wgs * s + 511) / 512), per = (steps + s - 1) / s;
         const double sum = s > 1 ? 1.0 + s * static_cast<double>(rows) * seq * 4.0 / 12e6 : 0.0;  // 12 MB in a step's time
         const double cost = rounds * (per + 1.0) + sum;

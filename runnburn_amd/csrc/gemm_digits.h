@@ -351,7 +351,8 @@ struct DgPlan {
 // Token tiles of 32 are dealt into groups of two to four per workgroup, one workgroup fits a compute unit.  A block costs
 // a workgroup about a tile and a half beside its tiles (making the operands): the group size with the least of
 // rounds * blocks * (tiles + 1.5).  Up to 128 workgroups K is cut so that the slices fill the 256 units once (a slice
-// keeps at least 4 blocks).
+// keeps at least 4 blocks); their partial sums are at most 256 workgroups' results.
+static_assert(size_t(256) * kDgRows * 4 * 32 * sizeof(float) <= kSliceScratchBytes, "bound of the slices' workspace");
 inline DgPlan digits_plan(uint32_t rows, uint32_t nb, uint32_t seq) {
     const uint32_t tiles = (seq + 31) / 32;
     DgPlan best{};

@@ -1,6 +1,7 @@
 """No-GPU checks of the C-ABI library: it loads, exports every symbol include/rnb_hip.h declares,
 validates requests with the reference's messages before touching a device, and reports a
 distinguishable NoDevice status so callers can skip (crates/rnb-backend/cuda/src/runtime/tests.rs:22831-22834)."""
+import ctypes
 import os
 import re
 
@@ -326,3 +327,30 @@ def test_kernels_of_the_32_element_gemm_keep_their_registers():
     found = {name: size for name, size in kernels.items() if "gemm_q8_mfma_kernel" in name}
     assert len(found) == 48  # six formats, strip and row loads, four forms
     assert not any(found.values()), {name: size for name, size in found.items() if size}
+
+
+def _plan(symbol, restype, *argtypes):
+    """A host-side planning function of the library (C++ linkage)."""
+    fn = getattr(rnb.lib(), symbol)
+    fn.restype, fn.argtypes = restype, list(argtypes)
+    return fn
+
+
+def test_partial_sums_of_the_prefill_gemms_are_bounded():
+    """Batches of more than 32 tokens: the K slices of the 32-element formats' GEMM and of the two-digit GEMM write at most
+    32 MiB of partial sums, so the workspace that outlives the call has a bound whatever the shape."""
+    u32 = ctypes.c_uint32
+    blocks = _plan("_ZN3rnb24gemm_blocks_slice_floatsEjjjj", ctypes.c_size_t, u32, u32, u32, u32)
+    digits = _plan("_ZN3rnb24gemm_digits_slice_floatsEjjj", ctypes.c_size_t, u32, u32, u32)
+    sliced = 0
+    for rows in (1, 127, 512, 2048, 4096, 9289, 17920, 28672, 128256):
+        for nb in (1, 4, 16, 25, 56, 64):  # super-blocks of a row, the 256-element steps of a 32-element format
+            for seq in (33, 65, 128, 200, 333, 512, 1024, 2048, 16384):
+                for quant in (2, 3, 6, 7, 8, 9):
+                    need = 4 * blocks(quant, rows, nb, seq)
+                    assert need <= 32 << 20, (quant, rows, nb, seq, need)
+                    sliced += need > 0
+                need = 4 * digits(rows, nb, seq)
+                assert need <= 32 << 20, ("digits", rows, nb, seq, need)
+                sliced += need > 0
+    assert sliced > 500
