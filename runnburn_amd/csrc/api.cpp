@@ -125,9 +125,11 @@ int reserve_fail(hipError_t e) {
     } while (0)
 
 // A fixed span of device memory that a call carves its scratch from instead of the state's grow-only buffers: the
-// entry point that must not allocate passes one over its static array.
+// entry point that must not allocate passes one over its static array.  `slices` holds kSliceScratchBytes for the partial
+// sums of the kernels that bound theirs.
 struct Arena {
     uint8_t *base = nullptr;
+    float *slices = nullptr;
     size_t cap = 0, used = 0;
     const char *who = "";
 };
@@ -246,6 +248,16 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         *ws = p;
         return RNB_HIP_OK;
     };
+    // ... and of those whose slices are bounded: an arena has room of its own for any shape's, so that a shape has one kernel
+    // and one order of its sums whoever calls
+    auto bounded_slices = [&](size_t floats, float **ws) -> int {
+        if (arena == nullptr || floats == 0) return slice_floats(floats, ws);
+        if (arena->slices == nullptr || floats * sizeof(float) > kSliceScratchBytes)
+            return fail(RNB_HIP_EXECUTION_FAILED, std::string(arena->who) + " has no room for " +
+                                                      std::to_string(floats * sizeof(float)) + " bytes of partial sums");
+        *ws = arena->slices;
+        return RNB_HIP_OK;
+    };
     // a kernel with smaller slices follows where a fixed span has no room for these
     auto fits = [&](size_t floats) {
         return arena == nullptr || (arena->used + 255) / 256 * 256 + floats * sizeof(float) <= arena->cap;
@@ -308,7 +320,7 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         }
     } else if (seq >= min_gemm_seq && gemm_q8_mfma_supported(quant, static_cast<uint32_t>(cols / 32))) {
         const uint32_t nb32 = static_cast<uint32_t>(cols / 32);
-        if (int st = slice_ws((nb32 + 7) / 8, &ws); st != RNB_HIP_OK) return st;
+        if (int st = bounded_slices(gemm_blocks_slice_floats(quant, r, (nb32 + 7) / 8, q), &ws); st != RNB_HIP_OK) return st;
         launch_gemm_q8_mfma(w_dev, quant, act, out_dev, ws, r, nb32, q, s.stream);
     } else {
         launch_gemv_block32(w_dev, quant, act, out_dev, r, static_cast<uint32_t>(cols / 32), q, s.stream);
@@ -1555,6 +1567,7 @@ int rnb_hip_gemv_dev_noalloc(uint32_t quant, const void *w_dev, size_t rows, siz
     arena.who = "rnb_hip_gemv_dev_noalloc";
     st = static_scratch_ptr(*g.state, &arena.base);
     if (st != RNB_HIP_OK) return st;
+    arena.slices = static_cast<float *>(g.state->noalloc_slices);
     return run_matmul_dev(*g.state, quant, static_cast<const uint8_t *>(w_dev), rows, cols, x_dev, seq_len, out_dev, &arena);
 }
 

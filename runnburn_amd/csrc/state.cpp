@@ -250,6 +250,10 @@ Guard::Guard() : lock(g_mutex) {
         fail(RNB_HIP_EXECUTION_FAILED, std::string("hipStreamCreate: ") + hipGetErrorString(e));
         return;
     }
+    if (hipMalloc(&s->noalloc_slices, kSliceScratchBytes) != hipSuccess) {  // reported by the call that needs it
+        (void)hipGetLastError();
+        s->noalloc_slices = nullptr;
+    }
     s->allocator.reset(new HipAllocator(s));
     s->table.reset(new ResidentTable(s->allocator.get()));
     // resident weights may take 85% of what is free now unless RNB_HIP_RESIDENT_BUDGET_MB says otherwise

@@ -1,11 +1,11 @@
 """rnb_hip_gemv_dev_noalloc: the device-resident GEMV / small-batch GEMM with its scratch (quantised activations,
-K-slice partial sums) in the library's fixed device array instead of the grow-only buffers.  It runs the same kernels
+K-slice partial sums) in the library's fixed device arrays instead of the grow-only buffers.  It runs the same kernels
 on the same operands as rnb_hip_gemv_dev, so the outputs must be the same bits, call after call, also when a smaller
-call follows a larger one over the array's stale contents."""
+call follows a larger one over the arrays' stale contents."""
 import numpy as np
 import pytest
 
-Q4_K, Q6_K, Q8_0 = 12, 14, 8
+Q4_0, Q4_1, Q5_1, Q8_0, Q4_K, Q6_K = 2, 3, 7, 8, 12, 14
 
 
 def _both(rnb, oracle, quant, rows, cols, seq, seed):
@@ -40,6 +40,27 @@ def test_noalloc_matches_gemv_dev_twice(rnb, oracle, quant, big, small):
         gold = np.asarray(oracle.gemv(quant, w, rows, cols, x, gold=True), np.float64).ravel()
         rms = float(np.sqrt(np.mean(gold * gold))) or 1.0
         assert float(np.abs(got.astype(np.float64) - gold).max()) <= 2e-5 * rms
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,rows,cols,seq", [
+    (Q8_0, 4096, 4096, 65),    # eight K slices, with the activations more than the first array holds
+    (Q8_0, 5120, 5120, 64),    # ten
+    (Q5_1, 8192, 4096, 40),
+    (Q4_0, 9472, 5120, 222),   # 296 workgroups, three slices of 8 MB
+    (Q4_1, 4096, 4064, 97),    # a last step of seven blocks
+])
+def test_noalloc_partial_sums_beyond_the_first_array(rnb, oracle, quant, rows, cols, seq):
+    """K slices whose partial sums leave the first array's room: taken all the same, same bits as rnb_hip_gemv_dev, and
+    rows at both ends and between against the oracle's f64 statement (|gpu - gold| <= 2e-5 * rms(gold))."""
+    print(f"noalloc case quant={quant} rows={rows} cols={cols} seq={seq}", flush=True)
+    w, x, ref, got = _both(rnb, oracle, quant, rows, cols, seq, 5100 + rows)
+    assert np.array_equal(ref.view(np.uint32), got.view(np.uint32))
+    pick = [0, 127, 128, rows // 2, rows - 1]
+    ws = np.ascontiguousarray(w.reshape(rows, -1)[pick]).reshape(-1)
+    gold = np.asarray(oracle.gemv(quant, ws, len(pick), cols, x, gold=True), np.float64).reshape(seq, len(pick))
+    rms = float(np.sqrt(np.mean(gold * gold)))
+    assert float(np.abs(got.reshape(seq, rows)[:, pick] - gold).max()) <= 2e-5 * rms
 
 
 @pytest.mark.gpu
