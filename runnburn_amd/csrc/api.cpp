@@ -258,18 +258,14 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         *ws = arena->slices;
         return RNB_HIP_OK;
     };
-    // a kernel with smaller slices follows where a fixed span has no room for these
-    auto fits = [&](size_t floats) {
-        return arena == nullptr || (arena->used + 255) / 256 * 256 + floats * sizeof(float) <= arena->cap;
-    };
     auto slice_ws = [&](uint32_t k_steps, float **ws) -> int {
         return slice_floats(gemm_blocks_slice_floats(quant, r, k_steps, q), ws);
     };
     float *ws = nullptr;
     if (is_iq_quant(quant)) {
         // importance quants: the matrix-core GEMM for batches, else the GEMV (a pass per group of up to four tokens)
-        if (gemm_iq_digits_pays(quant, w_dev, rows, cols, seq) && fits(gemm_digits_slice_floats(r, nb, q))) {
-            if (int st = slice_floats(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
+        if (gemm_iq_digits_pays(quant, w_dev, rows, cols, seq)) {
+            if (int st = bounded_slices(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
             launch_gemm_iq_digits(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
         } else if (seq >= kIqGemmMinSeq) {
             if (int st = slice_floats(gemm_iq_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
@@ -277,9 +273,8 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         } else {
             launch_gemv_iq(w_dev, quant, act, out_dev, r, nb, q, s.stream);
         }
-    } else if (gemm_digits_pays(quant, w_dev, rows, cols, seq) && (quant == kQ6K || act.digits != nullptr) &&
-               fits(gemm_digits_slice_floats(r, nb, q))) {
-        if (int st = slice_floats(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
+    } else if (gemm_digits_pays(quant, w_dev, rows, cols, seq) && (quant == kQ6K || act.digits != nullptr)) {
+        if (int st = bounded_slices(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
         launch_gemm_digits(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
     } else if (quant == kQ4K) {
         // the GEMM fills LDS with 16-byte loads: weights at other alignments take the vector kernels

@@ -5,7 +5,7 @@ call follows a larger one over the arrays' stale contents."""
 import numpy as np
 import pytest
 
-Q4_0, Q4_1, Q5_1, Q8_0, Q4_K, Q6_K = 2, 3, 7, 8, 12, 14
+Q4_0, Q4_1, Q5_1, Q8_0, Q4_K, Q5_K, Q6_K, IQ2_S, IQ4_XS = 2, 3, 7, 8, 12, 13, 14, 22, 23
 
 
 def _both(rnb, oracle, quant, rows, cols, seq, seed):
@@ -49,6 +49,13 @@ def test_noalloc_matches_gemv_dev_twice(rnb, oracle, quant, big, small):
     (Q5_1, 8192, 4096, 40),
     (Q4_0, 9472, 5120, 222),   # 296 workgroups, three slices of 8 MB
     (Q4_1, 4096, 4064, 97),    # a last step of seven blocks
+    # formats with a second GEMM for large batches (two-digit operands), whose slices leave the first array's room
+    (Q6_K, 2048, 10752, 100),  # ten slices
+    (Q6_K, 4352, 4096, 345),
+    (Q5_K, 2111, 14336, 170),
+    (Q4_K, 4096, 14336, 333),
+    (IQ2_S, 4111, 8192, 150),
+    (IQ4_XS, 2048, 14336, 75),
 ])
 def test_noalloc_partial_sums_beyond_the_first_array(rnb, oracle, quant, rows, cols, seq):
     """K slices whose partial sums leave the first array's room: taken all the same, same bits as rnb_hip_gemv_dev, and
