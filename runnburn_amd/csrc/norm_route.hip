@@ -13,12 +13,14 @@
 #include "act_quant.h"
 #include "device_utils.h"
 #include "kernels.h"
+#include <type_traits>
 
 namespace rnb {
 
 namespace {
 
 constexpr int kNormMaxWaves = 16;
+constexpr uint32_t kNormManyRows = 513;  // two workgroups of sixteen waves fit a compute unit: 512 rows at once
 
 // sum over the wave on the DPP data path, in lane 63 (f64: its two halves move separately)
 template <int kCtrl, int kRowMask>
@@ -39,12 +41,15 @@ __device__ __forceinline__ float row16_sum(float v) { return seg_sum<16>(v); }
 __device__ __forceinline__ double wave_sum63(double v) { return dpp_add<0x143, 0xc>(dpp_add<0x142, 0xa>(row16_sum(v))); }
 __device__ __forceinline__ float wave_sum63(float v) { return seg_sum<64>(v); }
 
-// sum over the workgroup's `waves` waves, every thread gets the total; s_part holds kNormMaxWaves zeros before its first
-// use (slots of absent waves stay zero) and one slot array serves one call
+// sum over the workgroup: every wave puts its sums into slots, every thread gets the total of the sixteen slots.  They hold
+// zeros before (slots that nobody puts to stay zero) and one slot array serves one sum
 template <typename T>
-__device__ __forceinline__ T wg_sum(T v, T *s_part) {
+__device__ __forceinline__ void put_sum(T v, T *s_part, uint32_t slot) {
     const T total = wave_sum63(v);
-    if ((threadIdx.x & 63) == 63) s_part[threadIdx.x >> 6] = total;
+    if ((threadIdx.x & 63) == 63) s_part[slot] = total;
+}
+template <typename T>
+__device__ __forceinline__ T wg_sum(const T *s_part) {
     __syncthreads();
     return row16_sum(s_part[threadIdx.x & 15]);
 }
@@ -67,12 +72,12 @@ __device__ __forceinline__ void add_squares(typename NormSum<kUnit>::type &acc, 
     acc += static_cast<T>(v.w) * static_cast<T>(v.w);
 }
 template <bool kUnit>
-__device__ __forceinline__ float rms_of(typename NormSum<kUnit>::type acc, uint32_t nb, float eps, typename NormSum<kUnit>::type *s_part) {
+__device__ __forceinline__ float rms_of(uint32_t nb, float eps, const typename NormSum<kUnit>::type *s_part) {
     const float n = static_cast<float>(nb) * 256.0f;
     if constexpr (kUnit)
-        return sqrtf(wg_sum<float>(acc, s_part) / n + eps);
+        return sqrtf(wg_sum(s_part) / n + eps);
     else
-        return static_cast<float>(sqrt(wg_sum<double>(acc, s_part) / static_cast<double>(n) + static_cast<double>(eps)));
+        return static_cast<float>(sqrt(wg_sum(s_part) / static_cast<double>(n) + static_cast<double>(eps)));
 }
 
 template <bool kUnit>
@@ -91,8 +96,13 @@ __device__ __forceinline__ float4 unit_scale(float4 w) {
 // of the first sum and stay in registers (rows of up to kPer * 16 blocks).  One row of 4096 with the residual add: 9.4 ->
 // 5.2 us (6.1 -> 3.8 us without it, twelve rows 10.0 -> 5.8); with four waves that read the row again for every step each
 // wave went through four blocks and four dependent round trips, and with loads behind `b < nb` (four dword loads and a
-// branch each) sixteen waves took 7.6.  kPer == 0 is the form for longer rows: blocks are read again in each step.
-template <bool kAdd, bool kUnitPost, bool kUnit, int kPer>
+// branch each) sixteen waves took 7.6.  kPer == 0 is the form for longer rows: blocks are read again in each step.  It is also
+// the form for many rows (kByBlock, four waves): rows of other workgroups hide a row's latencies then, and sixteen waves
+// that wait for each other leave the chip less to do: 2048 rows of 1536 with the residual add 15.4 us with a wave per block
+// against 13.2, of 4096 without it 19.4 against 17.7 (4096 x 640 rows 9.3 : 8.8; x 512 7.3 : 7.7; four waves with their
+// blocks in registers 19.2 at 2048 rows).  Its blocks' sums are added as the wave per block adds them: a row's bits do not
+// depend on the number of rows.
+template <bool kAdd, bool kUnitPost, bool kUnit, int kPer, bool kByBlock>
 __global__ void __launch_bounds__(kWave * kNormMaxWaves)
     rms_norm_kernel(const float *__restrict__ input, const float *__restrict__ post_weight, float post_eps,
                     float *__restrict__ residual, const float *__restrict__ weight, float eps, uint32_t nb,
@@ -133,16 +143,25 @@ __global__ void __launch_bounds__(kWave * kNormMaxWaves)
     }
     __syncthreads();
 
+    // squares of a block: into the wave's sum, or (kByBlock) a sum and a slot of its own
+    auto square = [&](auto unit, auto &acc, auto *s_part, uint32_t b, const float4 q) {
+        if constexpr (kByBlock) acc = 0;
+        add_squares<decltype(unit)::value>(acc, q);
+        if constexpr (kByBlock) put_sum(acc, s_part, b);
+    };
+    const std::bool_constant<kUnitPost> post{};
+    const std::bool_constant<kUnit> pre{};
     typename NormSum<kUnit>::type acc = 0;
     if constexpr (kAdd) {
         typename NormSum<kUnitPost>::type pacc = 0;
         if constexpr (kPer > 0) {
 #pragma unroll
-            for (int i = 0; i < kPer; i++) add_squares<kUnitPost>(pacc, v[i]);
+            for (int i = 0; i < kPer; i++) square(post, pacc, s_post, wave + i * waves, v[i]);
         } else {
-            for (uint32_t b = wave; b < nb; b += waves) add_squares<kUnitPost>(pacc, x[static_cast<size_t>(b) * 64]);
+            for (uint32_t b = wave; b < nb; b += waves) square(post, pacc, s_post, b, x[static_cast<size_t>(b) * 64]);
         }
-        const float post_rms = rms_of<kUnitPost>(pacc, nb, post_eps, s_post);
+        if constexpr (!kByBlock) put_sum(pacc, s_post, wave);
+        const float post_rms = rms_of<kUnitPost>(nb, post_eps, s_post);
         auto add = [&](float4 q, const float4 a, const float4 raw) {
             const float4 s = unit_scale<kUnitPost>(raw);
             q.x += (a.x / post_rms) * s.x;
@@ -158,7 +177,7 @@ __global__ void __launch_bounds__(kWave * kNormMaxWaves)
                 v[i] = add(r[i], v[i], p[i]);
                 if (b < nb) {
                     res[static_cast<size_t>(b) * 64] = v[i];
-                    add_squares<kUnit>(acc, v[i]);
+                    square(pre, acc, s_sum, b, v[i]);
                 }
             }
         } else {
@@ -166,19 +185,20 @@ __global__ void __launch_bounds__(kWave * kNormMaxWaves)
                 const size_t at = static_cast<size_t>(b) * 64;
                 const float4 q = add(res[at], x[at], pw[at]);
                 res[at] = q;  // read again below by the same thread
-                add_squares<kUnit>(acc, q);
+                square(pre, acc, s_sum, b, q);
             }
             x = res;
         }
     } else {
         if constexpr (kPer > 0) {
 #pragma unroll
-            for (int i = 0; i < kPer; i++) add_squares<kUnit>(acc, v[i]);
+            for (int i = 0; i < kPer; i++) square(pre, acc, s_sum, wave + i * waves, v[i]);
         } else {
-            for (uint32_t b = wave; b < nb; b += waves) add_squares<kUnit>(acc, x[static_cast<size_t>(b) * 64]);
+            for (uint32_t b = wave; b < nb; b += waves) square(pre, acc, s_sum, b, x[static_cast<size_t>(b) * 64]);
         }
     }
-    const float rms = rms_of<kUnit>(acc, nb, eps, s_sum);
+    if constexpr (!kByBlock) put_sum(acc, s_sum, wave);
+    const float rms = rms_of<kUnit>(nb, eps, s_sum);
     auto finish = [&](uint32_t b, const float4 a, const float4 raw) {
         const float4 s = unit_scale<kUnit>(raw);
         const float4 o = make_float4((a.x / rms) * s.x, (a.y / rms) * s.y, (a.z / rms) * s.z, (a.w / rms) * s.w);
@@ -270,22 +290,27 @@ void launch_rms_norm(const float *input, const float *post_weight, float post_ep
                      const float *weight, float eps, bool unit, uint32_t seq, uint32_t nb, float *out_f32, int8_t *qs,
                      float *d, int16_t *bsums, uint8_t *digits, hipStream_t stream) {
     if (seq == 0 || nb == 0) return;
-    // rows of up to 16 blocks: a wave per block; up to 64 blocks: sixteen waves with their two or four blocks in registers
-    const uint32_t waves = nb < kNormMaxWaves ? nb : kNormMaxWaves, per = (nb + waves - 1) / waves;
+    // rows of up to 16 blocks: a wave per block, or four waves per row for many rows; up to 64 blocks: sixteen waves with
+    // their two or four blocks in registers
+    const bool many = seq >= kNormManyRows && nb >= 4 && nb <= kNormMaxWaves;
+    const uint32_t most = many ? 4 : kNormMaxWaves;
+    const uint32_t waves = nb < most ? nb : most, per = (nb + waves - 1) / waves;
     const dim3 grid(seq), block(kWave * waves);
-#define RNB_NORM_PER(ADD, UP, U, PER)                                                                                      \
-    hipLaunchKernelGGL((rms_norm_kernel<ADD, UP, U, PER>), grid, block, 0, stream, input, post_weight, post_eps, residual, \
-                       weight, eps, nb, out_f32, qs, d, bsums, digits)
-#define RNB_NORM(ADD, UP, U)                  \
-    do {                                      \
-        if (per == 1)                         \
-            RNB_NORM_PER(ADD, UP, U, 1);      \
-        else if (per == 2)                    \
-            RNB_NORM_PER(ADD, UP, U, 2);      \
-        else if (per <= 4)                    \
-            RNB_NORM_PER(ADD, UP, U, 4);      \
-        else                                  \
-            RNB_NORM_PER(ADD, UP, U, 0);      \
+#define RNB_NORM_PER(ADD, UP, U, PER, BY_BLOCK)                                                                         \
+    hipLaunchKernelGGL((rms_norm_kernel<ADD, UP, U, PER, BY_BLOCK>), grid, block, 0, stream, input, post_weight, post_eps, \
+                       residual, weight, eps, nb, out_f32, qs, d, bsums, digits)
+#define RNB_NORM(ADD, UP, U)                    \
+    do {                                        \
+        if (many)                               \
+            RNB_NORM_PER(ADD, UP, U, 0, true);  \
+        else if (per == 1)                      \
+            RNB_NORM_PER(ADD, UP, U, 1, false); \
+        else if (per == 2)                      \
+            RNB_NORM_PER(ADD, UP, U, 2, false); \
+        else if (per <= 4)                      \
+            RNB_NORM_PER(ADD, UP, U, 4, false); \
+        else                                    \
+            RNB_NORM_PER(ADD, UP, U, 0, false); \
     } while (0)
     if (residual == nullptr) {
         if (unit)

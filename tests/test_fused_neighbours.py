@@ -126,6 +126,40 @@ def test_rms_norm_rows_around_the_wave_and_register_limits(rnb, oracle, seq, blo
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("seq,blocks", [(513, 4), (700, 5), (514, 15), (513, 16), (513, 3)])
+@pytest.mark.parametrize("unit", [False, True])
+def test_rms_norm_row_bits_with_many_rows(rnb, oracle, seq, blocks, unit):
+    """Many rows take four waves per row instead of a wave per block (4 to 16 blocks): the same bits as the row alone, with
+    and without the residual add, and the oracle's result within the bounds above (n <= 4096)."""
+    hidden = 256 * blocks
+    rng = np.random.default_rng(60 + blocks)
+    inp, res = rng.standard_normal((2, seq, hidden)).astype(np.float32)
+    pw, qw = (rng.standard_normal((2, hidden)) * 0.3 + 1.0).astype(np.float32)
+    pwd, qwd = rnb.DeviceBuffer.from_host(pw), rnb.DeviceBuffer.from_host(qw)
+
+    def both(rows):
+        n = len(rows)
+        x, r, o, plain = (rnb.DeviceBuffer.from_host(a) for a in (inp[rows], res[rows], inp[rows], inp[rows]))
+        rnb.rms_norm_add_rms_norm_quantize_dev(x, pwd, 1e-6, r, qwd, 1e-5, n, hidden, o, post_unit_offset=unit, pre_unit_offset=unit)
+        rnb.rms_norm_dev(x, qwd, 1e-5, n, hidden, plain, unit_offset=unit)
+        rnb.sync()
+        out = [b.to_host(np.float32).reshape(n, hidden) for b in (r, o, plain)]
+        for b in (x, r, o, plain):
+            b.free()
+        return out
+
+    got = both(list(range(seq)))
+    for row in (0, 1, 255, seq - 1):
+        for a, b in zip(got, both([row])):
+            assert np.array_equal(a[row].view(np.uint32), b[0].view(np.uint32)), row
+    rel = 4e-6 if unit else 3e-7
+    assert _close(got[2].ravel(), oracle.rms_norm(inp.ravel(), qw, 1e-5, unit_offset=unit), rel)
+    assert _close(got[1].ravel(), oracle.rms_norm(got[0].ravel(), qw, 1e-5, unit_offset=unit), rel)
+    for b in (pwd, qwd):
+        b.free()
+
+
+@pytest.mark.gpu
 def test_rms_norm_rejects_bad_shapes(rnb):
     x = rnb.DeviceBuffer(4096)
     with pytest.raises(rnb.BackendError) as err:
