@@ -71,7 +71,7 @@ __device__ __forceinline__ TileUnit find_unit(uint32_t unit, uint32_t n_units, c
             return {g0 + at, (unit - __shfl(end - mine, at, kWave)) * toks};
         }
         unit -= __shfl(end, kWave - 1, kWave);
-        if (g0 + kWave >= n_groups) return {n_groups - 1, 0xffffffffu};  // not reached: the grid has n_units rows
+        if (g0 + kWave >= n_groups) return {n_groups - 1, 0xffffffffu};  // not reached: the launches have n_units rows
     }
 }
 
@@ -359,7 +359,8 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
                             const int8_t *__restrict__ aq, const float *__restrict__ ad, const uint8_t *__restrict__ adig,
                             const uint32_t *__restrict__ grp_expert, const uint32_t *__restrict__ grp_start, uint32_t n_groups,
                             const uint32_t *__restrict__ sorted_slot, const uint32_t *__restrict__ sorted_token,
-                            float *__restrict__ mid, uint32_t n_ff, uint32_t nb, uint32_t img_toks, uint32_t tiles_per_wg) {
+                            float *__restrict__ mid, uint32_t n_ff, uint32_t nb, uint32_t img_toks, uint32_t tiles_per_wg,
+                            uint32_t unit0, uint32_t n_units) {
     constexpr bool kFifth = false;
     constexpr int kPair = 2 * kQ4FillBytes;  // a gate strip and an up strip
     extern __shared__ __attribute__((aligned(16))) uint8_t s_dyn[];
@@ -371,7 +372,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
     const int lrow = lane & 31, khalf = lane >> 5;
     uint8_t *strips = s_dyn + wave * kPair;
     const uint32_t lds_strips = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)strips));
-    const TileUnit unit = find_unit(blockIdx.y, gridDim.y, grp_start, n_groups, img_toks, lane);
+    const TileUnit unit = find_unit(unit0 + blockIdx.y, n_units, grp_start, n_groups, img_toks, lane);
     const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
     const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
     if (tile0 >= count) return;
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(kGbThreads, 2)
                          const uint32_t *__restrict__ grp_expert,
                          const uint32_t *__restrict__ grp_start, uint32_t n_groups, const uint32_t *__restrict__ sorted_slot,
                          const float *__restrict__ slot_route, float *__restrict__ slot_out, uint32_t n_embd, uint32_t nb,
-                         uint32_t tiles_per_wg, uint32_t img_toks) {
+                         uint32_t tiles_per_wg, uint32_t img_toks, uint32_t unit0, uint32_t n_units) {
     constexpr bool kSix = kQuant == kQ6K;
     constexpr bool kFifth = kQuant == kQ5K;
     constexpr int kStride = kSix ? kGbStride64 : kGbStride128;
@@ -502,7 +503,7 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: the wave's row addresses are scalar bases plus lane offsets
     const int lrow = lane & 31, khalf = lane >> 5;
-    const TileUnit unit = find_unit(blockIdx.y, gridDim.y, grp_start, n_groups, img_toks, lane);
+    const TileUnit unit = find_unit(unit0 + blockIdx.y, n_units, grp_start, n_groups, img_toks, lane);
     const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
     const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
     if (tile0 >= count) return;
@@ -657,6 +658,7 @@ constexpr size_t kMmLdsLimit = 150 * 1024;
 constexpr size_t kMmLdsWide = 158 * 1024;  // for the eight-wave gate/up kernel (the token map is all it has besides)
 constexpr size_t kMmGateUpImageLimit = kMmLdsLimit - kMmGateUpStripBytes;
 constexpr size_t kMmQ6DownLdsLimit = kMmLdsLimit - kGbWaves * 32 * kQ6StripStride;
+constexpr uint32_t kMaxGridY = 65535;  // token tiles per launch: grid rows that a device is sure to take
 constexpr uint32_t kMmMinToks = 16;  // below this the matrix-core path re-reads the weights too often to pay
 
 template <int kStride, bool kDigits>
@@ -722,13 +724,15 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     }
     const size_t lds = static_cast<size_t>(waves) * 2 * kQ4FillBytes + image;
     const uint32_t rows_per_wg = 32 * waves, row_tiles = (n_ff + rows_per_wg - 1) / rows_per_wg;
-    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, units, 1);
+    const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
     // tiles of at most 8 / 16 / 32 tokens: the kernel finishes only that many results per lane
 #define RNB_LAUNCH_GUW(J, W)                                                                                          \
-    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, W == 8 ? kMmLdsWide : kMmLdsLimit)) return;                                   \
-    hipLaunchKernelGGL((moe_gate_up_mfma_kernel<J, W>), grid, dim3(kWave * W), lds, stream, gate_all, up_all, shared.gate, \
-                       shared.up, shared.n_routed, act.qs, act.d, act.digits, groups.expert, groups.start,            \
-                       groups.n_groups, groups.sorted_slot, groups.sorted_token, mid, n_ff, nb_in, toks, tiles_per_wg)
+    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, W == 8 ? kMmLdsWide : kMmLdsLimit)) return;             \
+    for (uint32_t u = 0; u < units; u += kMaxGridY)                                                                   \
+    hipLaunchKernelGGL((moe_gate_up_mfma_kernel<J, W>), dim3(wgs_x, std::min(units - u, kMaxGridY), 1), dim3(kWave * W), lds, \
+                       stream, gate_all, up_all, shared.gate, shared.up, shared.n_routed, act.qs, act.d, act.digits,  \
+                       groups.expert, groups.start, groups.n_groups, groups.sorted_slot, groups.sorted_token, mid,    \
+                       n_ff, nb_in, toks, tiles_per_wg, u, units)
     if (toks > 16 && waves == 8) {
         RNB_LAUNCH_GUW(4, 8);
     } else if (toks > 16) {
@@ -770,11 +774,13 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
         while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
             tiles_per_wg *= 2;
     }
-    const dim3 grid((row_tiles + tiles_per_wg - 1) / tiles_per_wg, units, 1), block(kGbThreads);
+    const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
 #define RNB_LAUNCH_DMJ(Q, J, LDS)                                                                                     \
     if (!allow_lds<static_cast<int>(Q) * 8 + J>(moe_down_mfma_kernel<Q, J>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
-    hipLaunchKernelGGL((moe_down_mfma_kernel<Q, J>), grid, block, LDS, stream, down_all, shared.down, shared.n_routed, mid, \
-                       groups.expert, groups.start, groups.n_groups, groups.sorted_slot, slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks)
+    for (uint32_t u = 0; u < units; u += kMaxGridY)                                                                   \
+    hipLaunchKernelGGL((moe_down_mfma_kernel<Q, J>), dim3(wgs_x, std::min(units - u, kMaxGridY), 1), dim3(kGbThreads), LDS, \
+                       stream, down_all, shared.down, shared.n_routed, mid, groups.expert, groups.start, groups.n_groups, \
+                       groups.sorted_slot, slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks, u, units)
 #define RNB_LAUNCH_DM(Q, LDS)                                                                                         \
     if (toks <= 8) {                                                                                                  \
         RNB_LAUNCH_DMJ(Q, 1, LDS);                                                                                    \

@@ -1402,6 +1402,32 @@ def test_moe_few_experts_take_most_tokens(rnb, oracle, tokens, n_ff, n_embd, dow
         rnb.release(w)
 
 
+def test_moe_more_token_tiles_than_grid_rows(rnb, oracle):
+    """60000 tokens routed to 36 of 64 experts each: 2.16 million slots, 67500 token tiles, more than a launch has grid rows
+    (65535).  Tokens and routes repeat every 48 tokens, so every output row is, bit for bit, that of a 48-token call."""
+    period, tokens, k, n_expert, n_ff, n_embd = 48, 60000, 36, 64, 256, 256
+    gate, up, down, *_ = _moe_case(oracle, n_expert, n_ff, n_embd, 1, 1, 1700, Q6_K)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((period, n_embd)).astype(np.float32)
+    expert = np.argsort(rng.random((period, n_expert)), axis=1)[:, :k].astype(np.uint32)
+    route = rng.uniform(0.01, 0.05, (period, k)).astype(np.float32)
+    bufs = [rnb.DeviceBuffer.from_host(w) for w in (gate, up, down)]
+    out = {}
+    for n in (period, tokens):
+        at = np.arange(n) % period
+        xd, od = rnb.DeviceBuffer.from_host(x[at]), rnb.DeviceBuffer(n * n_embd * 4)
+        print(f"{n} tokens, {n * k} slots", flush=True)
+        rnb.moe_sparse_experts_by_token_dev(*bufs, n_expert, expert[at].ravel(), route[at].ravel(),
+                                            np.repeat(np.arange(n, dtype=np.uint32), k), n, Q6_K, n_ff, n_embd, xd, od)
+        rnb.sync()
+        out[n] = od.to_host(np.uint32).reshape(n, n_embd)
+        xd.free(), od.free()
+    assert np.array_equal(out[tokens], out[period][np.arange(tokens) % period])
+    assert np.any(out[period])
+    for b in bufs:
+        b.free()
+
+
 @pytest.mark.parametrize("tokens,n_expert,k,n_ff,n_embd,down_quant,shared", [(64, 128, 8, 1024, 512, Q6_K, False),
                                                                             (48, 60, 8, 1280, 768, Q5_K, False),
                                                                             (100, 128, 2, 512, 256, Q4_K, False),
