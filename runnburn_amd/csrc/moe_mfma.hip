@@ -1,11 +1,11 @@
 // Gathered sparse-MoE experts for batches (prefill) on the matrix cores: the grouped form of gemm_blocks.hip.
-// Slots are sorted by expert on the host (api.cpp); workgroup (row tile, expert group) walks the group's slots in tiles
-// of 32 tokens: the tokens' quantised activations are gathered into LDS by the sorted lists, the expert's weight rows go
-// from global memory to the registers of the lane that owns the row, one int8 matrix instruction per scale group, the
-// group's scale on the vector units (see gemm_blocks.hip).  With a handful of tokens per expert most of a 32-token tile
-// is padding, which costs no arithmetic: the work per tile is the same whatever the number of live tokens, where the
-// integer-dot kernels of moe.hip cost per token (measured crossover on 128 experts x top-8: 64 tokens).  Padding costs
-// no LDS either: only the live tokens are staged, the matrix instruction's padding lanes read the last live token's
+// Slots are sorted by expert on the host (api.cpp) and every expert's group is cut into tiles of up to 32 tokens; workgroup
+// (row tiles, token tile of all groups): the tile's quantised activations are gathered into LDS by the sorted lists, the
+// expert's weight rows go from global memory to the registers of the lane that owns the row, one int8 matrix instruction
+// per scale group, the group's scale on the vector units (see gemm_blocks.hip).  With a handful of tokens per expert most of
+// a 32-token tile is padding, which costs no arithmetic: the work per tile is the same whatever the number of live tokens,
+// where the integer-dot kernels of moe.hip cost per token (measured crossover on 128 experts x top-8: 64 tokens).  Padding
+// costs no LDS either: only the live tokens are staged, the matrix instruction's padding lanes read the last live token's
 // row, and the launch sizes the image for the largest group of the call, so that several workgroups share a compute
 // unit when the groups are small.
 //   gate/up   mid[slot][n_ff] = silu(Wg[e] . a_tok) * (Wu[e] . a_tok), both Q4_K: the two matrices share the activation
@@ -701,7 +701,7 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
         // group the rule below is ahead, 64 tokens 114 against 120.)
         uint64_t best = ~0ull;
         for (const int w : {8, 4}) {
-            if (w == 8 && 8 * 2 * kQ4FillBytes + image > kMmLdsWide) continue;
+            if (w == 8 && (toks <= 16 || 8 * 2 * kQ4FillBytes + image > kMmLdsWide)) continue;  // no such kernel below 17 tokens
             const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
             for (uint32_t t = 1; t <= tiles && t <= 8; t++) {
                 const uint64_t wgs = static_cast<uint64_t>(units) * ((tiles + t - 1) / t);
