@@ -141,7 +141,9 @@ struct Rows<kQ6K> {
 // 36 -> 31, 4096 x 4096 x 192 40 -> 33; below: 4096 x 4096 x 128 27 against 32), Q5_K from 5e9 (14336 x 4096 x 96 41 ->
 // 37; 4096 x 4096 x 256 32 against 37), Q4_K, whose ping-pong kernel already folds the scales, from 18e9 (14336 x 4096 x 333
 // 79 -> 72, 26742 x 11264 x 117 111 -> 108; 14336 x 4096 x 256 47 against 55).  The last two lose where the last round of
-// workgroups is nearly empty (Q4_K 9289 x 6400 x 779, 259 workgroups: 143 against 152), see digits_fill_the_chip.
+// workgroups is nearly empty (Q4_K 9289 x 6400 x 779, 259 workgroups: 143 against 152), see digits_fill_the_chip.  Q4_K
+// gains nothing either where a workgroup is dealt two token tiles, the 64 tokens its ping-pong kernel makes operands for
+// (20284 x 7936 x 134 80.3 us against 82.7, 17567 x 11776 x 157 109 against 115); Q5_K does (20430 x 4352 x 191 74 -> 63).
 bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(w);
     const double macs = static_cast<double>(rows) * static_cast<double>(cols) * static_cast<double>(seq);
@@ -149,6 +151,8 @@ bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols
     if (quant == kQ6K) return a % 4 == 0 && macs >= 2.2e9;
     if (quant != kQ4K && quant != kQ5K) return false;
     if (a % 16 != 0 || macs < (quant == kQ4K ? 18e9 : 5e9)) return false;
+    if (quant == kQ4K && digits_plan(static_cast<uint32_t>(rows), static_cast<uint32_t>(cols / 256), static_cast<uint32_t>(seq)).tiles_per_wg == 2)
+        return false;
     return digits_fill_the_chip(static_cast<uint32_t>(rows), static_cast<uint32_t>(cols / 256), static_cast<uint32_t>(seq));
 }
 

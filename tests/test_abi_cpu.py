@@ -354,3 +354,18 @@ def test_partial_sums_of_the_prefill_gemms_are_bounded():
                 assert need <= 32 << 20, ("digits", rows, nb, seq, need)
                 sliced += need > 0
     assert sliced > 500
+
+
+def test_two_digit_gemm_route():
+    """Which prefill shapes take the two-digit GEMM: enough work, a full chip, weights aligned for it, and for Q4_K more than
+    two token tiles per workgroup."""
+    pays = _plan("_ZN3rnb16gemm_digits_paysEjPKhmmm", ctypes.c_bool, ctypes.c_uint32, ctypes.c_void_p, *[ctypes.c_size_t] * 3)
+    q4k, q5k, q6k = 12, 13, 14
+    assert pays(q4k, 256, 14336, 4096, 512) and pays(q5k, 256, 14336, 4096, 512) and pays(q6k, 256, 14336, 4096, 512)
+    assert not pays(q4k, 256 + 8, 14336, 4096, 512) and pays(q6k, 256 + 8, 14336, 4096, 512)  # 16- and 4-byte loads
+    assert not pays(q6k, 256 + 2, 14336, 4096, 512)
+    assert not any(pays(q, 256, 128256, 8192, 32) for q in (q4k, q5k, q6k))  # one token tile
+    assert not pays(q4k, 256, 14336, 4096, 256) and not pays(q5k, 256, 4096, 4096, 256) and not pays(q6k, 256, 4096, 4096, 128)
+    assert not pays(q4k, 256, 9289, 6400, 779)  # 259 workgroups
+    for rows, cols, seq in ((20284, 7936, 134), (17567, 11776, 157), (4628, 8448, 775)):  # 64 tokens per workgroup
+        assert not pays(q4k, 256, rows, cols, seq) and pays(q5k, 256, rows, cols, seq)
