@@ -143,7 +143,11 @@ struct Rows<kQ6K> {
 // 79 -> 72, 26742 x 11264 x 117 111 -> 108; 14336 x 4096 x 256 47 against 55).  The last two lose where the last round of
 // workgroups is nearly empty (Q4_K 9289 x 6400 x 779, 259 workgroups: 143 against 152), see digits_fill_the_chip.  Q4_K
 // gains nothing either where a workgroup is dealt two token tiles, the 64 tokens its ping-pong kernel makes operands for
-// (20284 x 7936 x 134 80.3 us against 82.7, 17567 x 11776 x 157 109 against 115); Q5_K does (20430 x 4352 x 191 74 -> 63).
+// (20284 x 7936 x 134 80.3 us against 82.7, 17567 x 11776 x 157 109 against 115); Q5_K does (20430 x 4352 x 191 74 -> 63),
+// but not on rows of fewer than 16 blocks: there the start of a workgroup wants four tiles behind it (10000 x 1280 x 1500
+// 85 -> 67) or one round of whole rows (threes of 8192 x 2048 x 700 53 -> 46), else it is behind (15360 x 1024 x 639 dealt in
+// threes 43.6 against 47.7, 13959 x 3328 x 513 in twos 97 against 101, 10850 x 3072 x 287 in one round of twos 46.6 against
+// 48.2, 4255 x 3328 x 658 in two slices 45 against 50).
 bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(w);
     const double macs = static_cast<double>(rows) * static_cast<double>(cols) * static_cast<double>(seq);
@@ -151,9 +155,11 @@ bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols
     if (quant == kQ6K) return a % 4 == 0 && macs >= 2.2e9;
     if (quant != kQ4K && quant != kQ5K) return false;
     if (a % 16 != 0 || macs < (quant == kQ4K ? 18e9 : 5e9)) return false;
-    if (quant == kQ4K && digits_plan(static_cast<uint32_t>(rows), static_cast<uint32_t>(cols / 256), static_cast<uint32_t>(seq)).tiles_per_wg == 2)
-        return false;
-    return digits_fill_the_chip(static_cast<uint32_t>(rows), static_cast<uint32_t>(cols / 256), static_cast<uint32_t>(seq));
+    const uint32_t r = static_cast<uint32_t>(rows), nb = static_cast<uint32_t>(cols / 256), q = static_cast<uint32_t>(seq);
+    const DgPlan p = digits_plan(r, nb, q);
+    const bool one_round = p.slices == 1 && static_cast<uint64_t>(p.row_tiles) * p.groups <= 256;
+    const uint32_t min_tiles = quant == kQ4K ? 3 : nb >= 16 ? 2 : one_round ? 3 : 4;
+    return p.tiles_per_wg >= min_tiles && digits_fill_the_chip(r, nb, q);
 }
 
 size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq) {

@@ -357,8 +357,8 @@ def test_partial_sums_of_the_prefill_gemms_are_bounded():
 
 
 def test_two_digit_gemm_route():
-    """Which prefill shapes take the two-digit GEMM: enough work, a full chip, weights aligned for it, and for Q4_K more than
-    two token tiles per workgroup."""
+    """Which prefill shapes take the two-digit GEMM: enough work, a full chip, weights aligned for it, and enough token
+    tiles per workgroup (Q4_K three, Q5_K's short rows four)."""
     pays = _plan("_ZN3rnb16gemm_digits_paysEjPKhmmm", ctypes.c_bool, ctypes.c_uint32, ctypes.c_void_p, *[ctypes.c_size_t] * 3)
     q4k, q5k, q6k = 12, 13, 14
     assert pays(q4k, 256, 14336, 4096, 512) and pays(q5k, 256, 14336, 4096, 512) and pays(q6k, 256, 14336, 4096, 512)
@@ -367,5 +367,9 @@ def test_two_digit_gemm_route():
     assert not any(pays(q, 256, 128256, 8192, 32) for q in (q4k, q5k, q6k))  # one token tile
     assert not pays(q4k, 256, 14336, 4096, 256) and not pays(q5k, 256, 4096, 4096, 256) and not pays(q6k, 256, 4096, 4096, 128)
     assert not pays(q4k, 256, 9289, 6400, 779)  # 259 workgroups
-    for rows, cols, seq in ((20284, 7936, 134), (17567, 11776, 157), (4628, 8448, 775)):  # 64 tokens per workgroup
+    for rows, cols, seq in ((20284, 7936, 134), (17567, 11776, 157), (4628, 8448, 775)):  # two tiles each
         assert not pays(q4k, 256, rows, cols, seq) and pays(q5k, 256, rows, cols, seq)
+    for rows, cols, seq in ((15360, 1280, 639), (20976, 1024, 1943), (13959, 3328, 513), (10850, 3072, 287),
+                            (4255, 3328, 658)):  # short rows
+        assert not pays(q5k, 256, rows, cols, seq) and pays(q6k, 256, rows, cols, seq)
+    assert pays(q5k, 256, 10000, 1280, 1500) and pays(q5k, 256, 8192, 2048, 700)
