@@ -1,3 +1,4 @@
+import ctypes
 import os
 import sys
 
@@ -29,3 +30,25 @@ def rnb():
     if not pkg.device_available():
         pytest.skip(f"no HIP device: {pkg.last_error()}")
     return pkg
+
+
+@pytest.fixture(scope="session")
+def host_plan():
+    """Host-side planning functions of the library (C++ linkage, no device needed), by mangled name and signature."""
+    import runnburn_amd as pkg
+
+    def bind(symbol, restype, *argtypes):
+        fn = getattr(pkg.lib(), symbol)
+        fn.restype, fn.argtypes = restype, list(argtypes)
+        return fn
+
+    return bind
+
+
+@pytest.fixture(scope="session")
+def two_digit_route(host_plan):
+    """pays(quant, weight address, rows, cols, tokens): whether a K-quant / an importance-quant shape takes the two-digit GEMM."""
+    sig = (ctypes.c_bool, ctypes.c_uint32, ctypes.c_void_p, *[ctypes.c_size_t] * 3)
+    k_quants = host_plan("_ZN3rnb16gemm_digits_paysEjPKhmmm", *sig)
+    importance = host_plan("_ZN3rnb19gemm_iq_digits_paysEjPKhmmm", *sig)
+    return lambda quant, *args: (importance if quant >= 16 else k_quants)(quant, *args)

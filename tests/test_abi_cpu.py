@@ -329,19 +329,12 @@ def test_kernels_of_the_32_element_gemm_keep_their_registers():
     assert not any(found.values()), {name: size for name, size in found.items() if size}
 
 
-def _plan(symbol, restype, *argtypes):
-    """A host-side planning function of the library (C++ linkage)."""
-    fn = getattr(rnb.lib(), symbol)
-    fn.restype, fn.argtypes = restype, list(argtypes)
-    return fn
-
-
-def test_partial_sums_of_the_prefill_gemms_are_bounded():
+def test_partial_sums_of_the_prefill_gemms_are_bounded(host_plan):
     """Batches of more than 32 tokens: the K slices of the 32-element formats' GEMM and of the two-digit GEMM write at most
     32 MiB of partial sums, so the workspace that outlives the call has a bound whatever the shape."""
     u32 = ctypes.c_uint32
-    blocks = _plan("_ZN3rnb24gemm_blocks_slice_floatsEjjjj", ctypes.c_size_t, u32, u32, u32, u32)
-    digits = _plan("_ZN3rnb24gemm_digits_slice_floatsEjjj", ctypes.c_size_t, u32, u32, u32)
+    blocks = host_plan("_ZN3rnb24gemm_blocks_slice_floatsEjjjj", ctypes.c_size_t, u32, u32, u32, u32)
+    digits = host_plan("_ZN3rnb24gemm_digits_slice_floatsEjjj", ctypes.c_size_t, u32, u32, u32)
     sliced = 0
     for rows in (1, 127, 512, 2048, 4096, 9289, 17920, 28672, 128256):
         for nb in (1, 4, 16, 25, 56, 64):  # super-blocks of a row, the 256-element steps of a 32-element format
@@ -356,10 +349,10 @@ def test_partial_sums_of_the_prefill_gemms_are_bounded():
     assert sliced > 500
 
 
-def test_two_digit_gemm_route():
+def test_two_digit_gemm_route(two_digit_route):
     """Which prefill shapes take the two-digit GEMM: enough work, a full chip, weights aligned for it, and enough token
     tiles per workgroup (Q4_K three, Q5_K's short rows four)."""
-    pays = _plan("_ZN3rnb16gemm_digits_paysEjPKhmmm", ctypes.c_bool, ctypes.c_uint32, ctypes.c_void_p, *[ctypes.c_size_t] * 3)
+    pays = two_digit_route
     q4k, q5k, q6k = 12, 13, 14
     assert pays(q4k, 256, 14336, 4096, 512) and pays(q5k, 256, 14336, 4096, 512) and pays(q6k, 256, 14336, 4096, 512)
     assert not pays(q4k, 256 + 8, 14336, 4096, 512) and pays(q6k, 256 + 8, 14336, 4096, 512)  # 16- and 4-byte loads

@@ -563,13 +563,15 @@ def test_gemm_k_slices(rnb, oracle, quant, rows, nblk, seq):
 @pytest.mark.parametrize("quant,rows,nblk,seq", [(Q6_K, 8451, 11, 97), (Q6_K, 2111, 56, 75), (Q6_K, 40000, 7, 33),
                                                  (Q5_K, 16385, 17, 71), (Q5_K, 4071, 40, 130), (Q4_K, 16500, 16, 273),
                                                  (Q4_K, 8500, 25, 333), (Q4_K, 16385, 9, 491)])
-def test_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
+def test_gemm_two_digit_operands(rnb, oracle, two_digit_route, quant, rows, nblk, seq):
     """Enough work for the GEMM that makes a super-block's operands once for up to 128 tokens: two, three and four token tiles
     per workgroup, a last wave of one row, a last group of one token, K slices of unequal length, Q6_K rows of an odd
     number of blocks (every other one off a 4-byte boundary).  Rows at both ends, around the 32- and 256-row tile edges and
-    spread between against the oracle, the tight bound of the module; extreme scales and codes in three of them; a token's
-    row has the same bits in the reversed batch."""
+    spread between against the oracle, the tight bound of the module; extreme scales and codes in three of them; every row
+    of four tokens against the one-token kernel (twice the bound: both are within it of the f64 sum); a token's row has the
+    same bits in the reversed batch."""
     cols = nblk * 256
+    assert two_digit_route(quant, 256, rows, cols, seq), "another kernel's shape"
     w = oracle.make_weights(quant, rows, cols, 70 + rows).copy()
     per_row = w.size // rows
     rng = np.random.default_rng(rows)
@@ -588,6 +590,11 @@ def test_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
     ref, gold = (oracle.gemv(quant, ws, len(pick), cols, x, gold=g).reshape(seq, len(pick)) for g in (False, True))
     for i, r in enumerate(pick):
         check_close(got[:, r], ref[:, i], gold[:, i], f"quant {quant} rows {rows} nblk {nblk} seq {seq} row {r}")
+    rms = np.sqrt(np.mean(got.astype(np.float64) ** 2, axis=0))
+    for t in (0, 31, 32, seq - 1):
+        one = gemv_fn(rnb, quant)(w, rows, cols, x[t])
+        off = np.flatnonzero(np.abs(got[t].astype(np.float64) - one) > 2 * TIGHT * rms)
+        assert off.size == 0, f"token {t}: rows {off[:8]} differ from the one-token kernel"
     rev = gemv_fn(rnb, quant, True)(w, rows, cols, x[::-1].copy())
     assert np.array_equal(rev[::-1], got)
     rnb.release(w)
@@ -614,10 +621,10 @@ def test_q2k_q3k_gemm_mfma_ragged_tiles(rnb, oracle, quant, rows, nblk, seq):
 @pytest.mark.parametrize("rows,cols,seq", [(32, 32, 17), (31, 96, 17), (33, 1056, 33), (130, 2080, 64), (257, 256, 65),
                                            (1, 4096, 17), (300, 288, 100)])
 def test_q8_gemm_mfma_ragged_tiles(rnb, oracle, quant, rows, cols, seq):
-    """Batches on the 32-element formats take the matrix-core GEMM (one K=32 instruction per block, the two f32 scales
-    on the vector units; the nibble formats' codes are split, given their fifth bit and offset in packed bytes, the
-    d n + m formats add m times the block's sum of activations from a second instruction against ones): block counts off
-    the 8-block step, rows and tokens off the tile."""
+    """Batches on the 32-element formats take the matrix-core GEMM (one K=32 instruction per block; the products of the two
+    f32 scales from a K=1 instruction over two blocks, or on the vector units for up to 16 tokens; the nibble formats' codes
+    are split, given their fifth bit and offset in packed bytes, the d n + m formats add m times the block's sum of
+    activations from a second instruction against ones): block counts off the 8-block step, rows and tokens off the tile."""
     w = oracle.make_weights(quant, rows, cols, 270 + rows)
     x = oracle.fill_normal(seq * cols, 280 + seq, 1.0)
     got = gemv_fn(rnb, quant, True)(w, rows, cols, x)

@@ -76,12 +76,14 @@ def test_iq_gemm_matrix_cores(rnb, oracle, quant, rows, cols, seq):
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant", [IQ2_XXS, IQ2_S, IQ3_XXS, IQ4_XS])
 @pytest.mark.parametrize("rows,nblk,seq", [(2111, 56, 75), (49153, 6, 33), (16385, 13, 75), (12545, 3, 510)])
-def test_iq_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
+def test_iq_gemm_two_digit_operands(rnb, oracle, two_digit_route, quant, rows, nblk, seq):
     """Enough work for the GEMM that makes a block's operands once for up to 128 tokens: two, three and four token tiles per
     workgroup, K slices, a last wave of one row.  Blocks of random bytes in a third of the rows (every grid index, sign
-    pattern and scale), rows at the tile edges and spread between against the oracle; a token's row has the same bits in
-    the reversed batch."""
+    pattern and scale), rows at the tile edges and spread between against the oracle; every row of four tokens against the
+    one-token kernel (twice the bound: both are within it of the f64 sum); a token's row has the same bits in the reversed
+    batch."""
     cols = nblk * 256
+    assert two_digit_route(quant, 256, rows, cols, seq), "another kernel's shape"
     w = oracle.make_weights(quant, rows, cols, 1700 + quant + rows).copy().reshape(rows, nblk, -1)
     rng = np.random.default_rng(rows)
     w[::3, :, 2:] = rng.integers(0, 256, size=w[::3, :, 2:].shape, dtype=np.uint8)
@@ -95,6 +97,11 @@ def test_iq_gemm_two_digit_operands(rnb, oracle, quant, rows, nblk, seq):
     ref, gold = (np.asarray(oracle.gemv(quant, ws, len(pick), cols, x, gold=g)).reshape(seq, len(pick)) for g in (False, True))
     for i, r in enumerate(pick):
         _check(got[:, r], ref[:, i], gold[:, i], f"{LABEL[quant]} {rows}x{cols}x{seq} row {r}")
+    rms = np.sqrt(np.mean(got.astype(np.float64) ** 2, axis=0))
+    for t in (0, 31, 32, seq - 1):
+        one = np.asarray(_fns(rnb, quant)[0](w, rows, cols, x[t]), np.float64).ravel()
+        off = np.flatnonzero(np.abs(got[t] - one) > 2 * TIGHT * rms)
+        assert off.size == 0, f"token {t}: rows {off[:8]} differ from the one-token kernel"
     rev = _fns(rnb, quant)[1](w, rows, cols, x[::-1].copy()).reshape(seq, rows)
     assert np.array_equal(rev[::-1], got)
     rnb.release(w)
