@@ -765,7 +765,7 @@ def main() -> int:
         result["roofline_gemm"] = {
             "bound": "mfma", "achieved": tops, "peak": INT8_PEAK_TOPS, "unit": "TOP/s", "frac": tops / INT8_PEAK_TOPS,
             "traffic": None, "workload": "configs[3]: Q4_K prefill GEMM, 512 tokens x 4096 -> 14336",
-            "kernel": "gemm_q4k_mfma_kernel (Q4_K x Q8_K on v_mfma_i32_32x32x32_i8)", "ops_per_launch": ops,
+            "kernel": "gemm_digits_kernel<Q4_K, 4> (Q4_K x Q8_K on v_mfma_i32_32x32x32_i8)", "ops_per_launch": ops,
             "kernel_ms_mean": pq["mean"], "kernel_ms_median": pq["median"], "kernel_ms_p10": pq["p10"],
             "kernel_ms_p90": pq["p90"], "launches": pq["launches"],
             "step_ms_median": res4["step"]["median"], "step": "activation quantiser (512 x 4096 f32 -> Q8_K) + GEMM"}

@@ -1100,9 +1100,12 @@ static bool is_b32(uint32_t quant) {
     return quant == kQ8_0 || quant == kQ8_1 || quant == kQ4_0 || quant == kQ4_1 || quant == kQ5_0 || quant == kQ5_1;
 }
 
-// Q6_K spends the most vector work per tile, and the 64-token form saves the most of it: it also wins where its
-// workgroups fill the 256 compute units just once (4096 rows x 512 tokens x 14336: 164 vs 189 us; with 224 or 320
-// workgroups the 32-token form is level or ahead)
+// Q6_K spends the most vector work per tile, and the 64-token form saves the most of it.  From 2.2e9 multiply-adds on the
+// two-digit GEMM takes weights at 4-byte addresses (gemm_digits_pays), which leaves this form the large batches on short rows
+// (8192 x 512 x 512 tokens 19.2 us against 23.2, 16384 x 512 x 256 18.9 : 22.3, 4096 x 256 x 1024 14.3 : 16.7) and weights at
+// other addresses, parts of a resident tensor: there it also wins where its workgroups fill the 256 compute units just once
+// (4096 rows x 512 tokens x 14336: 164 vs 189 us; with 224 or 320 workgroups the 32-token form is level or ahead, and on
+// rows of up to 1024 both are level)
 static bool q6_wide_tiles(uint32_t row_tiles, uint32_t seq) {
     const uint64_t tiles = static_cast<uint64_t>(row_tiles) * ((seq + 63) / 64);
     return seq > 32 && (tiles >= 512 || (tiles > 224 && tiles <= 256));
