@@ -1114,16 +1114,21 @@ static bool q6_wide_tiles(uint32_t row_tiles, uint32_t seq) {
 // The 64-token form of the 32-element formats: two workgroups fit a compute unit, so 512 run at once and 576 take two
 // rounds.  The number of slices with the least of rounds * (steps + about one for the ends) plus the sum of the slices (about
 // one step's time and what its reads take).  4096 x 4096 x 333 tokens, 192 workgroups: 2 slices instead of 3, 8 steps in a row
-// instead of 12; 4096 x 14336 x 300 135 -> 112 us, 9289 x 6400 x 200 120 -> 108.  The partial sums stay within
+// instead of 12; 4096 x 14336 x 300 135 -> 112 us, 9289 x 6400 x 200 120 -> 108; Q4_0 5468 x 6752 x 93, 516
+// workgroups of which the last 86 have two steps of five, 73 -> 63 against 430 of six.  The partial sums stay within
 // kSliceScratchBytes: the workspace is kept for the next call.
 static uint32_t b32_wide_slices(uint64_t wgs, uint32_t steps, uint32_t rows, uint32_t seq) {
     uint32_t best = 1;
     double best_cost = 1e30;
     for (uint32_t s = 1; s <= kSliceMax && s <= std::max(1u, steps / 2); s++) {
         if (s > 1 && static_cast<uint64_t>(s) * rows * seq * sizeof(float) > kSliceScratchBytes) break;
-        const double rounds = static_cast<double>((wgs * s + 511) / 512), per = (steps + s - 1) / s;
+        const uint32_t per = (steps + s - 1) / s, last = steps % per;  // slices of `per` steps and, where it is not 0, one of `last`
+        const uint64_t full = wgs * (steps / per), rounds = (full + 511) / 512, spare = rounds * 512 - full;
+        // the last slice's workgroups are dispatched last: one after the other into the places that the full ones leave, the
+        // rest in rounds of their own
+        const uint64_t fit = spare * ((per + 1) / (last + 1)), left = last == 0 || wgs <= fit ? 0 : wgs - fit;
         const double sum = s > 1 ? 1.0 + s * static_cast<double>(rows) * seq * 4.0 / 12e6 : 0.0;  // 12 MB in a step's time
-        const double cost = rounds * (per + 1.0) + sum;
+        const double cost = static_cast<double>(rounds * (per + 1) + (left + 511) / 512 * (last + 1)) + sum;
         if (cost < best_cost) best_cost = cost, best = s;
     }
     return best;
