@@ -282,7 +282,7 @@ int rnb_hip_gemv_dev(uint32_t quant, const void *w_dev, size_t rows, size_t cols
  * that forbid hipMalloc).  No counterpart in the reference.  Same arguments, arithmetic and results as
  * rnb_hip_gemv_dev, but the quantised activations and the K-slice partial sums live in fixed arrays, held until the
  * process ends, instead of the grow-only scratch, so the call never allocates or frees device memory:
- * rnb_hip_gemv_dev_noalloc_scratch_bytes() bytes inside the library's code object, and 32 MiB, allocated when the library
+ * rnb_hip_gemv_dev_noalloc_scratch_bytes() bytes inside the library's code object, and 128 MiB, allocated when the library
  * opens the GPU, for the partial sums of the prefill GEMMs that bound theirs to that (the 32-element formats, and the other
  * formats' large batches).  Shapes that need more of the first array than it holds are rejected with
  * RNB_HIP_INVALID_REQUEST (about 1.32 bytes per activation element, seq_len * cols, plus slices * seq_len * rows * 4 for

@@ -153,8 +153,10 @@ size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq);
 void launch_gemm_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
                         uint32_t seq, hipStream_t stream);
 
-// Bound on the partial sums of launch_gemm_digits, launch_gemm_iq_digits and launch_gemm_q8_mfma, whatever the shape.
-constexpr size_t kSliceScratchBytes = size_t(32) << 20;
+// Bound on the partial sums of launch_gemm_digits, launch_gemm_iq_digits and launch_gemm_q8_mfma, whatever the shape (at 32 MiB a
+// tenth of the 32-element formats' prefill shapes lose a slice, Q5_1 7110 x 12032 x 904 tokens 522 -> 615 us; at 128 MiB one
+// in a hundred).
+constexpr size_t kSliceScratchBytes = size_t(128) << 20;
 // out[i] = parts[0][i] + parts[1][i] + ... in that order (n floats per slice)
 void launch_sum_slices(const float *parts, float *out, size_t n, uint32_t slices, hipStream_t stream);
 

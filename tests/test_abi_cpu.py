@@ -330,8 +330,8 @@ def test_kernels_of_the_32_element_gemm_keep_their_registers():
 
 
 def test_partial_sums_of_the_prefill_gemms_are_bounded(host_plan):
-    """Batches of more than 32 tokens: the K slices of the 32-element formats' GEMM and of the two-digit GEMM write at most
-    32 MiB of partial sums, so the workspace that outlives the call has a bound whatever the shape."""
+    """Batches of more than 32 tokens: the K slices of the 32-element formats' GEMM write at most 128 MiB of partial sums, the
+    two-digit GEMM's 32 MiB, so the workspace that outlives the call has a bound whatever the shape."""
     u32 = ctypes.c_uint32
     blocks = host_plan("_ZN3rnb24gemm_blocks_slice_floatsEjjjj", ctypes.c_size_t, u32, u32, u32, u32)
     digits = host_plan("_ZN3rnb24gemm_digits_slice_floatsEjjj", ctypes.c_size_t, u32, u32, u32)
@@ -341,7 +341,7 @@ def test_partial_sums_of_the_prefill_gemms_are_bounded(host_plan):
             for seq in (33, 65, 128, 200, 333, 512, 1024, 2048, 16384):
                 for quant in (2, 3, 6, 7, 8, 9):
                     need = 4 * blocks(quant, rows, nb, seq)
-                    assert need <= 32 << 20, (quant, rows, nb, seq, need)
+                    assert need <= 128 << 20, (quant, rows, nb, seq, need)
                     sliced += need > 0
                 need = 4 * digits(rows, nb, seq)
                 assert need <= 32 << 20, ("digits", rows, nb, seq, need)
