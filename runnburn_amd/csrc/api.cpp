@@ -91,7 +91,7 @@ size_t gemm_min_seq(uint32_t quant, size_t rows, size_t cols) {
     }
 }
 // The Q8_K quantiser adds the per-32 sums as two digits (the Q4_K / Q5_K GEMMs' mins term) from this many tokens on.
-constexpr size_t kDigitsMinSeq = 4;  // the smallest value gemm_min_seq returns
+constexpr size_t kDigitsMinSeq = 3;  // the fewest tokens gemm_few_pays answers for
 // Minimum tokens for which the importance-quant formats take their matrix-core GEMM instead of the GEMV that dots a
 // decoded block against up to four tokens (14336 x 4096, 4 tokens: 20.8 - 22.9 us against 21.8 - 25.8; 5 tokens: 29 - 35
 // against 21.5 - 25.7).
@@ -273,6 +273,9 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         } else {
             launch_gemv_iq(w_dev, quant, act, out_dev, r, nb, q, s.stream);
         }
+    } else if (gemm_few_supported(quant, w_dev, rows, nb, seq) && gemm_few_pays(quant, rows, nb, seq) &&
+               (quant == kQ6K || act.digits != nullptr)) {
+        launch_gemm_few(w_dev, quant, act, out_dev, r, nb, q, s.stream);
     } else if (gemm_digits_pays(quant, w_dev, rows, cols, seq) && (quant == kQ6K || act.digits != nullptr)) {
         if (int st = bounded_slices(gemm_digits_slice_floats(r, nb, q), &ws); st != RNB_HIP_OK) return st;
         launch_gemm_digits(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
@@ -501,7 +504,14 @@ int run_dense_ffn_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, 
     }
     st = quantize_activations(s, kQ4K, x_dev, seq, n_embd, &act);
     if (st != RNB_HIP_OK) return st;
-    if (small) {
+    // gate and up in one launch of the few-token GEMM: four tokens 36.5 us against the pair's 44 for the whole layer, three 36.4
+    // against 34.2 (rows of more than 16 blocks, which the paired GEMV does not take: 18.8 against 22.6)
+    const bool few = gemm_few_pays(kQ4K, n_ff, nb_in, seq) && (seq > 3 || nb_in > 16) && act.digits != nullptr &&
+                     gemm_few_supported(kQ4K, gate_dev, n_ff, nb_in, seq) && gemm_few_supported(kQ4K, up_dev, n_ff, nb_in, seq);
+    if (few) {
+        launch_gemm_few_gate_up(gate_dev, up_dev, act, s.ffn_mid.as<float>(), static_cast<uint32_t>(n_ff),
+                                static_cast<uint32_t>(nb_in), static_cast<uint32_t>(seq), gelu, s.stream);
+    } else if (small) {
         launch_gemv_q4k_gate_up(gate_dev, up_dev, act, s.ffn_mid.as<float>(), static_cast<uint32_t>(n_ff),
                                 static_cast<uint32_t>(nb_in), static_cast<uint32_t>(seq), gelu, s.stream);
     } else {

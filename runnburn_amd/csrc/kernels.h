@@ -153,6 +153,15 @@ size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq);
 void launch_gemm_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
                         uint32_t seq, hipStream_t stream);
 
+// Q4_K, Q5_K and Q6_K against at most 32 tokens, the K slices inside a workgroup: no workspace (act needs digits for Q4_K /
+// Q5_K); the gate_up form is mid = act(Wg a) * (Wu a) on Q4_K
+bool gemm_few_pays(uint32_t quant, size_t rows, size_t nb, size_t seq);
+bool gemm_few_supported(uint32_t quant, const uint8_t *w, size_t rows, size_t nb, size_t seq);
+void launch_gemm_few(const uint8_t *w, uint32_t quant, ActView act, float *out, uint32_t rows, uint32_t nb, uint32_t seq,
+                     hipStream_t stream);
+void launch_gemm_few_gate_up(const uint8_t *wg, const uint8_t *wu, ActView act, float *mid, uint32_t rows, uint32_t nb,
+                             uint32_t seq, bool gelu, hipStream_t stream);
+
 // Bound on the partial sums of launch_gemm_digits, launch_gemm_iq_digits and launch_gemm_q8_mfma, whatever the shape (at 32 MiB a
 // tenth of the 32-element formats' prefill shapes lose a slice, Q5_1 7110 x 12032 x 904 tokens 522 -> 615 us; at 128 MiB one
 // in a hundred).
