@@ -316,6 +316,9 @@ int run_matmul_quantized_dev(State &s, uint32_t quant, const uint8_t *w_dev, siz
         } else {
             launch_gemv_q6k(w_dev, act, out_dev, r, nb, q, s.stream);
         }
+    } else if (gemm_b32_pays(quant, w_dev, rows, cols, seq)) {
+        if (int st = bounded_slices(gemm_b32_slice_floats(quant, r, nb, q), &ws); st != RNB_HIP_OK) return st;
+        launch_gemm_b32(w_dev, quant, act, out_dev, ws, r, nb, q, s.stream);
     } else if (seq >= min_gemm_seq && gemm_q8_mfma_supported(quant, static_cast<uint32_t>(cols / 32))) {
         const uint32_t nb32 = static_cast<uint32_t>(cols / 32);
         if (int st = bounded_slices(gemm_blocks_slice_floats(quant, r, (nb32 + 7) / 8, q), &ws); st != RNB_HIP_OK) return st;

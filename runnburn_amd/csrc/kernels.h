@@ -162,6 +162,12 @@ void launch_gemm_few(const uint8_t *w, uint32_t quant, ActView act, float *out, 
 void launch_gemm_few_gate_up(const uint8_t *wg, const uint8_t *wu, ActView act, float *mid, uint32_t rows, uint32_t nb,
                              uint32_t seq, bool gelu, hipStream_t stream);
 
+// 32-element formats, batches of more than 32 tokens on rows of whole 256-element steps (nb of them)
+bool gemm_b32_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq);
+size_t gemm_b32_slice_floats(uint32_t quant, uint32_t rows, uint32_t nb, uint32_t seq);
+void launch_gemm_b32(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
+                     uint32_t seq, hipStream_t stream);
+
 // Bound on the partial sums of launch_gemm_digits, launch_gemm_iq_digits and launch_gemm_q8_mfma, whatever the shape (at 32 MiB a
 // tenth of the 32-element formats' prefill shapes lose a slice, Q5_1 7110 x 12032 x 904 tokens 522 -> 615 us; at 128 MiB one
 // in a hundred).
