@@ -135,6 +135,24 @@ __device__ __forceinline__ int byte_of(uint32_t lo, uint32_t hi, int j) {
     return static_cast<int>((wsel >> ((j & 3) * 8)) & 0xffu);
 }
 
+// A GEMM's launch can carry two matrices of the same shape (kPair: the gate and up halves of a gated FFN): grid.x = row tiles of
+// both, results [slice][matrix][seq][rows].  Returns the workgroup's row tile; `out` becomes its slice's and matrix's.
+template <bool kPair, typename Weights, typename Out>
+__device__ __forceinline__ uint32_t gemm_matrix(Weights &w, const uint8_t *w2, Out &out, uint32_t rows, uint32_t seq,
+                                                uint32_t rows_per_wg) {
+    uint32_t tile = blockIdx.x, slot = blockIdx.z;
+    if constexpr (kPair) {
+        const uint32_t tiles = (rows + rows_per_wg - 1) / rows_per_wg;
+        slot = 2 * slot + (tile >= tiles ? 1 : 0);
+        if (tile >= tiles) {
+            w = w2;
+            tile -= tiles;
+        }
+    }
+    out += static_cast<size_t>(slot) * seq * rows;
+    return tile;
+}
+
 // Expert `e` of one projection: routed experts lie back to back in `all` (base + e * bytes_per_expert, the slicing of
 // crates/rnb-llm/src/engine/models/shared_expert_moe/moe_view/fanout.rs:4-22); ids from n_routed up name the shared
 // expert, a tensor of its own (fanout.rs:804-812).

@@ -464,11 +464,11 @@ __global__ void __launch_bounds__(kGbThreads, 2)
 // quantiser's digits (bsum32 = b0 + 64 * b1): two K=16 instructions with eight live K slots per token tile.
 // Per super-block out += d_x * (d * float(tot) - dmin * float(S)): crates/rnb-cpu/src/gemm/neon_dot.rs:1742-1800.
 // ---------------------------------------------------------------------------------------------
-template <int kTT, bool kFifth, int kLive>
+template <int kTT, bool kFifth, int kLive, bool kPair>
 __global__ void __launch_bounds__(kGbThreads, 2)
-    gemm_q45k_mfma_kernel(const uint8_t *__restrict__ w, const int8_t *__restrict__ aq, const float *__restrict__ ad,
-                         const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows, uint32_t nb,
-                         uint32_t seq, uint32_t nb_slice) {
+    gemm_q45k_mfma_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, const int8_t *__restrict__ aq,
+                          const float *__restrict__ ad, const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows,
+                          uint32_t nb, uint32_t seq, uint32_t nb_slice) {
     constexpr int kToks = 32 * kTT;
     __shared__ __attribute__((aligned(16))) uint8_t s_a[2][kToks * kGbStride128];
     __shared__ __attribute__((aligned(16))) float s_dx[2][kToks];
@@ -476,7 +476,8 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1), wave = tid >> 6;
     const int lrow = lane & 31, khalf = lane >> 5;
-    const uint32_t row = blockIdx.x * kGbRows + wave * 32 + lrow;
+    const uint32_t row_tile = gemm_matrix<kPair>(w, w2, out, rows, seq, kGbRows);
+    const uint32_t row = row_tile * kGbRows + wave * 32 + lrow;
     const uint32_t tok0 = blockIdx.y * kToks, last_tok = seq - 1;
     constexpr size_t kBlockBytes = kFifth ? kQ5KBytes : kQ4KBytes;
     const uint8_t *wrow = w + static_cast<size_t>(min(row, rows - 1)) * nb * kBlockBytes;
@@ -512,7 +513,6 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     };
     // K slice of this workgroup (blockIdx.z): blocks b0 .. b1, its sums go to the slice's own copy of the output
     const uint32_t b0 = blockIdx.z * nb_slice, b1 = min(nb, b0 + nb_slice);
-    out += static_cast<size_t>(blockIdx.z) * seq * rows;
     stage_load5(b0);
     Q5Row cur = q45_load_row<kFifth>(wrow + static_cast<size_t>(b0) * kBlockBytes, khalf);
     stage_store5(0);
@@ -1096,6 +1096,13 @@ void launch_sum_slices(const float *parts, float *out, size_t n, uint32_t slices
 #undef RNB_SUM
 }
 
+void finish_slices(const float *parts, float *out, size_t n, uint32_t slices, uint32_t *left, hipStream_t stream) {
+    if (left != nullptr)
+        *left = slices;
+    else if (slices > 1)
+        launch_sum_slices(parts, out, n, slices, stream);
+}
+
 static bool is_b32(uint32_t quant) {
     return quant == kQ8_0 || quant == kQ8_1 || quant == kQ4_0 || quant == kQ4_1 || quant == kQ5_0 || quant == kQ5_1;
 }
@@ -1216,38 +1223,42 @@ void launch_gemm_q23k_mfma(const uint8_t *w, uint32_t quant, ActView act, float 
     if (nz > 1) launch_sum_slices(slice_out, out, static_cast<size_t>(seq) * rows, nz, stream);
 }
 
-template <bool kFifth>
-static void launch_gemm_q45k(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                             uint32_t seq, hipStream_t stream) {
+template <bool kFifth, bool kPair>
+static void launch_gemm_q45k(const uint8_t *w, const uint8_t *w2, ActView act, float *out, float *slice_out, uint32_t rows,
+                             uint32_t nb, uint32_t seq, uint32_t *left, hipStream_t stream) {
     if (rows == 0 || seq == 0 || nb == 0) return;
-    const uint32_t row_tiles = (rows + kGbRows - 1) / kGbRows;
+    constexpr uint32_t mats = kPair ? 2 : 1;
+    const uint32_t row_tiles = mats * ((rows + kGbRows - 1) / kGbRows);
     const bool wide = wide_tiles(row_tiles, seq);
-    const uint32_t slices = slice_out ? k_slices(tile_grid(rows, seq, wide), nb, false) : 1;
+    const uint32_t slices = slice_out ? k_slices(tile_grid(mats * rows, seq, wide), nb, false) : 1;
     const uint32_t nb_slice = (nb + slices - 1) / slices, nz = (nb + nb_slice - 1) / nb_slice;
     float *dst = nz > 1 ? slice_out : out;
     if (wide) {
         const dim3 grid(row_tiles, (seq + 63) / 64, nz);
-        hipLaunchKernelGGL((gemm_q45k_mfma_kernel<2, kFifth, 16>), grid, dim3(kGbThreads), 0, stream, w, act.qs, act.d,
+        hipLaunchKernelGGL((gemm_q45k_mfma_kernel<2, kFifth, 16, kPair>), grid, dim3(kGbThreads), 0, stream, w, w2, act.qs, act.d,
                            act.digits, dst, rows, nb, seq, nb_slice);
     } else {
         const dim3 grid(row_tiles, (seq + 31) / 32, nz);
 #define RNB_LAUNCH_Q45(LIVE)                                                                                           \
-    hipLaunchKernelGGL((gemm_q45k_mfma_kernel<1, kFifth, LIVE>), grid, dim3(kGbThreads), 0, stream, w, act.qs, act.d,  \
+    hipLaunchKernelGGL((gemm_q45k_mfma_kernel<1, kFifth, LIVE, kPair>), grid, dim3(kGbThreads), 0, stream, w, w2, act.qs, act.d,  \
                        act.digits, dst, rows, nb, seq, nb_slice)
         RNB_BY_LIVE_TOKENS(seq, RNB_LAUNCH_Q45);
 #undef RNB_LAUNCH_Q45
     }
-    if (nz > 1) launch_sum_slices(slice_out, out, static_cast<size_t>(seq) * rows, nz, stream);
+    finish_slices(slice_out, out, static_cast<size_t>(mats) * seq * rows, nz, left, stream);
 }
 
 void launch_gemm_q5k_mfma(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
                           uint32_t seq, hipStream_t stream) {
-    launch_gemm_q45k<true>(w, act, out, slice_out, rows, nb, seq, stream);
+    launch_gemm_q45k<true, false>(w, nullptr, act, out, slice_out, rows, nb, seq, nullptr, stream);
 }
 
 void launch_gemm_q4k_small(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                           uint32_t seq, hipStream_t stream) {
-    launch_gemm_q45k<false>(w, act, out, slice_out, rows, nb, seq, stream);
+                           uint32_t seq, hipStream_t stream, const uint8_t *w2, uint32_t *left) {
+    if (w2 != nullptr)
+        launch_gemm_q45k<false, true>(w, w2, act, out, slice_out, rows, nb, seq, left, stream);
+    else
+        launch_gemm_q45k<false, false>(w, nullptr, act, out, slice_out, rows, nb, seq, nullptr, stream);
 }
 
 bool gemm_q8_mfma_supported(uint32_t quant, uint32_t nb32) { return is_b32(quant) && nb32 >= 1; }

@@ -99,11 +99,11 @@ struct DgLds {
     static_assert(kBytes <= 160 * 1024, "LDS of a compute unit");
 };
 
-template <uint32_t kFmt, int kT>
+template <uint32_t kFmt, int kT, bool kPair>
 __global__ void __launch_bounds__(kDgThreads, 2)
-    gemm_digits_kernel(const uint8_t *__restrict__ w, const int8_t *__restrict__ aq, const float *__restrict__ ad,
-                       const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows, uint32_t nb, uint32_t seq,
-                       uint32_t nb_slice) {
+    gemm_digits_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, const int8_t *__restrict__ aq,
+                       const float *__restrict__ ad, const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows,
+                       uint32_t nb, uint32_t seq, uint32_t nb_slice) {
     typedef DgLds<kFmt, kT> L;
     typedef Rows<kFmt> R;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -112,7 +112,8 @@ __global__ void __launch_bounds__(kDgThreads, 2)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: what derives from it stays in SGPRs
     const int lrow = lane & 31, khalf = lane >> 5;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds));
-    const uint32_t row0 = blockIdx.x * kDgRows + wave * 32;
+    const uint32_t row_tile = gemm_matrix<kPair>(w, w2, out, rows, seq, kDgRows);
+    const uint32_t row0 = row_tile * kDgRows + wave * 32;
     // clamped loads, masked stores; a multiple of 32, so that Q6_K rows sit as far off a 4-byte boundary as their index says
     const uint32_t first = min(row0, (rows - 1) & ~31u), last_row = min(rows - 1 - first, 31u);
     const uint32_t tok0 = blockIdx.y * L::kToks, last_tok = seq - 1 - tok0;
@@ -120,7 +121,6 @@ __global__ void __launch_bounds__(kDgThreads, 2)
 
     // K slice of this workgroup (blockIdx.z): blocks slice0 .. slice0 + nbs, its sums go to the slice's own copy of the output
     const uint32_t slice0 = blockIdx.z * nb_slice, nbs = min(nb - slice0, nb_slice);
-    out += static_cast<size_t>(blockIdx.z) * seq * rows;
     const uint8_t *w_base = w + static_cast<size_t>(first) * row_bytes;
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(aq) + (static_cast<size_t>(tok0) * nb + slice0) * 256;
     const uint8_t *dig_base = adig + (static_cast<size_t>(tok0) * nb + slice0) * 16;
@@ -347,6 +347,7 @@ __global__ void __launch_bounds__(kDgThreads, 2)
 
 struct DgPlan {
     uint32_t tiles_per_wg, groups, row_tiles, slices;
+    uint64_t cost;  // rounds * blocks of a slice * half tiles
 };
 // Token tiles of 32 are dealt into groups of two to four per workgroup, one workgroup fits a compute unit.  A block costs
 // a workgroup about a tile and a half beside its tiles (making the operands): the group size with the least of
@@ -364,9 +365,9 @@ inline DgPlan digits_plan(uint32_t rows, uint32_t nb, uint32_t seq) {
         p.row_tiles = (rows + kDgRows - 1) / kDgRows;
         const uint64_t wgs = static_cast<uint64_t>(p.row_tiles) * p.groups;
         p.slices = wgs > 128 ? 1 : static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(256 / wgs, nb / 4)));
-        const uint64_t cost = (wgs * p.slices + 255) / 256 * ((nb + p.slices - 1) / p.slices) * (2 * per + 3);
-        if (cost < best_cost) {
-            best_cost = cost;
+        p.cost = (wgs * p.slices + 255) / 256 * ((nb + p.slices - 1) / p.slices) * (2 * per + 3);
+        if (p.cost < best_cost) {
+            best_cost = p.cost;
             best = p;
         }
     }
@@ -381,30 +382,30 @@ inline bool digits_fill_the_chip(uint32_t rows, uint32_t nb, uint32_t seq) {
     return 10 * wgs >= 7 * ((wgs + 255) / 256 * 256);
 }
 
-template <uint32_t kFmt, int kT>
-void launch_digits(const DgPlan &p, const uint8_t *w, const ActView &act, float *out, float *slice_out, uint32_t rows,
-                          uint32_t nb, uint32_t seq, hipStream_t stream) {
+template <uint32_t kFmt, int kT, bool kPair>
+void launch_digits(const DgPlan &p, const uint8_t *w, const uint8_t *w2, const ActView &act, float *out, float *slice_out,
+                   uint32_t rows, uint32_t nb, uint32_t seq, uint32_t *left, hipStream_t stream) {
     static bool configured = false;  // above the default 64 KB of dynamic LDS
     constexpr size_t lds = DgLds<kFmt, kT>::kBytes;
-    if (!allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<kFmt, kT>), lds, &configured, "gemm_digits_kernel"))
+    if (!allow_dynamic_lds(reinterpret_cast<const void *>(gemm_digits_kernel<kFmt, kT, kPair>), lds, &configured, "gemm_digits_kernel"))
         return;
     const uint32_t slices = slice_out ? p.slices : 1;
     const uint32_t nb_slice = (nb + slices - 1) / slices, nz = (nb + nb_slice - 1) / nb_slice;
-    hipLaunchKernelGGL((gemm_digits_kernel<kFmt, kT>), dim3(p.row_tiles, p.groups, nz), dim3(kDgThreads), lds, stream, w, act.qs,
-                       act.d, act.digits, nz > 1 ? slice_out : out, rows, nb, seq, nb_slice);
-    if (nz > 1) launch_sum_slices(slice_out, out, static_cast<size_t>(seq) * rows, nz, stream);
+    hipLaunchKernelGGL((gemm_digits_kernel<kFmt, kT, kPair>), dim3(p.row_tiles, p.groups, nz), dim3(kDgThreads), lds, stream, w, w2,
+                       act.qs, act.d, act.digits, nz > 1 ? slice_out : out, rows, nb, seq, nb_slice);
+    finish_slices(slice_out, out, (kPair ? 2 : 1) * static_cast<size_t>(seq) * rows, nz, left, stream);
 }
 
-template <uint32_t kFmt>
+template <uint32_t kFmt, bool kPair = false>
 void launch_digits_plan(const uint8_t *w, const ActView &act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                        uint32_t seq, hipStream_t stream) {
-    const DgPlan p = digits_plan(rows, nb, seq);
+                        uint32_t seq, hipStream_t stream, const uint8_t *w2 = nullptr, uint32_t *left = nullptr) {
+    const DgPlan p = digits_plan(kPair ? 2 * rows : rows, nb, seq);
     if (p.tiles_per_wg == 4)
-        launch_digits<kFmt, 4>(p, w, act, out, slice_out, rows, nb, seq, stream);
+        launch_digits<kFmt, 4, kPair>(p, w, w2, act, out, slice_out, rows, nb, seq, left, stream);
     else if (p.tiles_per_wg == 3)
-        launch_digits<kFmt, 3>(p, w, act, out, slice_out, rows, nb, seq, stream);
+        launch_digits<kFmt, 3, kPair>(p, w, w2, act, out, slice_out, rows, nb, seq, left, stream);
     else
-        launch_digits<kFmt, 2>(p, w, act, out, slice_out, rows, nb, seq, stream);
+        launch_digits<kFmt, 2, kPair>(p, w, w2, act, out, slice_out, rows, nb, seq, left, stream);
 }
 
 }  // namespace

@@ -162,6 +162,12 @@ bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols
     return p.tiles_per_wg >= min_tiles && digits_fill_the_chip(r, nb, q);
 }
 
+bool gemm_digits_pair_pays(size_t rows, size_t nb, size_t seq) {
+    const uint32_t r = static_cast<uint32_t>(rows), b = static_cast<uint32_t>(nb), q = static_cast<uint32_t>(seq);
+    const DgPlan one = digits_plan(r, b, q);
+    return one.slices > 1 || digits_plan(2 * r, b, q).cost < 2 * one.cost;
+}
+
 size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq) {
     if (rows == 0 || nb == 0 || seq == 0) return 0;
     const DgPlan p = digits_plan(rows, nb, seq);
@@ -169,9 +175,11 @@ size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq) {
 }
 
 void launch_gemm_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                        uint32_t seq, hipStream_t stream) {
+                        uint32_t seq, hipStream_t stream, const uint8_t *w2, uint32_t *left) {
     if (rows == 0 || seq == 0 || nb == 0) return;
-    if (quant == kQ4K)
+    if (quant == kQ4K && w2 != nullptr)
+        launch_digits_plan<kQ4K, true>(w, act, out, slice_out, rows, nb, seq, stream, w2, left);
+    else if (quant == kQ4K)
         launch_digits_plan<kQ4K>(w, act, out, slice_out, rows, nb, seq, stream);
     else if (quant == kQ5K)
         launch_digits_plan<kQ5K>(w, act, out, slice_out, rows, nb, seq, stream);

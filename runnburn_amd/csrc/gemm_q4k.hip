@@ -71,17 +71,19 @@ constexpr int kPpAPerWave = (kPpAInstr + kPpWaves - 1) / kPpWaves;  // 3
 constexpr uint32_t kMagicBits = 0x4B400000u;      // 1.5 * 2^23: int bits of 12582912.0f
 constexpr float kMagic = 12582912.0f;
 
+template <bool kPair>
 __global__ void __launch_bounds__(kPpThreads, 1)
-    gemm_q4k_mfma_kernel(const uint8_t *__restrict__ w, const int8_t *__restrict__ aq, const float *__restrict__ ad,
-                             const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows, uint32_t nb,
-                             uint32_t seq, uint32_t nb_slice) {
+    gemm_q4k_mfma_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, const int8_t *__restrict__ aq,
+                         const float *__restrict__ ad, const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows,
+                         uint32_t nb, uint32_t seq, uint32_t nb_slice) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: what derives from it stays in SGPRs
     const int lrow = lane & 31, khalf = lane >> 5;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds));
-    const uint32_t wg_row0 = blockIdx.x * kPpRowsPerWg;
+    const uint32_t row_tile = gemm_matrix<kPair>(w, w2, out, rows, seq, kPpRowsPerWg);
+    const uint32_t wg_row0 = row_tile * kPpRowsPerWg;
     const uint32_t row0 = wg_row0 + wave * 32;
     const uint32_t tok0 = blockIdx.y * kPpToks;
     const uint32_t row_bytes = nb * static_cast<uint32_t>(kQ4KBytes);
@@ -91,7 +93,6 @@ __global__ void __launch_bounds__(kPpThreads, 1)
     // K slice of this workgroup (blockIdx.z): nbs blocks from slice0 on, counted from 0 below (the bases move instead);
     // its sums go to the slice's own copy of the output
     const uint32_t slice0 = blockIdx.z * nb_slice, nbs = min(nb - slice0, nb_slice);
-    out += static_cast<size_t>(blockIdx.z) * seq * rows;
     const uint8_t *w_base = w + static_cast<size_t>(wg_row0) * row_bytes + slice0 * 144u;
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(aq) + (static_cast<size_t>(tok0) * nb + slice0) * 256;
     const uint8_t *dig_base = adig + (static_cast<size_t>(tok0) * nb + slice0) * 16;
@@ -308,18 +309,28 @@ size_t gemm_q4k_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq) {
     return slices > 1 ? static_cast<size_t>(slices) * seq * rows : 0;
 }
 
-void launch_gemm_q4k_mfma(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                          uint32_t seq, hipStream_t stream) {
-    if (rows == 0 || seq == 0 || nb == 0) return;
+template <bool kPair>
+static void launch_pp(const uint8_t *w, const uint8_t *w2, const ActView &act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
+                      uint32_t seq, uint32_t *left, hipStream_t stream) {
     static bool configured = false;  // 111 KB exceed the default 64 KB dynamic LDS limit
-    if (!allow_dynamic_lds(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel), kPpLdsBytes, &configured, "gemm_q4k_mfma_kernel"))
+    if (!allow_dynamic_lds(reinterpret_cast<const void *>(gemm_q4k_mfma_kernel<kPair>), kPpLdsBytes, &configured, "gemm_q4k_mfma_kernel"))
         return;
-    const uint32_t slices = slice_out ? pp_slices(rows, nb, seq) : 1;
+    constexpr uint32_t kMats = kPair ? 2 : 1;
+    const uint32_t slices = slice_out ? pp_slices(kMats * rows, nb, seq) : 1;
     const uint32_t nb_slice = (nb + slices - 1) / slices, nz = (nb + nb_slice - 1) / nb_slice;
-    const dim3 grid((rows + kPpRowsPerWg - 1) / kPpRowsPerWg, (seq + kPpToks - 1) / kPpToks, nz);
-    hipLaunchKernelGGL(gemm_q4k_mfma_kernel, grid, dim3(kPpThreads), kPpLdsBytes, stream, w, act.qs, act.d,
+    const dim3 grid(kMats * ((rows + kPpRowsPerWg - 1) / kPpRowsPerWg), (seq + kPpToks - 1) / kPpToks, nz);
+    hipLaunchKernelGGL(gemm_q4k_mfma_kernel<kPair>, grid, dim3(kPpThreads), kPpLdsBytes, stream, w, w2, act.qs, act.d,
                        act.digits, nz > 1 ? slice_out : out, rows, nb, seq, nb_slice);
-    if (nz > 1) launch_sum_slices(slice_out, out, static_cast<size_t>(seq) * rows, nz, stream);
+    finish_slices(slice_out, out, kMats * static_cast<size_t>(seq) * rows, nz, left, stream);
+}
+
+void launch_gemm_q4k_mfma(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
+                          uint32_t seq, hipStream_t stream, const uint8_t *w2, uint32_t *left) {
+    if (rows == 0 || seq == 0 || nb == 0) return;
+    if (w2 != nullptr)
+        launch_pp<true>(w, w2, act, out, slice_out, rows, nb, seq, left, stream);
+    else
+        launch_pp<false>(w, nullptr, act, out, slice_out, rows, nb, seq, nullptr, stream);
 }
 
 }  // namespace rnb

@@ -128,8 +128,11 @@ void launch_gemm_q5k_mfma(const uint8_t *w, ActView act, float *out, float *slic
                           uint32_t seq, hipStream_t stream);
 // Q4_K through the same kernel (scales on the vector units): for shapes that give gemm_q4k.hip's 256 x 64 tiles too few
 // workgroups to fill the chip
+// This kernel and the two below can take two matrices of the same shape in one launch (w2; rows a multiple of 256): out =
+// [matrix][seq][rows], workspaces for 2 * rows.  With `left` the slices' sums stay in slice_out ([slice][matrix][seq][rows]) and
+// *left says how many there are (1: everything is in out).
 void launch_gemm_q4k_small(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                           uint32_t seq, hipStream_t stream);
+                           uint32_t seq, hipStream_t stream, const uint8_t *w2 = nullptr, uint32_t *left = nullptr);
 // Q2_K / Q3_K (needs act.bsums, which the Q8_K quantiser always writes)
 void launch_gemm_q23k_mfma(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows,
                            uint32_t nb, uint32_t seq, hipStream_t stream);
@@ -140,7 +143,7 @@ void launch_gemm_q8_mfma(const uint8_t *w, uint32_t quant, ActView act, float *o
 // Up to 128 tiles the K range is cut into slices (workspace: gemm_q4k_slice_floats floats, as for the kernels above)
 size_t gemm_q4k_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq);
 void launch_gemm_q4k_mfma(const uint8_t *w, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                          uint32_t seq, hipStream_t stream);
+                          uint32_t seq, hipStream_t stream, const uint8_t *w2 = nullptr, uint32_t *left = nullptr);
 // the importance quants in the same kernel as launch_gemm_digits (workspace: gemm_digits_slice_floats)
 bool gemm_iq_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq);
 void launch_gemm_iq_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows,
@@ -150,8 +153,11 @@ void launch_gemm_iq_digits(const uint8_t *w, uint32_t quant, ActView act, float 
 // Q4_K / Q5_K); workspace for K slices as for the kernels above.  _pays: weights aligned for it and enough work.
 bool gemm_digits_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq);
 size_t gemm_digits_slice_floats(uint32_t rows, uint32_t nb, uint32_t seq);
+// whether two matrices in one launch of it take fewer rounds of workgroups than a launch each
+bool gemm_digits_pair_pays(size_t rows, size_t nb, size_t seq);
+// (w2 and left: Q4_K only)
 void launch_gemm_digits(const uint8_t *w, uint32_t quant, ActView act, float *out, float *slice_out, uint32_t rows, uint32_t nb,
-                        uint32_t seq, hipStream_t stream);
+                        uint32_t seq, hipStream_t stream, const uint8_t *w2 = nullptr, uint32_t *left = nullptr);
 
 // Q4_K, Q5_K and Q6_K against at most 32 tokens, the K slices inside a workgroup: no workspace (act needs digits for Q4_K /
 // Q5_K); the gate_up form is mid = act(Wg a) * (Wu a) on Q4_K
@@ -174,6 +180,8 @@ void launch_gemm_b32(const uint8_t *w, uint32_t quant, ActView act, float *out, 
 constexpr size_t kSliceScratchBytes = size_t(128) << 20;
 // out[i] = parts[0][i] + parts[1][i] + ... in that order (n floats per slice)
 void launch_sum_slices(const float *parts, float *out, size_t n, uint32_t slices, hipStream_t stream);
+// the same where there is more than one slice, or (left != null) only their number
+void finish_slices(const float *parts, float *out, size_t n, uint32_t slices, uint32_t *left, hipStream_t stream);
 
 // ---- gathered sparse-MoE ------------------------------------------------------------------
 // Slots grouped by expert (device arrays).  Group i covers sorted positions [start[i], start[i+1]);
@@ -192,9 +200,10 @@ struct MoeGroups {
         return n;
     }
 };
-// Q8_K of act(gate[i]) * up[i] (SiLU, or the tanh form of GELU): the gated FFN's intermediate quantised as it is made
-void launch_quantize_q8k_gated(const float *gate, const float *up, size_t n_blocks, bool gelu, int8_t *qs, float *d,
-                               int16_t *bsums, uint8_t *digits, hipStream_t stream);
+// Q8_K of act(gate[i]) * up[i] (SiLU, or the tanh form of GELU): the gated FFN's intermediate quantised as it is made; both are
+// the sums of `slices` parts `stride` floats apart, added in that order
+void launch_quantize_q8k_gated(const float *gate, const float *up, size_t n_blocks, uint32_t slices, size_t stride, bool gelu,
+                               int8_t *qs, float *d, int16_t *bsums, uint8_t *digits, hipStream_t stream);
 // Decode-sized routing tables travel as a kernel argument instead of a host-to-device copy: the
 // activation quantiser's launch also writes them to their device buffer.
 constexpr uint32_t kMoeInlineWords = 240;  // 960 bytes of kernel argument
