@@ -721,21 +721,33 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     }
     grp_start.push_back(static_cast<uint32_t>(n_slots));
     const size_t n_groups = grp_expert.size();
-    // one table image: route[n] | tok_offsets[T+1] | tok_slots[n] | sorted_slot[n] | sorted_token[n] | grp_expert[G] |
-    // grp_start[G+1] | slot_expert[n]
-    const size_t table_words = 5 * n_slots + (token_count + 1) + n_groups + (n_groups + 1);
+    uint32_t max_group = 0;
+    for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
     // Batches with at least 1.8 slots per routed expert on average: the expert GEMMs run on the matrix cores (a
     // 32-token tile costs the same whatever its number of live tokens, the integer-dot kernels cost per token; measured
     // on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot kernels, 79.0 / 85.7 / 88.2
     // on the matrix cores; the ratio is 1.6 / 1.8 / 1.9 there) and need the quantiser's digits
     // (its gate/up rows arrive as 16-byte LDS-direct loads: other alignments take the vector kernels)
     // (and the Q6_K down rows as dword-aligned pieces: an even base address and whole 128-row tiles)
-    const bool aligned16 = ((reinterpret_cast<uintptr_t>(gate_dev) | reinterpret_cast<uintptr_t>(up_dev) |
-                             reinterpret_cast<uintptr_t>(down_dev) | reinterpret_cast<uintptr_t>(shared.gate) |
-                             reinterpret_cast<uintptr_t>(shared.up) | reinterpret_cast<uintptr_t>(shared.down)) & 15u) == 0;
+    const uintptr_t addresses = reinterpret_cast<uintptr_t>(gate_dev) | reinterpret_cast<uintptr_t>(up_dev) |
+                                reinterpret_cast<uintptr_t>(down_dev) | reinterpret_cast<uintptr_t>(shared.gate) |
+                                reinterpret_cast<uintptr_t>(shared.up) | reinterpret_cast<uintptr_t>(shared.down);
+    const bool aligned16 = addresses % 16 == 0, aligned4 = addresses % 4 == 0;
     const bool mfma = token_count >= kMoeMfmaMinTokens && 10 * n_slots >= 18 * n_groups && aligned16 && n_embd % 128 == 0 &&
                       moe_mfma_supported(static_cast<uint32_t>(sh.nb_in), static_cast<uint32_t>(sh.nb_mid), down_quant);
+    // one table image: route[n] | tok_offsets[T+1] | tok_slots[n] | sorted_slot[n] | sorted_token[n] | grp_expert[G] |
+    // grp_start[G+1] | slot_expert[n] | units
+    size_t table_words = 5 * n_slots + (token_count + 1) + n_groups + (n_groups + 1);
     const bool inline_tables = !mfma && table_words <= kMoeInlineWords;  // decode-sized: rides in a kernel argument
+    const bool few = !inline_tables && aligned4 && moe_few_pays(token_count, n_slots, n_groups, max_group, sh.nb_mid, down_quant) &&
+                     moe_few_supported(sh.nb_in, sh.nb_mid, token_count, n_slots, n_ff, n_embd, down_quant);
+    const uint32_t unit_tokens = moe_few_tile(n_slots, n_groups);
+    std::vector<uint32_t> units;
+    if (few)
+        for (size_t g = 0; g < n_groups; g++)
+            for (uint32_t p = grp_start[g]; p < grp_start[g + 1]; p += unit_tokens)
+                units.insert(units.end(), {grp_expert[g], p, std::min(unit_tokens, grp_start[g + 1] - p)});
+    table_words += units.size();
     MoeInlineTables inl;
     uint32_t *h = inl.words;
     TableSlot *ring_slot = nullptr;
@@ -773,13 +785,13 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     }
     if (n_groups) std::memcpy(h_gexp, grp_expert.data(), n_groups * 4);
     std::memcpy(h_gstart, grp_start.data(), (n_groups + 1) * 4);
+    if (!units.empty()) std::memcpy(h_sexp + n_slots, units.data(), units.size() * 4);
     uint32_t *d = s.moe_tables.as<uint32_t>();
     const float *d_route = reinterpret_cast<const float *>(d);
     const uint32_t *d_off = d + n_slots, *d_list = d_off + token_count + 1;
-    uint32_t max_group = 0;
-    for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
-    const MoeGroups groups{d_list + 3 * n_slots, d_list + 3 * n_slots + n_groups, d_list + n_slots, d_list + 2 * n_slots,
-                           static_cast<uint32_t>(n_groups), max_group, grp_start.data()};
+    const uint32_t *d_gstart = d_list + 3 * n_slots + n_groups, *d_units = d_gstart + n_groups + 1 + n_slots;
+    const MoeGroups groups{d_list + 3 * n_slots, d_gstart, d_list + n_slots, d_list + 2 * n_slots, static_cast<uint32_t>(n_groups),
+                           max_group, grp_start.data(), d_units, static_cast<uint32_t>(units.size() / 3), unit_tokens};
 
     ActView act;
     if (inline_tables) {
@@ -812,6 +824,24 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     }
     RESERVE_TRY(s.moe_mid, n_slots * n_ff * sizeof(float));
     RESERVE_TRY(s.moe_slot_out, n_slots * n_embd * sizeof(float));
+    if (few && act.digits != nullptr) {
+        const size_t blocks = n_slots * sh.nb_mid;
+        RESERVE_TRY(s.moe_mid_qs, n_slots * n_ff);
+        RESERVE_TRY(s.moe_mid_d, blocks * sizeof(float));
+        RESERVE_TRY(s.moe_mid_bsums, blocks * 16 * sizeof(int16_t));
+        RESERVE_TRY(s.moe_mid_digits, blocks * 16);
+        launch_moe_few_gate_up(gate_dev, up_dev, shared, act, groups, s.moe_mid.as<float>(), static_cast<uint32_t>(n_ff),
+                               static_cast<uint32_t>(sh.nb_in), s.stream);
+        launch_quantize_q8k(s.moe_mid.as<float>(), blocks, s.moe_mid_qs.as<int8_t>(), s.moe_mid_d.as<float>(),
+                            s.moe_mid_bsums.as<int16_t>(), s.moe_mid_digits.as<uint8_t>(), s.stream);
+        const ActView mid{s.moe_mid_qs.as<int8_t>(), s.moe_mid_d.as<float>(), s.moe_mid_bsums.as<int16_t>(), s.moe_mid_digits.as<uint8_t>()};
+        launch_moe_few_down(down_dev, shared, down_quant, mid, groups, d_route, s.moe_slot_out.as<float>(),
+                            static_cast<uint32_t>(n_embd), static_cast<uint32_t>(sh.nb_mid), s.stream);
+        launch_moe_reduce(s.moe_slot_out.as<float>(), d_off, d_list, out_dev, static_cast<uint32_t>(token_count),
+                          static_cast<uint32_t>(n_embd), s.stream);
+        if (int ls = check_launches(); ls != RNB_HIP_OK) return ls;
+        return RNB_HIP_OK;
+    }
     if (mfma && act.digits != nullptr) {
         // prefill: grouped GEMMs on the matrix cores; the down kernel quantises the intermediate as it stages it
         launch_moe_gate_up_mfma(gate_dev, up_dev, shared, act, groups, s.moe_mid.as<float>(), static_cast<uint32_t>(n_ff),

@@ -194,6 +194,9 @@ struct MoeGroups {
     uint32_t n_groups;
     uint32_t max_group = 32;       // slots of the largest group (host-side knowledge: sizes the matrix-core kernels' LDS)
     const uint32_t *host_start = nullptr;  // `start` in host memory, for the length of the call
+    // the groups' slots in tiles of unit_tokens (device array): {expert, first sorted position, slots} each
+    const uint32_t *units = nullptr;
+    uint32_t n_units = 0, unit_tokens = 0;
     uint32_t tiles_of(uint32_t slots) const {  // the groups' slots in tiles of `slots`
         uint32_t n = 0;
         for (uint32_t g = 0; g < n_groups; g++) n += (host_start[g + 1] - host_start[g] + slots - 1) / slots;
@@ -236,6 +239,15 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
                              MoeGroups groups, float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);
 void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, const float *mid, MoeGroups groups,
                           const float *slot_route, float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream);
+// the same two steps on the few-token GEMM's tiles (moe_few.hip): groups with units of moe_few_tile slots, weights at 4-byte
+// addresses, both activations quantised with digits
+uint32_t moe_few_tile(size_t n_slots, size_t n_groups);
+bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_mid, uint32_t down_quant);
+bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant);
+void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
+                            float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);
+void launch_moe_few_down(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act, const MoeGroups &g,
+                         const float *slot_route, float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream);
 // down + route weight + ordered per-token sum in one launch (rows of at most 16 super-blocks); slot_expert [n_slots]
 void launch_moe_down_token(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act, const uint32_t *tok_offsets,
                            const uint32_t *tok_slots, const uint32_t *slot_expert, const float *slot_route, float *out,

@@ -1,0 +1,186 @@
+// Routed experts of a batch on the few-token GEMM's tiles (gemm_few.h): every expert's slots in tiles of 16 or 32, a workgroup per
+// (tile, 64 rows), a wave per 16 rows.
+//   gate/up   mid[slot][n_ff] = silu(Wg[e] . a_tok) * (Wu[e] . a_tok), both Q4_K            fanout.rs:260-327, activation.rs:73-89
+//   down      slot_out[slot][n_embd] = route[slot] * (Wd[e] . Q8_K(mid[slot])), Q4_K, Q5_K or Q6_K
+// (crates/rnb-llm/src/engine/models/shared_expert_moe/moe_view/fanout.rs, crates/rnb-cpu/src/kernels/activation.rs)
+//
+// An expert's rows are read once per tile and little is computed with them, so what counts are waves in flight: a wave needs its stage
+// of LDS and about 90 registers and waits for nobody.  moe_mfma.hip's workgroups stage a whole tile of 32 slots first and leave most of
+// the chip idle where experts are few.  A wave walks its rows' blocks in order with the same roundings, so the bits are those of
+// moe_mfma.hip.  Two and four K slices a row tile, as in gemm_few.hip, were up to 10 % faster on the smallest grids (8 experts of 2048 x 4096
+// at 64 tokens 61 us against 68) and 5 % slower on large ones; 32 rows a wave 5 - 25 % slower.
+#include "gemm_few.h"
+
+namespace rnb {
+
+namespace {
+
+constexpr int kMfWaves = 4;
+
+template <uint32_t kFmt, int kMT, int kMats>
+__global__ void __launch_bounds__(kWave *kMfWaves)
+    moe_few_kernel(const uint8_t *__restrict__ w_all, const uint8_t *__restrict__ w2_all, const uint8_t *__restrict__ w_shared,
+                   const uint8_t *__restrict__ w2_shared, uint32_t n_routed, const int8_t *__restrict__ aq,
+                   const float *__restrict__ ad, const uint8_t *__restrict__ adig, const uint32_t *__restrict__ units,
+                   const uint32_t *__restrict__ act_rows, const uint32_t *__restrict__ out_rows,
+                   const float *__restrict__ out_scale, float *__restrict__ out, uint32_t rows, uint32_t nb, uint32_t unit0) {
+    typedef FewLds<kFmt, kMT, 1, kMats> L;
+    typedef FewRows<kFmt> R;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, kq = lane >> 4;
+    const uint32_t *unit = units + 3 * (unit0 + blockIdx.y);
+    const uint32_t expert = unit[0], start = unit[1], live = unit[2];
+    const uint32_t row0 = (blockIdx.x * kMfWaves + wave) * 16;
+    const uint32_t first = min(row0, (rows - 1) & ~15u), last_row = min(rows - 1 - first, 15u);  // clamped loads, masked stores
+    const uint32_t row_bytes = nb * static_cast<uint32_t>(R::kBytes), last_tok = live - 1;
+    constexpr int kStage = L::kStage + 256;  // and a scale per lane
+    uint8_t *stage = lds + wave * kStage;
+    const uint32_t stage0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds)) + wave * kStage;
+    const size_t per_expert = static_cast<size_t>(rows) * row_bytes, at = static_cast<size_t>(first) * row_bytes;
+    const uint8_t *w_base[2] = {expert_base(w_all, w_shared, n_routed, expert, per_expert) + at,
+                                expert_base(w2_all, w2_shared, n_routed, expert, per_expert) + at};
+
+    // the list before the first fill: loads return in order, and the compiler counts its own only
+    const uint32_t *list = act_rows + start;
+    const uint32_t rr = __umul24(lane, R::kInv) >> 16, j = lane - rr * R::kPieces;
+    uint32_t row_off[L::kFills], act_off[4 * kMT], dig_off[kMT];
+#pragma unroll
+    for (int g = 0; g < 4 * kMT; g++)
+        act_off[g] = list[min(static_cast<uint32_t>(4 * g + kq), last_tok)] * (nb * 256u) + 16 * (l16 ^ (4 * (g & 3) + kq));
+#pragma unroll
+    for (int t = 0; t < kMT; t++)  // a token's sixteen bytes are four lanes' dwords
+        dig_off[t] = list[min(static_cast<uint32_t>(16 * t + (lane >> 2)), last_tok)] * (nb * 16u) + 4 * (lane & 3);
+    const uint32_t dx_off = list[min(static_cast<uint32_t>(lane), last_tok)] * (nb * 4u);
+#pragma unroll
+    for (int k = 0; k < L::kFills; k++) row_off[k] = min(k * R::kPer + rr, last_row) * row_bytes;
+
+    auto run = [&](auto tiles_tag) {  // with the token tiles that have live slots
+        constexpr int kLive = decltype(tiles_tag)::value;
+        auto issue = [&](uint32_t b) {
+#pragma unroll
+            for (int m = 0; m < kMats; m++) {
+                const uint8_t *src = w_base[m] + R::block_off(b);
+#pragma unroll
+                for (int k = 0; k < L::kFills; k++) lds_fill16(src, R::piece(row_off[k], j, b), stage0 + m * L::kStrip + k * 1024);
+            }
+            const uint8_t *act = reinterpret_cast<const uint8_t *>(aq) + b * 256u;
+#pragma unroll
+            for (int g = 0; g < 4 * kLive; g++) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);
+            if constexpr (R::kMins)
+#pragma unroll
+                for (int t = 0; t < kLive; t++) lds_fill4(adig + b * 16u, dig_off[t], stage0 + L::kDig + t * 256);
+            lds_fill4(reinterpret_cast<const uint8_t *>(ad) + b * 4u, dx_off, stage0 + L::kStage);
+        };
+        float acc[kMats][1][kLive][4];
+#pragma unroll
+        for (int m = 0; m < kMats; m++)
+#pragma unroll
+            for (int t = 0; t < kLive; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[m][0][t][r] = 0.0f;
+        issue(0);
+        for (uint32_t b = 0; b < nb; b++) {
+            wait_fills();
+            FewBlock<kFmt, kLive, 1, kMats> blk;
+            blk.read(stage, L::kAct, L::kDig, reinterpret_cast<const float *>(stage + L::kStage), l16, kq, last_row, nb, b);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read
+            if (b + 1 < nb) issue(b + 1);
+            blk.template multiply<true>(acc, kq);
+        }
+        const uint32_t row = row0 + l16;
+#pragma unroll
+        for (int t = 0; t < kLive; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t tok = 16 * t + 4 * kq + r;
+                if (tok < live && row < rows) {
+                    const uint32_t slot = out_rows[start + tok];
+                    // fanout.rs:306-308: the expert's output times the slot's route weight
+                    out[static_cast<size_t>(slot) * rows + row] =
+                        kMats == 2 ? act_mul<false>(acc[0][0][t][r], acc[kMats - 1][0][t][r]) : acc[0][0][t][r] * out_scale[slot];
+                }
+            }
+    };
+    if constexpr (kMT > 1) {
+        if (live <= 16) {  // workgroup-uniform
+            run(std::integral_constant<int, 1>{});
+            return;
+        }
+    }
+    run(std::integral_constant<int, kMT>{});
+}
+
+template <uint32_t kFmt, int kMT, int kMats>
+void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, const uint8_t *ws2, uint32_t n_routed, const ActView &act,
+                    const MoeGroups &g, const uint32_t *act_rows, const float *scale, float *out, uint32_t rows, uint32_t nb,
+                    hipStream_t stream) {
+    static bool configured = false;
+    constexpr size_t lds = kMfWaves * (FewLds<kFmt, kMT, 1, kMats>::kStage + 256);
+    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+    if (!allow_dynamic_lds(reinterpret_cast<const void *>(moe_few_kernel<kFmt, kMT, kMats>), lds, &configured, "moe_few_kernel")) return;
+    for (uint32_t u = 0; u < g.n_units; u += 65535)  // grid rows that a device is sure to take
+        hipLaunchKernelGGL((moe_few_kernel<kFmt, kMT, kMats>), dim3((rows + 16 * kMfWaves - 1) / (16 * kMfWaves), std::min(g.n_units - u, 65535u)),
+                           dim3(kWave * kMfWaves), lds, stream, w, w2, ws, ws2, n_routed, act.qs, act.d, act.digits, g.units, act_rows,
+                           g.sorted_slot, scale, out, rows, nb, u);
+}
+
+}  // namespace
+
+uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 16 * n_groups ? 16 : 32; }
+
+// Against the tiles of moe_mfma.hip and the integer-dot kernels of moe.hip, us a call, those : this.  From sixteen tokens on (a
+// smaller batch's rows are a lone token's bit for bit): 8 experts x top-2 of 1792 x 2304 at 52 tokens 64 : 40, 16 x top-2 of 1536 x
+// 1536 at 38 66 : 38, 128 x top-8 of 1536 x 2560 at 238 320 : 286, of 1024 x 1280 at 27 87 : 63.  Many experts with short intermediates and
+// several slots each stay on moe_mfma.hip, whose workgroups walk more rows per list and quantise as they stage (128 x top-8 of 768 x
+// 2048 at 512 tokens 189 : 204, at 64 104.7 : 106; 64 x top-8 of 512 x 2816 at 446 155 : 157); one slot or two per expert on
+// moe.hip, whose dots cost little then (16 x top-2 of 1536 x 3072 at 18 tokens, Q5_K down projection, 43.0 : 45.9, 32 x top-4 of 768 x
+// 1792 at 21 34.3 : 37.8).
+bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_mid, uint32_t down_quant) {
+    if (token_count < 16) return false;
+    if (nb_mid <= 3 && (n_slots >= 2048 || (n_groups >= 80 && n_slots >= 4 * n_groups))) return false;
+    if (nb_mid <= 4 && max_group <= 8 && 10 * n_slots < 16 * n_groups) return false;
+    return down_quant == kQ6K || n_slots >= 100 || n_slots >= 3 * n_groups;
+}
+
+bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant) {
+    // 32-bit offsets into the activations; every other Q6_K block's last piece ends two bytes behind it (gemm_few.h)
+    return nb_in <= kFewMaxBlocks && nb_mid <= kFewMaxBlocks && token_count * n_embd < (size_t(1) << 32) && n_slots * n_ff < (size_t(1) << 32) &&
+           (down_quant != kQ6K || n_embd * nb_mid % 2 == 0);
+}
+
+void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
+                            float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream) {
+    if (g.n_units == 0 || n_ff == 0) return;
+    if (g.unit_tokens == 16)
+        launch_moe_few<kQ4K, 1, 2>(gate_all, up_all, shared.gate, shared.up, shared.n_routed, act, g, g.sorted_token, nullptr, mid, n_ff,
+                                   nb_in, stream);
+    else
+        launch_moe_few<kQ4K, 2, 2>(gate_all, up_all, shared.gate, shared.up, shared.n_routed, act, g, g.sorted_token, nullptr, mid, n_ff,
+                                   nb_in, stream);
+}
+
+template <uint32_t kFmt>
+static void moe_few_down(const uint8_t *down_all, const MoeShared &shared, const ActView &act, const MoeGroups &g, const float *slot_route,
+                         float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream) {
+    if (g.unit_tokens == 16)
+        launch_moe_few<kFmt, 1, 1>(down_all, down_all, shared.down, shared.down, shared.n_routed, act, g, g.sorted_slot, slot_route, slot_out,
+                                   n_embd, nb_mid, stream);
+    else
+        launch_moe_few<kFmt, 2, 1>(down_all, down_all, shared.down, shared.down, shared.n_routed, act, g, g.sorted_slot, slot_route, slot_out,
+                                   n_embd, nb_mid, stream);
+}
+
+void launch_moe_few_down(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act, const MoeGroups &g,
+                         const float *slot_route, float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream) {
+    if (g.n_units == 0 || n_embd == 0) return;
+    if (down_quant == kQ4K)
+        moe_few_down<kQ4K>(down_all, shared, mid_act, g, slot_route, slot_out, n_embd, nb_mid, stream);
+    else if (down_quant == kQ5K)
+        moe_few_down<kQ5K>(down_all, shared, mid_act, g, slot_route, slot_out, n_embd, nb_mid, stream);
+    else
+        moe_few_down<kQ6K>(down_all, shared, mid_act, g, slot_route, slot_out, n_embd, nb_mid, stream);
+}
+
+}  // namespace rnb

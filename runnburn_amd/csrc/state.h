@@ -64,7 +64,7 @@ struct State {
     DeviceBuf out_f32;    // staged outputs
     DeviceBuf gemm_slices;  // per-slice outputs of a GEMM whose K range was cut to fill the chip
     void *noalloc_slices = nullptr;  // the same for rnb_hip_gemv_dev_noalloc: kSliceScratchBytes, allocated with the state
-    DeviceBuf moe_mid, moe_mid_qs, moe_mid_d, moe_mid_bsums, moe_slot_out, moe_tables;
+    DeviceBuf moe_mid, moe_mid_qs, moe_mid_d, moe_mid_bsums, moe_mid_digits, moe_slot_out, moe_tables;
     DeviceBuf gather_ids, gather_rows;  // embedding gather: token ids; the rows of a matrix that is not resident
     PinnedBuf bounce_in, bounce_out;
     TableSlot table_ring[kTableRing];  // MoE routing tables too large for a kernel argument

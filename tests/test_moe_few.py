@@ -1,0 +1,53 @@
+"""Routed experts on the few-token GEMM's tiles (moe_few.hip): groups of every size around the 16- and 32-slot tiles, row tiles with
+remainders, few and many workgroups (16 and 32 rows a wave, one to four K slices), a shared expert.  Against the oracle; outputs
+outside the plain per-row tolerance must be whole re-quantisation flips (oracle/flips.py)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+Q4_K, Q5_K, Q6_K = 12, 13, 14
+
+
+def _lists(groups, tokens, rng):
+    """Slot lists with the given number of slots per expert: each expert's tokens distinct, list in a shuffled order."""
+    e, t = [], []
+    for expert, n in enumerate(groups):
+        e += [expert] * n
+        t += list(rng.permutation(tokens)[:n])
+    order = rng.permutation(len(e))
+    return np.array(e, np.uint32)[order], (rng.random(len(e)) + 0.1).astype(np.float32), np.array(t, np.uint32)[order]
+
+
+@pytest.mark.parametrize("down_quant", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("tokens,groups,n_ff,n_embd,shared", [
+    (18, [9, 1, 0, 8, 7, 9, 9], 256, 256, False),           # one block, tiles of 16
+    (17, [1, 2, 15, 16, 17, 3], 768, 512, False),           # tiles of 16, one group in two of them
+    (40, [16, 17, 31, 32, 33, 1, 40], 512, 1024, False),    # tiles of 32: one and two token tiles, and a second unit of one slot
+    (70, [70, 65, 64, 2, 33], 1280, 768, True),             # groups of several units, K slices of unequal length
+    (16, [5, 4, 3] * 10, 1024, 1280, True),                 # small groups, five blocks in
+])
+def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant):
+    from oracle import flips
+
+    rng = np.random.default_rng(tokens + n_ff)
+    n_expert = len(groups)
+    print(f"moe few tokens={tokens} experts={n_expert} n_ff={n_ff} n_embd={n_embd} down={down_quant} shared={shared}", flush=True)
+    e, r, t = _lists(groups, tokens, rng)
+    gate, up = (oracle.make_weights(Q4_K, (n_expert + shared) * n_ff, n_embd, 70 + k) for k in range(2))
+    down = oracle.make_weights(down_quant, (n_expert + shared) * n_embd, n_ff, 72)
+    x = oracle.fill_normal(tokens * n_embd, 73, 1.0)
+    if shared:  # one more slot of every token, its matrices behind the routed ones for the oracle
+        e = np.concatenate([e, np.full(tokens, n_expert, np.uint32)])
+        r = np.concatenate([r, rng.random(tokens).astype(np.float32)])
+        t = np.concatenate([t, np.arange(tokens, dtype=np.uint32)])
+    g_len, d_len = gate.size // (n_expert + shared) * n_expert, down.size // (n_expert + shared) * n_expert
+    routed = [gate[:g_len].copy(), up[:g_len].copy(), down[:d_len].copy()]
+    own = [gate[g_len:].copy(), up[g_len:].copy(), down[d_len:].copy()] if shared else None
+    got = rnb.qwen35_sparse_experts_selected_base_by_token(*routed, e, r, t, tokens, down_quant, n_ff, n_embd, x, shared=own)
+    ref = oracle.moe_sparse_experts_by_token(gate, up, down, n_expert + shared, e, r, t, tokens, down_quant, n_ff, n_embd, x)
+    v = flips.moe_verdict(np.asarray(got).reshape(np.shape(ref)), ref, gate, up, down, n_expert + shared, e, r, t, tokens, down_quant,
+                          n_ff, n_embd, x)
+    assert v["ok"] or v["flip_aware_ok"], {key: v[key] for key in v if key != "flips"}
+    for a in routed + (own or []):
+        rnb.release(a)
