@@ -28,15 +28,15 @@ template <uint32_t kFmt, int kMT, int kN, int kWaves, int kMats, bool kGelu>
 __global__ void __launch_bounds__(kWave *kWaves)
     gemm_few_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, const int8_t *__restrict__ aq,
                     const float *__restrict__ ad, const uint8_t *__restrict__ adig, float *__restrict__ out, uint32_t rows,
-                    uint32_t nb, uint32_t seq, uint32_t slices) {
+                    uint32_t nb, uint32_t seq, uint32_t log_slices) {
     typedef FewLds<kFmt, kMT, kN, kMats> L;
     typedef FewRows<kFmt> R;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, kq = lane >> 4;
-    const uint32_t group = __builtin_amdgcn_readfirstlane(wave / slices), sl = wave - group * slices;  // divided on the vector units
-    const uint32_t row0 = __builtin_amdgcn_readfirstlane((blockIdx.x * (kWaves / slices) + group) * (16 * kN));
+    const uint32_t slices = 1u << log_slices, group = wave >> log_slices, sl = wave & (slices - 1);
+    const uint32_t row0 = (blockIdx.x * (kWaves >> log_slices) + group) * (16 * kN);
     const uint32_t first = min(row0, (rows - 1) & ~15u), last_row = min(rows - 1 - first, 16u * kN - 1);  // clamped loads, masked stores
     const uint32_t row_bytes = nb * static_cast<uint32_t>(R::kBytes), last_tok = seq - 1;
     // K slice of the wave: blocks sl, sl + slices, ...: the waves of a workgroup read neighbouring blocks at the same time
@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(kWave *kWaves)
         }
         const uint8_t *act = reinterpret_cast<const uint8_t *>(aq) + b * 256u;
 #pragma unroll
-        for (int g = 0; g < 4 * kMT; g++) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);
+        for (int g = 0; g < 4 * kMT; g++)
+            if (4u * g < seq) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);  // places of no token keep what they hold
         if constexpr (R::kMins)
 #pragma unroll
             for (int t = 0; t < kMT; t++) lds_fill4(adig + b * 16u, dig_off[t], stage0 + L::kDig + t * 256);
@@ -123,7 +124,7 @@ __global__ void __launch_bounds__(kWave *kWaves)
 
 template <uint32_t kFmt, int kMT, int kN, int kWaves, int kMats, bool kGelu>
 void launch_few(const uint8_t *w, const uint8_t *w2, const ActView &act, float *out, uint32_t rows, uint32_t nb, uint32_t seq,
-                uint32_t slices, hipStream_t stream) {
+                uint32_t slices, hipStream_t stream) {  // slices: a power of two, at most kWaves
     static bool configured = false;
     constexpr size_t most = kWaves * FewLds<kFmt, kMT, kN, kMats>::kStage + kFewMaxBlocks * 16 * kMT * sizeof(float);
     static_assert(most <= 160 * 1024, "LDS of a compute unit");
@@ -133,7 +134,7 @@ void launch_few(const uint8_t *w, const uint8_t *w2, const ActView &act, float *
         return;
     const uint32_t per_wg = kWaves / slices * 16 * kN;
     hipLaunchKernelGGL((gemm_few_kernel<kFmt, kMT, kN, kWaves, kMats, kGelu>), dim3((rows + per_wg - 1) / per_wg), dim3(kWave * kWaves),
-                       lds, stream, w, w2, act.qs, act.d, act.digits, out, rows, nb, seq, slices);
+                       lds, stream, w, w2, act.qs, act.d, act.digits, out, rows, nb, seq, __builtin_ctz(slices));
 }
 
 struct FewPlan {

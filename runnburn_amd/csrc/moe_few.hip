@@ -67,7 +67,8 @@ __global__ void __launch_bounds__(kWave *kMfWaves)
             }
             const uint8_t *act = reinterpret_cast<const uint8_t *>(aq) + b * 256u;
 #pragma unroll
-            for (int g = 0; g < 4 * kLive; g++) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);
+            for (int g = 0; g < 4 * kLive; g++)
+                if (4u * g < live) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);  // places of no slot keep what they hold
             if constexpr (R::kMins)
 #pragma unroll
                 for (int t = 0; t < kLive; t++) lds_fill4(adig + b * 16u, dig_off[t], stage0 + L::kDig + t * 256);
