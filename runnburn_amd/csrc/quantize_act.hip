@@ -86,6 +86,17 @@ __global__ void __launch_bounds__(kWave *kWavesPerWg)
     q8_quantize_span(x + span * 256, lane, left < 8 ? static_cast<int>(left) : 8, qs + span * 256, d_out + span * 8);
 }
 
+// Floats between pinned host memory and device memory, read or written over the bus by the kernel: a copy command costs about
+// 8 us of set-up and signalling whatever its size, a launch 2.5.
+__global__ void __launch_bounds__(256) copy_words_kernel(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, uint32_t n) {
+    const uint32_t i = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (i + 4 <= n) {
+        *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+    } else {
+        for (uint32_t k = i; k < n; k++) dst[k] = src[k];
+    }
+}
+
 // arg-max with the reference's rule (larger value, ties to the lower index; a NaN never wins; the search starts from
 // (-FLT_MAX, 0)): crates/rnb-backend/cuda/cuda/kernels/quant_batch_and_ops.cuh:3286-3328.  Stage 1 reduces `len`
 // values to one candidate per workgroup, stage 2 (one workgroup, in = stage 1's candidates) to the result.
@@ -120,6 +131,12 @@ __global__ void __launch_bounds__(256)
 }
 
 }  // namespace
+
+void launch_copy_words(const void *src, void *dst, size_t n_words, hipStream_t stream) {
+    if (n_words == 0) return;
+    hipLaunchKernelGGL(copy_words_kernel, dim3(static_cast<uint32_t>((n_words + 1023) / 1024)), dim3(256), 0, stream,
+                       static_cast<const uint32_t *>(src), static_cast<uint32_t *>(dst), static_cast<uint32_t>(n_words));
+}
 
 void launch_argmax(const float *values, uint32_t len, float *scratch_values, uint32_t *scratch_indices, float *out_value,
                    uint32_t *out_index, hipStream_t stream) {
