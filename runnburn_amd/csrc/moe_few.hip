@@ -4,11 +4,16 @@
 //   down      slot_out[slot][n_embd] = route[slot] * (Wd[e] . Q8_K(mid[slot])), Q4_K, Q5_K or Q6_K
 // (crates/rnb-llm/src/engine/models/shared_expert_moe/moe_view/fanout.rs, crates/rnb-cpu/src/kernels/activation.rs)
 //
-// An expert's rows are read once per tile and little is computed with them, so what counts are waves in flight: a wave needs its stage
-// of LDS and about 90 registers and waits for nobody.  moe_mfma.hip's workgroups stage a whole tile of 32 slots first and leave most of
-// the chip idle where experts are few.  A wave walks its rows' blocks in order with the same roundings, so the bits are those of
-// moe_mfma.hip.  Two and four K slices a row tile, as in gemm_few.hip, were up to 10 % faster on the smallest grids (8 experts of 2048 x 4096
-// at 64 tokens 61 us against 68) and 5 % slower on large ones; 32 rows a wave 5 - 25 % slower.
+// An expert's rows are read once per tile and little is computed with them, so what counts are waves in flight.  The four waves of a
+// workgroup share the tile's activations (each fetches a quarter of the next block's while the present one's are used, one barrier a
+// block) and have strips of LDS of their own for their rows: 42 KB for gate and up with 32 slots, three workgroups a compute unit.
+// moe_mfma.hip's workgroups stage a whole tile of all blocks first, which leaves room for one, and 191 tiles of 128 experts
+// x top-8 at 512 tokens kept 191 of 256 units busy.  A wave walks its rows' blocks in order with the same roundings, so the bits are
+// those of moe_mfma.hip.  Measured, us a call (moe_mfma.hip : every wave with activations of its own : shared): 128 x top-8 of 768 x
+// 2048 at 512 tokens 194 : 203 : 177, at 64 110 : 103 : 99, 64 x top-8 of 512 x 2816 at 446 161 : 138 : 130, 128 x top-8 of 1024 x 4096 at
+// 512 466 : 450 : 390; grids that fit at once wait for the barrier instead (8 x top-2 of 2048 x 4096 at 64 93 : 61 : 64).  Two waves a
+// workgroup 10 % slower, eight 7 - 15 %, 32 rows a wave 5 - 25 %; two and four K slices a row tile were up to 10 % faster on the smallest
+// grids and 5 % slower on large ones.
 #include "gemm_few.h"
 
 namespace rnb {
@@ -16,6 +21,16 @@ namespace rnb {
 namespace {
 
 constexpr int kMfWaves = 4;
+
+// a workgroup's LDS: the waves' strips (one per matrix), then two buffers with a block's activations, sums and scales of the tile's slots
+template <uint32_t kFmt, int kMT, int kMats>
+struct MfLds {
+    typedef FewLds<kFmt, kMT, 1, kMats> L;
+    static constexpr int kStrips = kMats * L::kStrip;  // a wave's
+    static constexpr int kDig = kMT * 4096, kDx = kDig + (FewRows<kFmt>::kMins ? kMT * 256 : 0), kBuf = kDx + 256;
+    static constexpr int kBytes = kMfWaves * kStrips + 2 * kBuf;
+    static_assert(kBytes <= 160 * 1024, "LDS of a compute unit");
+};
 
 template <uint32_t kFmt, int kMT, int kMats>
 __global__ void __launch_bounds__(kWave *kMfWaves)
@@ -25,7 +40,9 @@ __global__ void __launch_bounds__(kWave *kMfWaves)
                    const uint32_t *__restrict__ act_rows, const uint32_t *__restrict__ out_rows,
                    const float *__restrict__ out_scale, float *__restrict__ out, uint32_t rows, uint32_t nb, uint32_t unit0) {
     typedef FewLds<kFmt, kMT, 1, kMats> L;
+    typedef MfLds<kFmt, kMT, kMats> S;
     typedef FewRows<kFmt> R;
+    constexpr int kActs = kMfWaves * S::kStrips;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -35,44 +52,50 @@ __global__ void __launch_bounds__(kWave *kMfWaves)
     const uint32_t row0 = (blockIdx.x * kMfWaves + wave) * 16;
     const uint32_t first = min(row0, (rows - 1) & ~15u), last_row = min(rows - 1 - first, 15u);  // clamped loads, masked stores
     const uint32_t row_bytes = nb * static_cast<uint32_t>(R::kBytes), last_tok = live - 1;
-    constexpr int kStage = L::kStage + 256;  // and a scale per lane
-    uint8_t *stage = lds + wave * kStage;
-    const uint32_t stage0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds)) + wave * kStage;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds));
+    const uint8_t *strips = lds + wave * S::kStrips;
+    const uint32_t strips0 = lds0 + wave * S::kStrips;
     const size_t per_expert = static_cast<size_t>(rows) * row_bytes, at = static_cast<size_t>(first) * row_bytes;
     const uint8_t *w_base[2] = {expert_base(w_all, w_shared, n_routed, expert, per_expert) + at,
                                 expert_base(w2_all, w2_shared, n_routed, expert, per_expert) + at};
 
-    // the list before the first fill: loads return in order, and the compiler counts its own only
+    // the list before the first fill: loads return in order, and the compiler counts its own only.  The waves share the fetching of the
+    // tile's activations, four slots a load
     const uint32_t *list = act_rows + start;
     const uint32_t rr = __umul24(lane, R::kInv) >> 16, j = lane - rr * R::kPieces;
-    uint32_t row_off[L::kFills], act_off[4 * kMT], dig_off[kMT];
+    constexpr int kGroups = (4 * kMT + kMfWaves - 1) / kMfWaves;
+    uint32_t row_off[L::kFills], act_off[kGroups];
 #pragma unroll
-    for (int g = 0; g < 4 * kMT; g++)
-        act_off[g] = list[min(static_cast<uint32_t>(4 * g + kq), last_tok)] * (nb * 256u) + 16 * (l16 ^ (4 * (g & 3) + kq));
-#pragma unroll
-    for (int t = 0; t < kMT; t++)  // a token's sixteen bytes are four lanes' dwords
-        dig_off[t] = list[min(static_cast<uint32_t>(16 * t + (lane >> 2)), last_tok)] * (nb * 16u) + 4 * (lane & 3);
+    for (int i = 0; i < kGroups; i++) {
+        const uint32_t g = wave + i * kMfWaves;
+        act_off[i] = list[min(4 * g + kq, last_tok)] * (nb * 256u) + 16 * (l16 ^ (4 * (g & 3) + kq));
+    }
+    // a token's sixteen bytes of sums are four lanes' dwords
+    const uint32_t dig_off = list[min(16 * (wave % kMT) + (lane >> 2), last_tok)] * (nb * 16u) + 4 * (lane & 3);
     const uint32_t dx_off = list[min(static_cast<uint32_t>(lane), last_tok)] * (nb * 4u);
 #pragma unroll
     for (int k = 0; k < L::kFills; k++) row_off[k] = min(k * R::kPer + rr, last_row) * row_bytes;
 
     auto run = [&](auto tiles_tag) {  // with the token tiles that have live slots
         constexpr int kLive = decltype(tiles_tag)::value;
-        auto issue = [&](uint32_t b) {
+        auto issue_w = [&](uint32_t b) {
 #pragma unroll
             for (int m = 0; m < kMats; m++) {
                 const uint8_t *src = w_base[m] + R::block_off(b);
 #pragma unroll
-                for (int k = 0; k < L::kFills; k++) lds_fill16(src, R::piece(row_off[k], j, b), stage0 + m * L::kStrip + k * 1024);
+                for (int k = 0; k < L::kFills; k++) lds_fill16(src, R::piece(row_off[k], j, b), strips0 + m * L::kStrip + k * 1024);
             }
-            const uint8_t *act = reinterpret_cast<const uint8_t *>(aq) + b * 256u;
+        };
+        auto issue_a = [&](uint32_t b) {
+            const uint32_t dst = lds0 + kActs + (b & 1) * S::kBuf;
 #pragma unroll
-            for (int g = 0; g < 4 * kLive; g++)
-                if (4u * g < live) lds_fill16(act, act_off[g], stage0 + L::kAct + g * 1024);  // places of no slot keep what they hold
+            for (int i = 0; i < kGroups; i++) {
+                const uint32_t g = wave + i * kMfWaves;  // places of no slot keep what they hold
+                if (g < 4u * kLive && 4 * g < live) lds_fill16(reinterpret_cast<const uint8_t *>(aq) + b * 256u, act_off[i], dst + g * 1024);
+            }
             if constexpr (R::kMins)
-#pragma unroll
-                for (int t = 0; t < kLive; t++) lds_fill4(adig + b * 16u, dig_off[t], stage0 + L::kDig + t * 256);
-            lds_fill4(reinterpret_cast<const uint8_t *>(ad) + b * 4u, dx_off, stage0 + L::kStage);
+                if (wave < kLive) lds_fill4(adig + b * 16u, dig_off, dst + S::kDig + wave * 256);
+            if (wave == kMfWaves - 1) lds_fill4(reinterpret_cast<const uint8_t *>(ad) + b * 4u, dx_off, dst + S::kDx);
         };
         float acc[kMats][1][kLive][4];
 #pragma unroll
@@ -81,13 +104,17 @@ __global__ void __launch_bounds__(kWave *kMfWaves)
             for (int t = 0; t < kLive; t++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc[m][0][t][r] = 0.0f;
-        issue(0);
+        issue_a(0);
+        issue_w(0);
         for (uint32_t b = 0; b < nb; b++) {
             wait_fills();
+            __syncthreads();  // everybody's part of block b has come, block b - 1 has been read
+            if (b + 1 < nb) issue_a(b + 1);
+            const int at = static_cast<int>(kActs + (b & 1) * S::kBuf - wave * S::kStrips);  // from the wave's strips
             FewBlock<kFmt, kLive, 1, kMats> blk;
-            blk.read(stage, L::kAct, L::kDig, reinterpret_cast<const float *>(stage + L::kStage), l16, kq, last_row, nb, b);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read
-            if (b + 1 < nb) issue(b + 1);
+            blk.read(strips, at, at + S::kDig, reinterpret_cast<const float *>(strips + at + S::kDx), l16, kq, last_row, nb, b);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the strips have been read
+            if (b + 1 < nb) issue_w(b + 1);
             blk.template multiply<true>(acc, kq);
         }
         const uint32_t row = row0 + l16;
@@ -118,8 +145,7 @@ void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, cons
                     const MoeGroups &g, const uint32_t *act_rows, const float *scale, float *out, uint32_t rows, uint32_t nb,
                     hipStream_t stream) {
     static bool configured = false;
-    constexpr size_t lds = kMfWaves * (FewLds<kFmt, kMT, 1, kMats>::kStage + 256);
-    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+    constexpr size_t lds = MfLds<kFmt, kMT, kMats>::kBytes;
     if (!allow_dynamic_lds(reinterpret_cast<const void *>(moe_few_kernel<kFmt, kMT, kMats>), lds, &configured, "moe_few_kernel")) return;
     for (uint32_t u = 0; u < g.n_units; u += 65535)  // grid rows that a device is sure to take
         hipLaunchKernelGGL((moe_few_kernel<kFmt, kMT, kMats>), dim3((rows + 16 * kMfWaves - 1) / (16 * kMfWaves), std::min(g.n_units - u, 65535u)),
@@ -129,18 +155,22 @@ void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, cons
 
 }  // namespace
 
-uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 16 * n_groups ? 16 : 32; }
+// us a call with tiles of 16 : of 32: 15.7 slots a group on average (64 x top-8 of 1792 x 1792 at 120 tokens) 139 : 126, 15 (32 x top-4 of
+// 768 x 2048 at 120) 51.0 : 49.6; 12.5 (64 x top-8 of 512 x 2816 at 100) 61.9 : 65.4, (16 x top-2 of 1536 x 1536 at 100) 36.3 : 39.9
+uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 14 * n_groups ? 16 : 32; }
 
 // Against the tiles of moe_mfma.hip and the integer-dot kernels of moe.hip, us a call, those : this.  From sixteen tokens on (a
-// smaller batch's rows are a lone token's bit for bit): 8 experts x top-2 of 1792 x 2304 at 52 tokens 64 : 40, 16 x top-2 of 1536 x
-// 1536 at 38 66 : 38, 128 x top-8 of 1536 x 2560 at 238 320 : 286, of 1024 x 1280 at 27 87 : 63.  Many experts with short intermediates and
-// several slots each stay on moe_mfma.hip, whose workgroups walk more rows per list and quantise as they stage (128 x top-8 of 768 x
-// 2048 at 512 tokens 189 : 204, at 64 104.7 : 106; 64 x top-8 of 512 x 2816 at 446 155 : 157); one slot or two per expert on
-// moe.hip, whose dots cost little then (16 x top-2 of 1536 x 3072 at 18 tokens, Q5_K down projection, 43.0 : 45.9, 32 x top-4 of 768 x
-// 1792 at 21 34.3 : 37.8).
-bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_mid, uint32_t down_quant) {
+// smaller batch's rows are a lone token's bit for bit): 8 experts x top-2 of 1792 x 2304 at 52 tokens 66 : 43, 16 x top-2 of 1536 x
+// 1536 at 300 83 : 54, 128 x top-8 of 1536 x 2560 at 238 343 : 290, of 768 x 2048 at 2048 540 : 476.  Many experts with less than three
+// slots each and short rows have no wave in flight for long enough (128 x top-8 of 768 x 1536, Q5_K, at 35 tokens 60.7 : 66.3, of 768 x
+// 1280, Q4_K, at 21 46.2 : 51.5, of 1024 x 1280 at 30 57.2 : 59.7; with longer inputs of 768 x 2560 at 22 77.7 : 73.1, of 512 x 3072, Q5_K, at
+// 30 88.4 : 74.8, but a Q6_K down projection of 768 x 2048 at 30 78.3 : 80.4); one slot or two per expert stay on moe.hip, whose dots
+// cost little then (16 x top-2 of 1536 x 3072 at 18 tokens, Q5_K down projection, 42.4 : 46.0).
+bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid, uint32_t down_quant) {
     if (token_count < 16) return false;
-    if (nb_mid <= 3 && (n_slots >= 2048 || (n_groups >= 80 && n_slots >= 4 * n_groups))) return false;
+    if (nb_mid <= 4 && n_groups >= 80 && n_slots < 3 * n_groups &&
+        (nb_in <= 6 || (nb_mid <= 3 && down_quant == kQ6K && 10 * n_slots >= 18 * n_groups)))
+        return false;
     if (nb_mid <= 4 && max_group <= 8 && 10 * n_slots < 16 * n_groups) return false;
     return down_quant == kQ6K || n_slots >= 100 || n_slots >= 3 * n_groups;
 }

@@ -1,5 +1,5 @@
 """Routed experts on the few-token GEMM's tiles (moe_few.hip): groups of every size around the 16- and 32-slot tiles, row tiles with
-remainders, few and many workgroups (16 and 32 rows a wave, one to four K slices), a shared expert.  Against the oracle; outputs
+remainders, few and many workgroups, a shared expert.  Against the oracle; outputs
 outside the plain per-row tolerance must be whole re-quantisation flips (oracle/flips.py)."""
 import numpy as np
 import pytest
@@ -25,6 +25,7 @@ def _lists(groups, tokens, rng):
     (17, [1, 2, 15, 16, 17, 3], 768, 512, False),           # tiles of 16, one group in two of them
     (40, [16, 17, 31, 32, 33, 1, 40], 512, 1024, False),    # tiles of 32: one and two token tiles, and a second unit of one slot
     (70, [70, 65, 64, 2, 33], 1280, 768, True),             # groups of several units, K slices of unequal length
+    (48, [48, 20] * 41, 256, 512, False),                   # many experts with short intermediates, a block and an even number
     (16, [5, 4, 3] * 10, 1024, 1280, True),                 # small groups, five blocks in
 ])
 def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant):
