@@ -748,7 +748,7 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     const size_t n_groups = grp_expert.size();
     uint32_t max_group = 0;
     for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
-    // Batches with at least 1.8 slots per routed expert on average: the expert GEMMs run on the matrix cores (a
+    // Batches that moe_few.hip does not take (moe_few_pays), with at least 1.8 slots per routed expert on average: moe_mfma.hip (a
     // 32-token tile costs the same whatever its number of live tokens, the integer-dot kernels cost per token; measured
     // on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot kernels, 79.0 / 85.7 / 88.2
     // on the matrix cores; the ratio is 1.6 / 1.8 / 1.9 there) and need the quantiser's digits
