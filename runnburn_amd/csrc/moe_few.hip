@@ -156,7 +156,9 @@ void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, cons
 }  // namespace
 
 // us a call with tiles of 16 : of 32: 15.7 slots a group on average (64 x top-8 of 1792 x 1792 at 120 tokens) 139 : 126, 15 (32 x top-4 of
-// 768 x 2048 at 120) 51.0 : 49.6; 12.5 (64 x top-8 of 512 x 2816 at 100) 61.9 : 65.4, (16 x top-2 of 1536 x 1536 at 100) 36.3 : 39.9
+// 768 x 2048 at 120) 51.0 : 49.6; 12.5 (64 x top-8 of 512 x 2816 at 100) 61.9 : 65.4, (16 x top-2 of 1536 x 1536 at 100) 36.3 : 39.9.  Tiles of
+// 64 (200 registers, two waves a SIMD) against 32: 128 x top-8 of 768 x 2048 at 512 tokens 191 : 175, at 1024 275 : 273, at 2048 455 : 472, 16 x
+// top-2 of 1024 x 2304 at 400 72 : 66; only 8 x top-2 of 2048 x 4096 at 400 gained much (115 : 135).
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 14 * n_groups ? 16 : 32; }
 
 // Against the tiles of moe_mfma.hip and the integer-dot kernels of moe.hip, us a call, those : this.  From sixteen tokens on (a
