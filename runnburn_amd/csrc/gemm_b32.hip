@@ -1,7 +1,7 @@
 // Prefill GEMM of the 32-element formats (Q8_0, Q8_1, Q4_0, Q4_1, Q5_0, Q5_1) for batches of more than 32 tokens on rows of whole
 // 256-element steps: out[seq][rows], same contract as the GEMVs.  Per block of 32 elements
 //   out += (d * d_x) * I,  I = sum code * a (exact, one v_mfma_i32_32x32x32_i8)
-//   out += m * (d_x * sum a)                                                     (Q4_1, Q5_1)
+//   out += (m + c d) * (d_x * sum a), with code - c for the code                 (Q4_1, Q5_1)
 // (crates/rnb-cpu/src/gemm/neon_dot.rs:376-436, neon_quant.rs:236-253)
 //
 // What bounds it is the vector port: a result takes a conversion and a multiply-add per block, 32 instructions of 4 cycles
@@ -14,9 +14,15 @@
 //   part 2             the second block's I, beside the update with the first.
 // Two sets of d * d_x, 212 registers with four token tiles.  A pair takes 284 cycles of a wave, 256 of them the update's.
 // The mins are a product over the blocks by themselves, m[row][block] against d_x * sum a[block][token]: a K = 2 f32 product per
-// pair and one addition per result and step (before: a product with ones, conversion and update per block).
+// pair and one addition per result and step (before: a product with ones, conversion and update per block).  That adds eight blocks'
+// codes before their mins, so neither may be large where their sum is small, as d * code and m are with tokens of any mean: codes are
+// counted from c, the one nearest to the value 0 of its block, which leaves m + c d of at most d / 2 where a block's values have both
+// signs (rms error against f64, gemm_blocks.hip : c = 0 : this, geometric mean of 23 shapes: Q4_1 1.9e-7 : 2.2e-7 : 1.1e-7 with tokens of
+// mean 0, 2.4e-7 : 5.5e-7 : 1.0e-7 with mean 1, Q5_1 1.8 : 1.9 : 1.2 and 2.5 : 6.3 : 1.2.  An origin of 8 or 16 would do as well but for blocks
+// whose codes are mostly 0.)  It costs 27 vector instructions per pair of blocks and step, 5 % of a call.
 // Measured per call (quantiser and slice sum included), gemm_blocks.hip -> this, us: Q8_0 4096 x 4096 x 333 tokens 54.6 -> 34.4, x 2048
-// 166 -> 107, 4096 x 14336 x 300 107 -> 80, Q4_0 20 % less on average, Q5_1 4096 x 4096 x 2048 225 -> 165; over 101 random shapes 0.79.
+// 166 -> 107, 4096 x 14336 x 300 107 -> 80, Q4_0 20 % less on average, Q5_1 4096 x 4096 x 2048 223 -> 178, Q4_1 225 -> 165; over 101 random
+// shapes 0.79, the two with mins over 46 0.80.
 #include "gemm_digits.h"
 
 namespace rnb {
@@ -30,6 +36,7 @@ struct B32 {
     static constexpr bool kNibbles = kFmt == kQ4_0 || kFmt == kQ4_1 || kFmt == kQ5_0 || kFmt == kQ5_1;
     static constexpr bool kFifth = kFmt == kQ5_0 || kFmt == kQ5_1;
     static constexpr bool kMin = kFmt == kQ4_1 || kFmt == kQ5_1;  // value = d * code + m
+    static constexpr float kTop = kFifth ? 31.0f : 15.0f;
     static constexpr int kBytes = kFmt == kQ8_0 ? 34 : kFmt == kQ8_1 ? 36 : kFmt == kQ4_0 ? 18 : kFmt == kQ4_1 ? 20 : kFmt == kQ5_0 ? 22 : 24;
     static constexpr int kQhOff = kMin ? 4 : 2;
     static constexpr int kQsOff = kFmt == kQ8_0 ? 2 : kFmt == kQ8_1 ? 4 : kBytes - 16;
@@ -83,8 +90,8 @@ struct B32Block {
         }
     }
     // nibbles by K-half, fifth bits spread with one multiply per four (bit j of a 4-bit group to bit 8 j), the symmetric formats'
-    // offset (8, 16) taken in packed bytes
-    __device__ __forceinline__ v4i codes(int khalf) const {
+    // offset (8, 16) and the others' origin (zero_bytes: 128 - origin in each byte) taken in packed bytes
+    __device__ __forceinline__ v4i codes(int khalf, [[maybe_unused]] uint32_t zero_bytes) const {
         typedef B32<kFmt> F;
         v4i o;
 #pragma unroll
@@ -95,6 +102,7 @@ struct B32Block {
                 if constexpr (F::kFifth) v |= ((((qh >> (16 * khalf + 4 * i)) & 0xfu) * 0x00204081u) & 0x01010101u) << 4;
                 if constexpr (kFmt == kQ4_0) v = (v + 0x78787878u) ^ 0x80808080u;  // n - 8 per byte, no carries
                 if constexpr (kFmt == kQ5_0) v = (v + 0x70707070u) ^ 0x80808080u;  // n - 16
+                if constexpr (F::kMin) v = (v + zero_bytes) ^ 0x80808080u;         // n - origin
             }
             o[i] = static_cast<int>(v);
         }
@@ -191,10 +199,21 @@ __global__ void __launch_bounds__(kDgThreads, 2)
         return khalf ? upper : lower;
     };
     auto take = [&](int p) {  // the next step's pair p in place of the present one
-        bop[2 * p] = n0.codes(khalf);
-        bop[2 * p + 1] = n1.codes(khalf);
-        dk[p] = of_half(f16_bits_to_f32(n0.dh), f16_bits_to_f32(n1.dh));
-        if constexpr (F::kMin) mk[p] = of_half(f16_bits_to_f32(n0.dh >> 16), f16_bits_to_f32(n1.dh >> 16));
+        const float d = of_half(f16_bits_to_f32(n0.dh), f16_bits_to_f32(n1.dh));
+        uint32_t zero0 = 0, zero1 = 0;
+        dk[p] = d;
+        if constexpr (F::kMin) {
+            // d n + m = d (n - c) + (m + c d), c the code nearest to the value 0.  (No d, infinities, NaN: c = 0, m as it is.)
+            const float m = of_half(f16_bits_to_f32(n0.dh >> 16), f16_bits_to_f32(n1.dh >> 16));
+            const float c = __builtin_rintf(fminf(fmaxf(-m * __builtin_amdgcn_rcpf(d), 0.0f), F::kTop));
+            mk[p] = c > 0.0f ? __builtin_fmaf(c, d, m) : m;
+            const uint32_t z = __builtin_amdgcn_perm(0u, 128u - static_cast<uint32_t>(c), 0u);  // its low byte in all four
+            const auto both = __builtin_amdgcn_permlane32_swap(z, z, false, false);
+            zero0 = both[0];
+            zero1 = both[1];
+        }
+        bop[2 * p] = n0.codes(khalf, zero0);
+        bop[2 * p + 1] = n1.codes(khalf, zero1);
     };
 #define RNB_B32_FETCH(P)                            \
     {                                               \
@@ -294,6 +313,7 @@ __global__ void __launch_bounds__(kDgThreads, 2)
                 if (t == kT - 1) {
                     take(p);
                     asm volatile("" : "+v"(bop[2 * p]), "+v"(bop[2 * p + 1]), "+v"(dk[p]));
+                    if constexpr (F::kMin) asm volatile("" : "+v"(mk[p]));
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }

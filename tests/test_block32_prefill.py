@@ -81,3 +81,29 @@ def test_a_token_does_not_see_its_neighbours(rnb, oracle, quant):
     rnb.release(w)
     keep = [t for t in range(seq) if t not in (1, 40, seq - 1)]
     assert np.array_equal(a[keep].view(np.uint32), b[keep].view(np.uint32))
+
+
+@pytest.mark.parametrize("quant", [Q4_1, Q5_1])
+@pytest.mark.parametrize("mean", [0.0, 0.5, 1.0])
+@pytest.mark.parametrize("weights", ["quantised", "skewed"])
+def test_minimum_formats_on_tokens_of_any_mean(rnb, oracle, quant, mean, weights):
+    """d * code and m are of one size and opposite sign where a block's weights are centred, as are their products with tokens that are
+    not: an order of the sums that adds many blocks' codes before their mins carries the difference of two large numbers.  In an
+    order that does not, every addition rounds by at most 2^-24 of the running sum, whose rms grows with the root of the blocks added:
+    rms error <= 2^-24 * sqrt(blocks / 2) of the rms result.  Skewed: m = 0 and most codes 0, where a fixed offset of the codes would be
+    the large number."""
+    rows, cols, seq = 96, 8192, 65
+    if weights == "quantised":
+        w = oracle.make_weights(quant, rows, cols, 27)
+    else:
+        rng = np.random.default_rng(28)
+        blocks = np.zeros((rows * cols // 32, BYTES[quant]), np.uint8)
+        blocks[:, 0:2] = (np.abs(rng.standard_normal((len(blocks), 1))) * 0.01).astype(np.float16).view(np.uint8)
+        blocks[:, BYTES[quant] - 16:] = np.where(rng.random((len(blocks), 16)) < 0.1, rng.integers(0, 256, (len(blocks), 16)), 0)
+        w = blocks.reshape(-1)
+    x = oracle.fill_normal(seq * cols, 29, 1.0) + np.float32(mean)
+    got = np.asarray(getattr(rnb, BATCH[quant])(w, rows, cols, x), np.float64).reshape(seq, rows)
+    rnb.release(w)
+    gold = np.asarray(oracle.gemv(quant, w, rows, cols, x, gold=True), np.float64).reshape(seq, rows)
+    error = np.sqrt(np.mean((got - gold) ** 2) / np.mean(gold * gold))
+    assert error <= 2.0 ** -24 * np.sqrt(cols / 32 / 2), error
