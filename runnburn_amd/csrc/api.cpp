@@ -97,7 +97,7 @@ constexpr size_t kDigitsMinSeq = 3;  // the fewest tokens gemm_few_pays answers 
 // against 21.5 - 25.7).
 constexpr size_t kIqGemmMinSeq = 5;
 // Minimum tokens for which the grouped MoE GEMMs on the matrix cores are considered.
-constexpr size_t kMoeMfmaMinTokens = 16;
+constexpr size_t kMoeMatrixMinTokens = 16;
 // Minimum number of 256 x 64 tiles for which the Q4_K ping-pong GEMM replaces the smaller-tile kernel.
 constexpr uint64_t kGemmBigTilesMin = 32;
 
@@ -748,23 +748,24 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     const size_t n_groups = grp_expert.size();
     uint32_t max_group = 0;
     for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
-    // Batches that moe_few.hip does not take (moe_few_pays), with at least 1.8 slots per routed expert on average: moe_mfma.hip (a
-    // 32-token tile costs the same whatever its number of live tokens, the integer-dot kernels cost per token; measured
-    // on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot kernels, 79.0 / 85.7 / 88.2
-    // on the matrix cores; the ratio is 1.6 / 1.8 / 1.9 there) and need the quantiser's digits
-    // (its gate/up rows arrive as 16-byte LDS-direct loads: other alignments take the vector kernels)
-    // (and the Q6_K down rows as dword-aligned pieces: an even base address and whole 128-row tiles)
+    // Batches of sixteen tokens and more run on the matrix cores: moe_few.hip, or moe_mfma.hip for small calls (moe_few_pays) with at
+    // least 1.8 slots per routed expert on average (a 32-token tile costs the same whatever its number of live tokens, the
+    // integer-dot kernels cost per token; measured on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot
+    // kernels, 79.0 / 85.7 / 88.2 in moe_mfma.hip; the ratio is 1.6 / 1.8 / 1.9 there), which needs the quantiser's digits
+    // (its gate/up rows arrive as 16-byte LDS-direct loads and the Q6_K down rows as dword-aligned pieces: an even base address and
+    // whole 128-row tiles).  Tables of a kernel argument's size ride in one, with the integer-dot kernels, unless that ratio is met.
     const uintptr_t addresses = reinterpret_cast<uintptr_t>(gate_dev) | reinterpret_cast<uintptr_t>(up_dev) |
                                 reinterpret_cast<uintptr_t>(down_dev) | reinterpret_cast<uintptr_t>(shared.gate) |
                                 reinterpret_cast<uintptr_t>(shared.up) | reinterpret_cast<uintptr_t>(shared.down);
     const bool aligned16 = addresses % 16 == 0, aligned4 = addresses % 4 == 0;
-    const bool mfma = token_count >= kMoeMfmaMinTokens && 10 * n_slots >= 18 * n_groups && aligned16 && n_embd % 128 == 0 &&
+    const bool matrix_batch = token_count >= kMoeMatrixMinTokens;
+    const bool mfma = matrix_batch && 10 * n_slots >= 18 * n_groups && aligned16 && n_embd % 128 == 0 &&
                       moe_mfma_supported(static_cast<uint32_t>(sh.nb_in), static_cast<uint32_t>(sh.nb_mid), down_quant);
     // one table image: route[n] | tok_offsets[T+1] | tok_slots[n] | sorted_slot[n] | sorted_token[n] | grp_expert[G] |
     // grp_start[G+1] | slot_expert[n] | units
     size_t table_words = 5 * n_slots + (token_count + 1) + n_groups + (n_groups + 1);
     const bool inline_tables = !mfma && table_words <= kMoeInlineWords;  // decode-sized: rides in a kernel argument
-    const bool few = !inline_tables && aligned4 && moe_few_pays(token_count, n_slots, n_groups, max_group, sh.nb_in, sh.nb_mid, down_quant) &&
+    const bool few = matrix_batch && !inline_tables && aligned4 && (!mfma || moe_few_pays(n_groups, max_group, sh.nb_in, sh.nb_mid)) &&
                      moe_few_supported(sh.nb_in, sh.nb_mid, token_count, n_slots, n_ff, n_embd, down_quant);
     const uint32_t unit_tokens = moe_few_tile(n_slots, n_groups);
     std::vector<uint32_t> units;

@@ -244,7 +244,8 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
 // the same two steps on the few-token GEMM's tiles (moe_few.hip): groups with units of moe_few_tile slots, weights at 4-byte
 // addresses, both activations quantised with digits
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups);
-bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid, uint32_t down_quant);
+constexpr size_t kMoeMfmaMaxGroup = 8;
+bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid);
 bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant);
 void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
                             float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);

@@ -161,20 +161,15 @@ void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, cons
 // top-2 of 1024 x 2304 at 400 72 : 66; only 8 x top-2 of 2048 x 4096 at 400 gained much (115 : 135).
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 14 * n_groups ? 16 : 32; }
 
-// Against the tiles of moe_mfma.hip and the integer-dot kernels of moe.hip, us a call, those : this.  From sixteen tokens on (a
-// smaller batch's rows are a lone token's bit for bit): 8 experts x top-2 of 1792 x 2304 at 52 tokens 66 : 43, 16 x top-2 of 1536 x
-// 1536 at 300 83 : 54, 128 x top-8 of 1536 x 2560 at 238 343 : 290, of 768 x 2048 at 2048 540 : 476.  Many experts with less than three
-// slots each and short rows have no wave in flight for long enough (128 x top-8 of 768 x 1536, Q5_K, at 35 tokens 60.7 : 66.3, of 768 x
-// 1280, Q4_K, at 21 46.2 : 51.5, of 1024 x 1280 at 30 57.2 : 59.7; with longer inputs of 768 x 2560 at 22 77.7 : 73.1, of 512 x 3072, Q5_K, at
-// 30 88.4 : 74.8, but a Q6_K down projection of 768 x 2048 at 30 78.3 : 80.4); one slot or two per expert stay on moe.hip, whose dots
-// cost little then (16 x top-2 of 1536 x 3072 at 18 tokens, Q5_K down projection, 42.4 : 46.0).
-bool moe_few_pays(size_t token_count, size_t n_slots, size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid, uint32_t down_quant) {
-    if (token_count < 16) return false;
-    if (nb_mid <= 4 && n_groups >= 80 && n_slots < 3 * n_groups &&
-        (nb_in <= 6 || (nb_mid <= 3 && down_quant == kQ6K && 10 * n_slots >= 18 * n_groups)))
-        return false;
-    if (nb_mid <= 4 && max_group <= 8 && 10 * n_slots < 16 * n_groups) return false;
-    return down_quant == kQ6K || n_slots >= 100 || n_slots >= 3 * n_groups;
+// Against the integer-dot kernels of moe.hip from sixteen tokens on (a smaller batch's rows are a lone token's bit for bit), against
+// moe_mfma.hip unless every group is at most kMoeMfmaMaxGroup slots and the call small: that kernel finishes only the results of eight
+// slots and its down projection quantises the intermediates itself, one launch of 5 us less, which counts where the experts' weights
+// are read in 30 - 60 us; up to sixteen groups leave its one workgroup a unit idle.  Us a call, moe_mfma : this, Q5_K down projections:
+// 128 x top-8 of 256 x 2304 at 21 tokens 36.7 : 42.7, of 1024 x 1024 at 19 44.9 : 50.7; 512 x 3328 at 21 (2366 blocks) 92.7 : 76.1, 8 x top-2 of
+// 2048 x 1024, Q6_K, at 26 38.2 : 29.1.  780 random calls of 16 to 300 tokens (3 to 194 experts hit, rows of 3 to 18 blocks, intermediates of
+// 1 to 10): 0.25 % over the better one of the two on average, 19 of them 3 - 13 % behind moe_mfma.hip (mostly Q5_K with groups of 9 to 15).
+bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid) {
+    return max_group > kMoeMfmaMaxGroup || n_groups <= 16 || n_groups * nb_in * nb_mid >= 2000;
 }
 
 bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant) {

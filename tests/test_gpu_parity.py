@@ -893,12 +893,10 @@ def test_moe_small_batch_equals_general_sequence(rnb, oracle, tokens, n_ff, n_em
                                                                      (40, 5, 3, 1024, 256, Q4_K), (20, 64, 3, 256, 512, Q6_K),
                                                                      (64, 128, 8, 256, 1792, Q6_K), (48, 96, 8, 256, 1792, Q4_K)])
 def test_moe_prefill_matrix_core_path(rnb, oracle, tokens, n_expert, k, n_ff, n_embd, down_quant):
-    """16 or more tokens and at least 1.8 slots per routed expert on average: the grouped expert GEMMs on the matrix
-    cores (32-token tiles per expert; experts with more than 32 tokens take several tiles, experts with few run mostly
-    padding); the sixth case stays below that average and keeps the integer-dot kernels; in the last two the down
-    kernel's workgroups walk four row tiles each (14 row tiles x ~100 expert groups: the last workgroup of a group gets two).
-    Against the oracle, and a token's row must
-    not depend on the batch: the same bits with the tokens in reverse order."""
+    """16 or more tokens: the grouped expert GEMMs on the matrix cores in tiles of 16 or 32 slots (experts with more take
+    several tiles, experts with few run mostly padding); groups of a slot or two in the sixth case, about a hundred groups
+    in the last two.  Against the oracle, and a token's row must not depend on the batch: the same bits with the tokens in
+    reverse order."""
     gate, up, down, x, e, r, t = _moe_case(oracle, n_expert, n_ff, n_embd, tokens, k, 90 + tokens, down_quant)
     got = rnb.qwen35_sparse_experts_selected_base_by_token(gate, up, down, e, r, t, tokens, down_quant, n_ff, n_embd, x)
     ref = oracle.moe_sparse_experts_by_token(gate, up, down, n_expert, e, r, t, tokens, down_quant, n_ff, n_embd, x)
@@ -1385,8 +1383,7 @@ def test_moe_shared_expert_slot_on_the_matrix_cores_dev(rnb, oracle):
 @pytest.mark.parametrize("tokens,n_ff,n_embd,down_quant", [(100, 512, 256, Q6_K), (97, 256, 768, Q4_K), (64, 1280, 256, Q5_K)])
 def test_moe_few_experts_take_most_tokens(rnb, oracle, tokens, n_ff, n_embd, down_quant):
     """Two experts that every token is routed to (two to four token tiles each, the last of one to thirty-two slots) among a
-    hundred with a slot or two: workgroups find their group and token tile across three 64-group steps of the search.
-    Against the oracle, and the same bits with the tokens in reverse order."""
+    hundred with a slot or two.  Against the oracle, and the same bits with the tokens in reverse order."""
     n_expert = 140
     gate, up, down, x, *_ = _moe_case(oracle, n_expert, n_ff, n_embd, tokens, 1, 1500 + tokens, down_quant)
     rng = np.random.default_rng(tokens)
@@ -1440,11 +1437,10 @@ def test_moe_more_token_tiles_than_grid_rows(rnb, oracle):
                                                                             (100, 128, 2, 512, 256, Q4_K, False),
                                                                             (16, 48, 8, 1024, 512, Q6_K, True)])
 def test_moe_many_experts_wide_workgroups_ragged_row_tiles_dev(rnb, oracle, tokens, n_expert, k, n_ff, n_embd, down_quant, shared):
-    """Many routed experts with few tokens each: the gate/up kernel runs six-wave workgroups (192 rows a tile) that
-    walk two or three row tiles, and n_ff is no multiple of 192, so a group's last tile has idle waves and its last
-    workgroup fewer tiles.  Device buffers, slots in the callers' (expert, token) order; the last case has the shared
-    expert as the one group of sixteen tokens among groups of a few.  Against the oracle, and the same bits with the
-    tokens in reverse order."""
+    """Many routed experts with few tokens each; the third case, two slots a group, is a small call of moe_mfma.hip (six-wave
+    workgroups of 192 rows, n_ff no multiple of it: idle waves in a group's last tile), the others run in moe_few.hip, the last
+    with the shared expert as the one group of sixteen tokens among groups of a few.  Device buffers, slots in the callers'
+    (expert, token) order.  Against the oracle, and the same bits with the tokens in reverse order."""
     if shared:
         gate, up, down, sh, longer, x, e, r, t = _with_shared(oracle, n_expert, n_ff, n_embd, tokens, k, 700 + tokens, down_quant)
         ne = n_expert + 1

@@ -1,6 +1,6 @@
-"""Routed experts on the few-token GEMM's tiles (moe_few.hip): groups of every size around the 16- and 32-slot tiles, row tiles with
-remainders, few and many workgroups, a shared expert.  Against the oracle; outputs
-outside the plain per-row tolerance must be whole re-quantisation flips (oracle/flips.py)."""
+"""Routed experts of a batch on the matrix cores: on the few-token GEMM's tiles (moe_few.hip: groups of every size around the 16- and
+32-slot tiles, row tiles with remainders, few and many workgroups, a shared expert) and, small calls of groups of up to eight slots, in
+moe_mfma.hip.  Against the oracle; outputs outside the plain per-row tolerance must be whole re-quantisation flips (oracle/flips.py)."""
 import numpy as np
 import pytest
 
@@ -19,16 +19,7 @@ def _lists(groups, tokens, rng):
     return np.array(e, np.uint32)[order], (rng.random(len(e)) + 0.1).astype(np.float32), np.array(t, np.uint32)[order]
 
 
-@pytest.mark.parametrize("down_quant", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("tokens,groups,n_ff,n_embd,shared", [
-    (18, [9, 1, 0, 8, 7, 9, 9], 256, 256, False),           # one block, tiles of 16
-    (17, [1, 2, 15, 16, 17, 3], 768, 512, False),           # tiles of 16, one group in two of them
-    (40, [16, 17, 31, 32, 33, 1, 40], 512, 1024, False),    # tiles of 32: one and two token tiles, and a second unit of one slot
-    (70, [70, 65, 64, 2, 33], 1280, 768, True),             # groups of several units, K slices of unequal length
-    (48, [48, 20] * 41, 256, 512, False),                   # many experts with short intermediates, a block and an even number
-    (16, [5, 4, 3] * 10, 1024, 1280, True),                 # small groups, five blocks in
-])
-def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant):
+def _check(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant):
     from oracle import flips
 
     rng = np.random.default_rng(tokens + n_ff)
@@ -52,3 +43,31 @@ def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shar
     assert v["ok"] or v["flip_aware_ok"], {key: v[key] for key in v if key != "flips"}
     for a in routed + (own or []):
         rnb.release(a)
+
+
+@pytest.mark.parametrize("down_quant", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("tokens,groups,n_ff,n_embd,shared", [
+    (18, [9, 1, 0, 8, 7, 9, 9], 256, 256, False),           # one block, tiles of 16
+    (17, [1, 2, 15, 16, 17, 3], 768, 512, False),           # tiles of 16, one group in two of them
+    (40, [16, 17, 31, 32, 33, 1, 40], 512, 1024, False),    # tiles of 32: one and two token tiles, and a second unit of one slot
+    (70, [70, 65, 64, 2, 33], 1280, 768, True),             # groups of several units, K slices of unequal length
+    (48, [48, 20] * 41, 256, 512, False),                   # many experts with short intermediates, a block and an even number
+    (16, [5, 4, 3] * 10, 1024, 1280, True),                 # small groups, five blocks in
+])
+def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant):
+    _check(rnb, oracle, tokens, groups, n_ff, n_embd, shared, down_quant)
+
+
+# more than 16 groups of at most eight slots, 1.8 on average and more, groups * blocks in * blocks out below 2000
+@pytest.mark.parametrize("tokens,groups,n_ff,n_embd,down_quant", [
+    (16, [8, 1, 3, 5, 2] * 4, 256, 256, Q4_K),                # four waves, a row tile a workgroup; one block
+    (16, [8, 1, 3, 5, 2] * 4, 256, 256, Q5_K),
+    (16, [8, 1, 3, 5, 2] * 4, 256, 256, Q6_K),
+    (24, [2, 1, 2, 3, 8] * 20, 768, 1536, Q6_K),              # six waves, two row tiles a workgroup in both kernels
+    (16, [2, 2, 1, 4, 7] * 4 + [2, 1], 1536, 2048, Q5_K),     # four waves, two row tiles a workgroup
+    (20, [3, 1, 2] * 100, 256, 768, Q4_K),                    # more workgroups than units, no merging
+    (18, [1, 2, 3, 2] * 27, 256, 4352, Q6_K),                 # four row tiles a workgroup in the down kernel, two in its last
+    (18, [1, 2, 3, 2] * 27, 256, 4352, Q5_K),
+])
+def test_moe_small_groups(rnb, oracle, tokens, groups, n_ff, n_embd, down_quant):
+    _check(rnb, oracle, tokens, groups, n_ff, n_embd, False, down_quant)
