@@ -817,7 +817,7 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     const uint32_t *d_off = d + n_slots, *d_list = d_off + token_count + 1;
     const uint32_t *d_gstart = d_list + 3 * n_slots + n_groups, *d_units = d_gstart + n_groups + 1 + n_slots;
     const MoeGroups groups{d_list + 3 * n_slots, d_gstart, d_list + n_slots, d_list + 2 * n_slots, static_cast<uint32_t>(n_groups),
-                           max_group, grp_start.data(), d_units, static_cast<uint32_t>(units.size() / 3), unit_tokens};
+                           max_group, d_units, static_cast<uint32_t>(units.size() / 3), unit_tokens};
 
     ActView act;
     if (inline_tables) {
@@ -868,8 +868,8 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
         if (int ls = check_launches(); ls != RNB_HIP_OK) return ls;
         return RNB_HIP_OK;
     }
-    if (mfma && act.digits != nullptr) {
-        // prefill: grouped GEMMs on the matrix cores; the down kernel quantises the intermediate as it stages it
+    if (mfma && max_group <= kMoeMfmaMaxGroup && n_groups <= 65535 && act.digits != nullptr) {
+        // the down kernel quantises the intermediate as it stages it
         launch_moe_gate_up_mfma(gate_dev, up_dev, shared, act, groups, s.moe_mid.as<float>(), static_cast<uint32_t>(n_ff),
                                 static_cast<uint32_t>(sh.nb_in), s.stream);
         launch_moe_down_mfma(down_dev, shared, down_quant, s.moe_mid.as<float>(), groups, d_route, s.moe_slot_out.as<float>(),

@@ -194,16 +194,10 @@ struct MoeGroups {
     const uint32_t *sorted_slot;   // [n_slots]
     const uint32_t *sorted_token;  // [n_slots]
     uint32_t n_groups;
-    uint32_t max_group = 32;       // slots of the largest group (host-side knowledge: sizes the matrix-core kernels' LDS)
-    const uint32_t *host_start = nullptr;  // `start` in host memory, for the length of the call
+    uint32_t max_group = 0;  // slots of the largest group (sizes moe_mfma.hip's LDS)
     // the groups' slots in tiles of unit_tokens (device array): {expert, first sorted position, slots} each
     const uint32_t *units = nullptr;
     uint32_t n_units = 0, unit_tokens = 0;
-    uint32_t tiles_of(uint32_t slots) const {  // the groups' slots in tiles of `slots`
-        uint32_t n = 0;
-        for (uint32_t g = 0; g < n_groups; g++) n += (host_start[g + 1] - host_start[g] + slots - 1) / slots;
-        return n;
-    }
 };
 // Q8_K of act(gate[i]) * up[i] (SiLU, or the tanh form of GELU): the gated FFN's intermediate quantised as it is made; both are
 // the sums of `slices` parts `stride` floats apart, added in that order
@@ -234,9 +228,10 @@ void launch_moe_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const Mo
 bool moe_down_quantises(uint32_t nb_mid);  // whether that pays (short intermediates)
 void launch_moe_down(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act,
                      const float *mid_f32, MoeGroups groups, const float *slot_route, float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream);
-// the same two steps on the matrix cores for batches (act / mid_act carry digits, except a Q6_K down's mid_act):
-// 32-token tiles per expert group, see moe_mfma.hip
-bool moe_mfma_supported(uint32_t nb_in, uint32_t nb_mid, uint32_t down_quant);  // the tiles' LDS images fit
+// the same two steps on the matrix cores for small batches of groups of at most kMoeMfmaMaxGroup slots, up to 65535 of them (act
+// carries digits), see moe_mfma.hip
+constexpr size_t kMoeMfmaMaxGroup = 8;
+bool moe_mfma_supported(uint32_t nb_in, uint32_t nb_mid, uint32_t down_quant);  // the groups' LDS images fit
 void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act,
                              MoeGroups groups, float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);
 void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, const float *mid, MoeGroups groups,
@@ -244,7 +239,6 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
 // the same two steps on the few-token GEMM's tiles (moe_few.hip): groups with units of moe_few_tile slots, weights at 4-byte
 // addresses, both activations quantised with digits
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups);
-constexpr size_t kMoeMfmaMaxGroup = 8;
 bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid);
 bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant);
 void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,

@@ -166,7 +166,7 @@ uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 14 * 
 // slots and its down projection quantises the intermediates itself, one launch of 5 us less, which counts where the experts' weights
 // are read in 30 - 60 us; up to sixteen groups leave its one workgroup a unit idle.  Us a call, moe_mfma : this, Q5_K down projections:
 // 128 x top-8 of 256 x 2304 at 21 tokens 36.7 : 42.7, of 1024 x 1024 at 19 44.9 : 50.7; 512 x 3328 at 21 (2366 blocks) 92.7 : 76.1, 8 x top-2 of
-// 2048 x 1024, Q6_K, at 26 38.2 : 29.1.  780 random calls of 16 to 300 tokens (3 to 194 experts hit, rows of 3 to 18 blocks, intermediates of
+// 2048 x 1024, Q6_K, at 26 38.2 : 29.1.  780 random calls of 16 to 300 tokens (7 to 244 experts hit, rows of 3 to 18 blocks, intermediates of
 // 1 to 10): 0.25 % over the better one of the two on average, 19 of them 3 - 13 % behind moe_mfma.hip (mostly Q5_K with groups of 9 to 15).
 bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid) {
     return max_group > kMoeMfmaMaxGroup || n_groups <= 16 || n_groups * nb_in * nb_mid >= 2000;

@@ -1,13 +1,12 @@
-// Gathered sparse-MoE experts for batches (prefill) on the matrix cores: the grouped form of gemm_blocks.hip.
-// Slots are sorted by expert on the host (api.cpp) and every expert's group is cut into tiles of up to 32 tokens; workgroup
-// (row tiles, token tile of all groups): the tile's quantised activations are gathered into LDS by the sorted lists, the
-// expert's weight rows go from global memory to the registers of the lane that owns the row, one int8 matrix instruction
-// per scale group, the group's scale on the vector units (see gemm_blocks.hip).  With a handful of tokens per expert most of
-// a 32-token tile is padding, which costs no arithmetic: the work per tile is the same whatever the number of live tokens,
-// where the integer-dot kernels of moe.hip cost per token (measured crossover on 128 experts x top-8: 64 tokens).  Padding
+// Gathered sparse-MoE experts on the matrix cores, for small batches whose experts have at most eight slots each (larger ones:
+// moe_few.hip, moe_few_pays): the grouped form of gemm_blocks.hip.  Slots are sorted by expert on the host (api.cpp); workgroup
+// (row tiles, group): the group's quantised activations are gathered into LDS by the sorted lists, the expert's weight rows go
+// from global memory to the registers of the lane that owns the row, one int8 matrix instruction per scale group, the group's
+// scale on the vector units (see gemm_blocks.hip), which finish the results of eight tokens of the instruction's 32.  The work
+// per group is the same whatever the number of live tokens, where the integer-dot kernels of moe.hip cost per token.  Padding
 // costs no LDS either: only the live tokens are staged, the matrix instruction's padding lanes read the last live token's
 // row, and the launch sizes the image for the largest group of the call, so that several workgroups share a compute
-// unit when the groups are small.
+// unit.
 //   gate/up   mid[slot][n_ff] = silu(Wg[e] . a_tok) * (Wu[e] . a_tok), both Q4_K: the two matrices share the activation
 //             operand of every instruction                        fanout.rs:260-327, activation.rs:73-89
 //   down      slot_out[slot][n_embd] = route[slot] * (Wd[e] . Q8_K(mid[slot])), Q4_K, Q5_K or Q6_K; mid is quantised as the
@@ -17,14 +16,13 @@
 #include "device_utils.h"
 #include "kernels.h"
 #include "mfma_blocks.h"
-#include <algorithm>
-#include <type_traits>
 
 namespace rnb {
 
 namespace {
 
-constexpr int kMmToks = 32;  // tokens per tile
+constexpr int kMmToks = 32;     // tokens of a matrix instruction
+constexpr int kMmResults = 4;   // results of a lane that belong to the first eight of them, kMoeMfmaMaxGroup
 constexpr int kQ4FillInstr = (32 * kQ4Pieces + kWave - 1) / kWave;  // 5 wave-wide 16-byte loads per 32 rows of a Q4_K block
 constexpr int kQ4FillBytes = kQ4FillInstr * 1024;                   // what they write: 32 x 144 bytes of rows + the tail
 constexpr int kMmGateUpStripBytes = kGbWaves * 2 * kQ4FillBytes;    // gate and up strips of the four waves
@@ -45,33 +43,6 @@ __device__ __forceinline__ void tile_map_fill(TileMap &m, const uint32_t *__rest
         const uint32_t o = out_idx[p];
         m.out_row[tid] = live ? o : 0xffffffffu;
         m.scale[tid] = out_scale != nullptr ? out_scale[o] : 1.0f;
-    }
-}
-
-// Token tile `unit` of the call: the tiles of `toks` slots of group 0, then those of group 1, ...  A call whose groups are one
-// tile each (n_units == n_groups) skips the search; else every wave walks the groups 64 at a time, a group per lane.
-struct TileUnit {
-    uint32_t grp, first;  // group, first slot of the tile in it
-};
-__device__ __forceinline__ TileUnit find_unit(uint32_t unit, uint32_t n_units, const uint32_t *__restrict__ grp_start, uint32_t n_groups,
-                                              uint32_t toks, int lane) {
-    if (n_units == n_groups) return {unit, 0};
-    for (uint32_t g0 = 0;; g0 += kWave) {
-        const uint32_t g = min(g0 + lane, n_groups - 1);
-        const uint32_t mine = g0 + lane < n_groups ? (grp_start[g + 1] - grp_start[g] + toks - 1) / toks : 0;
-        uint32_t end = mine;  // tiles up to and with the lane's group
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const uint32_t below = __shfl_up(end, off, kWave);
-            if (lane >= off) end += below;
-        }
-        const uint64_t past = __ballot(end > unit);
-        if (past != 0) {
-            const int at = __builtin_ctzll(past);
-            return {g0 + at, (unit - __shfl(end - mine, at, kWave)) * toks};
-        }
-        unit -= __shfl(end, kWave - 1, kWave);
-        if (g0 + kWave >= n_groups) return {n_groups - 1, 0xffffffffu};  // not reached: the launches have n_units rows
     }
 }
 
@@ -120,9 +91,9 @@ __device__ __forceinline__ void tile_stage_store(const TileStage<kThreads> &st, 
 
 // One super-block of one 32-token tile against one Q4_K / Q5_K row share: I = sum_sb sc * (codes . a) and the mins sum
 // S = sum_sb mn * bsum32 (through the digits); returns d * I - dmin * S per result in `val`.
-// kJ = 1, 2 or 4: only the results of the tile's first 8 kJ tokens are finished on the vector units (result r of a lane
-// is token 8 * (r / 4) + 4 * khalf + r % 4, so they are the lane's first 4 kJ results); the matrix instructions always
-// compute all 32 tokens, which costs nothing extra.
+// Only the results of the tile's first eight tokens are finished on the vector units (result r of a lane is token
+// 8 * (r / 4) + 4 * khalf + r % 4, so they are the lane's first four); the matrix instructions always compute all 32
+// tokens, which costs nothing extra.
 // The matrix instruction of sub-block SB is issued before the results of sub-block SB - 1 are scaled: a wave that has
 // its SIMD to itself would otherwise sit out the instruction's latency (16 passes) eight times per block.
 #define RNB_Q45_ISSUE(SB, ROW, ACC, SC)                                                                  \
@@ -135,7 +106,7 @@ __device__ __forceinline__ void tile_stage_store(const TileStage<kThreads> &st, 
     }
 #define RNB_Q45_TAKE(ACC, SC, TOT)                                                                       \
     {                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < 4 * kJ; i++) {                                             \
+        _Pragma("unroll") for (int i = 0; i < kMmResults; i++) {                                             \
             TOT[i] += mul24(ACC[i], SC);                                                                 \
             asm volatile("" : "+v"(TOT[i])); /* keep the eight additions a chain, not a tree */          \
         }                                                                                                \
@@ -171,57 +142,27 @@ __device__ __forceinline__ void tile_ops_load(TileOps64 &o, const uint8_t *abase
     for (int sb = 0; sb < 16; sb++) o.v[sb] = *reinterpret_cast<const long *>(abase + 16 * sb);
 }
 
-template <bool kFifth, int kJ>
+template <bool kFifth>
 __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps128 &aops, const uint4 dig, int khalf,
-                                               float (&val)[4 * kJ]) {
+                                               float (&val)[kMmResults]) {
     const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const Q4KScales sc8 = unpack_q4k_scales(row.hdr.y, row.hdr.z, row.hdr.w);
-    int tot[4 * kJ];
-    // With at most 16 live tokens the scale costs 4 kJ <= 8 multiply-adds per sub-block on the results: fewer vector
-    // instructions than folding it into the operand (8 per sub-block and a second matrix instruction), which pays for
-    // whole tiles only.
-    if constexpr (kFifth || kJ < 4) {
+    // the scale on the results: four multiply-adds per sub-block, where folding it into the operand would take eight and a second
+    // matrix instruction
+    int tot[kMmResults];
 #pragma unroll
-        for (int i = 0; i < 4 * kJ; i++) tot[i] = 0;
-        v16i acc_a, acc_b;
-        int sc_a, sc_b;
-        RNB_Q45_SUB_BLOCK(0, row, tot)
-        RNB_Q45_SUB_BLOCK(1, row, tot)
-        RNB_Q45_SUB_BLOCK(2, row, tot)
-        RNB_Q45_SUB_BLOCK(3, row, tot)
-        RNB_Q45_SUB_BLOCK(4, row, tot)
-        RNB_Q45_SUB_BLOCK(5, row, tot)
-        RNB_Q45_SUB_BLOCK(6, row, tot)
-        RNB_Q45_SUB_BLOCK(7, row, tot)
-        RNB_Q45_TAKE(acc_b, sc_b, tot)
-    } else {
-        // Q4_K: the scale folded into the operand (sc = lo + 8 * hi, two accumulator chains), as in gemm_blocks.hip
-        const uint32_t dlo[2] = {sc8.sc_lo & 0x07070707u, sc8.sc_hi & 0x07070707u};
-        const uint32_t dhi[2] = {(sc8.sc_lo >> 3) & 0x07070707u, (sc8.sc_hi >> 3) & 0x07070707u};
-        v16i acc_lo = zero16, acc_hi = zero16;
-#define RNB_Q4_FOLD_SUB_BLOCK(SB)                                                                        \
-    {                                                                                                    \
-        const v4i nib = q45_operand<SB, false>(row);                                                     \
-        constexpr uint32_t sel = 0x0c000c00u | (((SB) & 3) << 16) | ((SB) & 3);                          \
-        const uint32_t slo = __builtin_amdgcn_perm(0u, dlo[(SB) >> 2], sel);                             \
-        const uint32_t shi = __builtin_amdgcn_perm(0u, dhi[(SB) >> 2], sel);                             \
-        const v4i wlo = {pk_scale(nib[0], slo), pk_scale(nib[1], slo), pk_scale(nib[2], slo), pk_scale(nib[3], slo)}; \
-        const v4i whi = {pk_scale(nib[0], shi), pk_scale(nib[1], shi), pk_scale(nib[2], shi), pk_scale(nib[3], shi)}; \
-        acc_lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(aops.v[SB], wlo, acc_lo, 0, 0, 0);                \
-        acc_hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(aops.v[SB], whi, acc_hi, 0, 0, 0);                \
-    }
-        RNB_Q4_FOLD_SUB_BLOCK(0)
-        RNB_Q4_FOLD_SUB_BLOCK(1)
-        RNB_Q4_FOLD_SUB_BLOCK(2)
-        RNB_Q4_FOLD_SUB_BLOCK(3)
-        RNB_Q4_FOLD_SUB_BLOCK(4)
-        RNB_Q4_FOLD_SUB_BLOCK(5)
-        RNB_Q4_FOLD_SUB_BLOCK(6)
-        RNB_Q4_FOLD_SUB_BLOCK(7)
-#undef RNB_Q4_FOLD_SUB_BLOCK
-#pragma unroll
-        for (int i = 0; i < 4 * kJ; i++) tot[i] = acc_lo[i] + 8 * acc_hi[i];
-    }
+    for (int i = 0; i < kMmResults; i++) tot[i] = 0;
+    v16i acc_a, acc_b;
+    int sc_a, sc_b;
+    RNB_Q45_SUB_BLOCK(0, row, tot)
+    RNB_Q45_SUB_BLOCK(1, row, tot)
+    RNB_Q45_SUB_BLOCK(2, row, tot)
+    RNB_Q45_SUB_BLOCK(3, row, tot)
+    RNB_Q45_SUB_BLOCK(4, row, tot)
+    RNB_Q45_SUB_BLOCK(5, row, tot)
+    RNB_Q45_SUB_BLOCK(6, row, tot)
+    RNB_Q45_SUB_BLOCK(7, row, tot)
+    RNB_Q45_TAKE(acc_b, sc_b, tot)
     const float d = f16_bits_to_f32(row.hdr.x), dmin = f16_bits_to_f32(row.hdr.x >> 16);
     // K slots 0..7 of the lower K-half carry the eight mins (weights) and the eight digits (tokens)
     const long mnop = khalf == 0 ? static_cast<long>(static_cast<unsigned long>(sc8.mn_lo) | (static_cast<unsigned long>(sc8.mn_hi) << 32)) : 0L;
@@ -230,7 +171,7 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
     const v16i c0 = __builtin_amdgcn_mfma_i32_32x32x16_i8(op0, mnop, zero16, 0, 0, 0);
     const v16i c1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(op1, mnop, zero16, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4 * kJ; i++) val[i] = d * static_cast<float>(tot[i]) - dmin * static_cast<float>(c0[i] + 64 * c1[i]);
+    for (int i = 0; i < kMmResults; i++) val[i] = d * static_cast<float>(tot[i]) - dmin * static_cast<float>(c0[i] + 64 * c1[i]);
 }
 #undef RNB_Q45_SUB_BLOCK
 #undef RNB_Q45_TAKE
@@ -247,7 +188,7 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
     }
 #define RNB_Q6_TILE_TAKE(ACC, SC)                                                                        \
     {                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < 4 * kJ; i++) {                                             \
+        _Pragma("unroll") for (int i = 0; i < kMmResults; i++) {                                             \
             tot[i] += mul24(ACC[i], SC);                                                                 \
             asm volatile("" : "+v"(tot[i]));                                                             \
         }                                                                                                \
@@ -265,12 +206,11 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
             RNB_Q6_TILE_TAKE(acc_a, sc_a)                                                                \
         }                                                                                                \
     }
-template <int kJ>
-__device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 &aops, float (&val)[4 * kJ]) {
+__device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 &aops, float (&val)[kMmResults]) {
     const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int tot[4 * kJ];
+    int tot[kMmResults];
 #pragma unroll
-    for (int i = 0; i < 4 * kJ; i++) tot[i] = 0;
+    for (int i = 0; i < kMmResults; i++) tot[i] = 0;
     v16i acc_a, acc_b;
     int sc_a, sc_b;
     RNB_Q6_TILE_SUB_BLOCK(0)
@@ -291,31 +231,27 @@ __device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 
     RNB_Q6_TILE_SUB_BLOCK(15)
     RNB_Q6_TILE_TAKE(acc_b, sc_b)
 #pragma unroll
-    for (int i = 0; i < 4 * kJ; i++) val[i] = row.d * static_cast<float>(tot[i]);
+    for (int i = 0; i < kMmResults; i++) val[i] = row.d * static_cast<float>(tot[i]);
 }
 #undef RNB_Q6_TILE_SUB_BLOCK
 #undef RNB_Q6_TILE_TAKE
 #undef RNB_Q6_TILE_ISSUE
 
-// accf[r] += d_x[token of result r] * val[r]; result r of a tile is token 8 * (r / 4) + 4 * khalf + r % 4
-template <int kJ>
-__device__ __forceinline__ void tile_scale_add(const float *dxbuf, int khalf, const float (&val)[4 * kJ], float (&accf)[4 * kJ]) {
+// accf[r] += d_x[token of result r] * val[r]; result r of a tile is token 4 * khalf + r
+__device__ __forceinline__ void tile_scale_add(const float *dxbuf, int khalf, const float (&val)[kMmResults], float (&accf)[kMmResults]) {
+    const float4 dx4 = reinterpret_cast<const float4 *>(dxbuf)[khalf];
+    const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
 #pragma unroll
-    for (int j = 0; j < kJ; j++) {
-        const float4 dx4 = reinterpret_cast<const float4 *>(dxbuf)[2 * j + khalf];
-        const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) accf[4 * j + i] += dx[i] * val[4 * j + i];
-    }
+    for (int i = 0; i < kMmResults; i++) accf[i] += dx[i] * val[i];
 }
 
 // LDS image of one tile: every 256-element block of the tile's live tokens, staged once and then only read
 //   act[nb][toks][kStride] | d_x[nb][32] | digits[nb][32] (16 bytes each; absent for Q6_K weights)
-// toks <= 32 is the number of token rows the launch made room for (the largest group of the call, capped at a tile)
+// toks <= 8 is the number of token rows the launch made room for (the largest group of the call)
 template <int kStride, bool kDigits>
 struct TileImage {
     static __host__ __device__ size_t act_bytes(uint32_t nb, uint32_t toks) { return static_cast<size_t>(nb) * toks * kStride; }
-    static __host__ __device__ size_t bytes(uint32_t nb, uint32_t toks = kMmToks) {
+    static __host__ __device__ size_t bytes(uint32_t nb, uint32_t toks) {
         return act_bytes(nb, toks) + static_cast<size_t>(nb) * kMmToks * (4 + (kDigits ? 16 : 0));
     }
     uint8_t *base;
@@ -343,25 +279,20 @@ __device__ __forceinline__ void tile_image_fill(const TileImage<kStride, kDigits
 }
 
 // ---------------------------------------------------------------------------------------------
-// gate + up + SiLU * up.  Grid (row tiles of 32 kW, token tiles of all groups, see find_unit).  A router's groups differ
-// severalfold in size: with one workgroup walking all token tiles of its group the largest group set the time (128 experts x
-// top-8 at 512 tokens, groups of 2 to 172: gate/up 282 -> 92 us, down 218 -> 94; a grid with empty workgroups for the tiles
-// that smaller groups have not: 153; 8 experts x top-2 at 300 tokens, the whole call: 917 -> 190).
+// gate + up + SiLU * up.  Grid (row tiles of 32 kW, groups).
 // The tile's activations are staged once, all blocks; after that the waves run without barriers, each streaming its 32 rows
 // of both matrices one block ahead.  The rows come in by whole cache lines as LDS-direct loads into the wave's two strips
 // (consecutive lanes take consecutive 16-byte pieces of a row, see RowRoute for why; no vector registers hold the data in
 // flight), and each lane reads its row's share back from there.  Dynamic LDS: the waves' strips, then the tile image.
 // ---------------------------------------------------------------------------------------------
-template <int kJ, int kW>
+template <int kW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * kW), amdgpu_waves_per_eu(2)))
     moe_gate_up_mfma_kernel(const uint8_t *__restrict__ gate_all, const uint8_t *__restrict__ up_all,
                             const uint8_t *__restrict__ gate_shared, const uint8_t *__restrict__ up_shared, uint32_t n_routed,
                             const int8_t *__restrict__ aq, const float *__restrict__ ad, const uint8_t *__restrict__ adig,
-                            const uint32_t *__restrict__ grp_expert, const uint32_t *__restrict__ grp_start, uint32_t n_groups,
+                            const uint32_t *__restrict__ grp_expert, const uint32_t *__restrict__ grp_start,
                             const uint32_t *__restrict__ sorted_slot, const uint32_t *__restrict__ sorted_token,
-                            float *__restrict__ mid, uint32_t n_ff, uint32_t nb, uint32_t img_toks, uint32_t tiles_per_wg,
-                            uint32_t unit0, uint32_t n_units) {
-    constexpr bool kFifth = false;
+                            float *__restrict__ mid, uint32_t n_ff, uint32_t nb, uint32_t img_toks, uint32_t tiles_per_wg) {
     constexpr int kPair = 2 * kQ4FillBytes;  // a gate strip and an up strip
     extern __shared__ __attribute__((aligned(16))) uint8_t s_dyn[];
     __shared__ TileMap s_map;
@@ -372,10 +303,8 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
     const int lrow = lane & 31, khalf = lane >> 5;
     uint8_t *strips = s_dyn + wave * kPair;
     const uint32_t lds_strips = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)strips));
-    const TileUnit unit = find_unit(unit0 + blockIdx.y, n_units, grp_start, n_groups, img_toks, lane);
-    const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
-    const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
-    if (tile0 >= count) return;
+    const uint32_t grp = blockIdx.y, expert = grp_expert[grp], start = grp_start[grp];
+    const uint32_t live = grp_start[grp + 1] - start;  // 1 .. img_toks
     const uint32_t row_bytes = nb * static_cast<uint32_t>(kQ4KBytes);
     const size_t per_expert = static_cast<size_t>(n_ff) * row_bytes;
     const uint8_t *gate_e = expert_base(gate_all, gate_shared, n_routed, expert, per_expert),
@@ -432,66 +361,50 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
     // the first weight blocks do not depend on the token lists: requested before them
     set_tile(0);
     request();
-    const uint32_t live = min(count - tile0, img_toks);
     const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);  // padding lanes read the last live row
-    tile_map_fill(s_map, sorted_token, sorted_slot, nullptr, start + tile0, live, tid);
+    tile_map_fill(s_map, sorted_token, sorted_slot, nullptr, start, live, tid);
     __syncthreads();
     tile_image_fill<kWave * kW>(img, s_map, aq, ad, adig, tid, live);
     Q5Row cg, cu;
     take(cg, cu);
     __syncthreads();
-    // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
-    auto walk = [&](auto jtag) {
-        constexpr int kJl = decltype(jtag)::value;
-        for (uint32_t rt = 0; rt < rt_n; rt++) {
-            const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
-            float accg[4 * kJl], accu[4 * kJl];
+    for (uint32_t rt = 0; rt < rt_n; rt++) {
+        const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
+        float accg[kMmResults] = {}, accu[kMmResults] = {};
+        for (uint32_t b = 0; b < nb; b++) {
+            request();  // the step after this one
+            const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
+            const uint4 dig = img.dig(b)[lrow];
+            float val[kMmResults];
+            TileOps128 aops;
+            tile_ops_load(aops, abase);
+            q45_block_tile<false>(cg, aops, dig, khalf, val);
+            tile_scale_add(img.dx(b), khalf, val, accg);
+            q45_block_tile<false>(cu, aops, dig, khalf, val);
+            tile_scale_add(img.dx(b), khalf, val, accu);
+            take(cg, cu);  // (after the last step: a repeat of it, unused)
+        }
+        if (row < n_ff) {
 #pragma unroll
-            for (int i = 0; i < 4 * kJl; i++) accg[i] = accu[i] = 0.0f;
-            for (uint32_t b = 0; b < nb; b++) {
-                request();  // the step after this one
-                const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
-                const uint4 dig = img.dig(b)[lrow];
-                float val[4 * kJl];
-                TileOps128 aops;
-                tile_ops_load(aops, abase);
-                q45_block_tile<kFifth, kJl>(cg, aops, dig, khalf, val);
-                tile_scale_add<kJl>(img.dx(b), khalf, val, accg);
-                q45_block_tile<kFifth, kJl>(cu, aops, dig, khalf, val);
-                tile_scale_add<kJl>(img.dx(b), khalf, val, accu);
-                take(cg, cu);  // (after the last step: a repeat of it, unused)
-            }
-            if (row < n_ff) {
-#pragma unroll
-                for (int r = 0; r < 4 * kJl; r++) {
-                    const uint32_t slot = s_map.out_row[8 * (r >> 2) + 4 * khalf + (r & 3)];
-                    if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
-                }
+            for (int r = 0; r < kMmResults; r++) {
+                const uint32_t slot = s_map.out_row[4 * khalf + r];
+                if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
             }
         }
-    };
-    if constexpr (kJ == 2) {  // (the 32-token kernel keeps its one form: its groups are large)
-        if (live <= 8)  // workgroup-uniform
-            walk(std::integral_constant<int, 1>{});
-        else
-            walk(std::integral_constant<int, 2>{});
-    } else {
-        walk(std::integral_constant<int, kJ>{});
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// down projection of the re-quantised intermediate, scaled by the route weight.  Grid (row tiles of 128, token tiles of all
-// groups).
+// down projection of the re-quantised intermediate, scaled by the route weight.  Grid (row tiles of 128, groups).
 // ---------------------------------------------------------------------------------------------
-template <uint32_t kQuant, int kJ>
+template <uint32_t kQuant>
 __global__ void __launch_bounds__(kGbThreads, 2)
     moe_down_mfma_kernel(const uint8_t *__restrict__ down_all, const uint8_t *__restrict__ down_shared, uint32_t n_routed,
                          const float *__restrict__ mid,
                          const uint32_t *__restrict__ grp_expert,
-                         const uint32_t *__restrict__ grp_start, uint32_t n_groups, const uint32_t *__restrict__ sorted_slot,
+                         const uint32_t *__restrict__ grp_start, const uint32_t *__restrict__ sorted_slot,
                          const float *__restrict__ slot_route, float *__restrict__ slot_out, uint32_t n_embd, uint32_t nb,
-                         uint32_t tiles_per_wg, uint32_t img_toks, uint32_t unit0, uint32_t n_units) {
+                         uint32_t tiles_per_wg, uint32_t img_toks) {
     constexpr bool kSix = kQuant == kQ6K;
     constexpr bool kFifth = kQuant == kQ5K;
     constexpr int kStride = kSix ? kGbStride64 : kGbStride128;
@@ -503,10 +416,8 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: the wave's row addresses are scalar bases plus lane offsets
     const int lrow = lane & 31, khalf = lane >> 5;
-    const TileUnit unit = find_unit(unit0 + blockIdx.y, n_units, grp_start, n_groups, img_toks, lane);
-    const uint32_t grp = __builtin_amdgcn_readfirstlane(unit.grp), tile0 = __builtin_amdgcn_readfirstlane(unit.first);
-    const uint32_t expert = grp_expert[grp], start = grp_start[grp], count = grp_start[grp + 1] - start;
-    if (tile0 >= count) return;
+    const uint32_t grp = blockIdx.y, expert = grp_expert[grp], start = grp_start[grp];
+    const uint32_t live = grp_start[grp + 1] - start;  // 1 .. img_toks
     const size_t row_bytes = static_cast<size_t>(nb) * kBlockBytes;
     const uint8_t *down_e = expert_base(down_all, down_shared, n_routed, expert, n_embd * row_bytes);
     // The workgroup walks tiles_per_wg row tiles of 128 against one staged token tile: map and image are made once,
@@ -547,9 +458,8 @@ __global__ void __launch_bounds__(kGbThreads, 2)
         q6_request(0, 0);
     else
         c5 = q45_load_row<kFifth>(block_ptr(0, 0), khalf);
-    const uint32_t live = min(count - tile0, img_toks);
     const uint32_t arow = min(static_cast<uint32_t>(lrow), live - 1);
-    tile_map_fill(s_map, sorted_slot, sorted_slot, slot_route, start + tile0, live, tid);
+    tile_map_fill(s_map, sorted_slot, sorted_slot, slot_route, start, live, tid);
     __syncthreads();
     // the tile's slots' intermediates (f32, [slot][nb * 256]) are quantised to Q8_K as they are staged, with the
     // stand-alone quantiser's wave-level routine (the same bits): wave w takes (token, block) pairs w, w + 4, ...,
@@ -580,12 +490,7 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     }
     if constexpr (kSix) q6_take(c6);
     __syncthreads();
-    // a tile of at most eight live tokens (most groups of a routed batch) finishes only a lane's first four results
-    auto walk = [&](auto jtag) {
-    constexpr int kJl = decltype(jtag)::value;
-    float accf[4 * kJl];
-#pragma unroll
-    for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
+    float accf[kMmResults] = {};
     uint32_t rt = 0, b = 0;
     for (uint32_t s = 0; s < steps; s++) {
         uint32_t rtn = rt, bn = b + 1;  // the step after this one; the last step reloads its own block, unused
@@ -598,27 +503,27 @@ __global__ void __launch_bounds__(kGbThreads, 2)
             bn = b;
         }
         Q5Row n5{};
-        float val[4 * kJl];
+        float val[kMmResults];
         if constexpr (kSix) {
             q6_request(rtn, bn);
             TileOps64 aops;
             tile_ops_load(aops, img.act(b) + arow * kStride + 8 * khalf);
-            q6_block_tile<kJl>(c6, aops, val);
+            q6_block_tile(c6, aops, val);
         } else {
             n5 = q45_load_row<kFifth>(block_ptr(rtn, bn), khalf);
             TileOps128 aops;
             tile_ops_load(aops, img.act(b) + arow * kStride + 16 * khalf);
-            q45_block_tile<kFifth, kJl>(c5, aops, img.dig(b)[lrow], khalf, val);
+            q45_block_tile<kFifth>(c5, aops, img.dig(b)[lrow], khalf, val);
         }
-        tile_scale_add<kJl>(img.dx(b), khalf, val, accf);
+        tile_scale_add(img.dx(b), khalf, val, accf);
         if constexpr (kSix) q6_take(c6);
         c5 = n5;
         if (b + 1 == nb) {  // the row tile is complete
             const uint32_t row = row_of(rt);
             if (row < n_embd) {
 #pragma unroll
-                for (int r = 0; r < 4 * kJl; r++) {
-                    const int t = 8 * (r >> 2) + 4 * khalf + (r & 3);
+                for (int r = 0; r < kMmResults; r++) {
+                    const int t = 4 * khalf + r;
                     const uint32_t slot = s_map.out_row[t];
                     // fanout.rs:306-308: the expert's output times the slot's route weight
                     if (slot != 0xffffffffu)
@@ -626,19 +531,10 @@ __global__ void __launch_bounds__(kGbThreads, 2)
                 }
             }
 #pragma unroll
-            for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
+            for (int i = 0; i < kMmResults; i++) accf[i] = 0.0f;
         }
         rt = rtn;
         b = bn;
-    }
-    };
-    if constexpr (kJ == 2) {
-        if (live <= 8)  // workgroup-uniform
-            walk(std::integral_constant<int, 1>{});
-        else
-            walk(std::integral_constant<int, 2>{});
-    } else {
-        walk(std::integral_constant<int, kJ>{});
     }
 }
 
@@ -653,35 +549,22 @@ bool allow_lds(K kernel, size_t bytes) {
 }  // namespace
 
 // the tile image (all blocks of the tile's tokens) must fit the LDS of a compute unit beside the waves' strips and the
-// small static arrays; a tile holds as many tokens as fit, at most 32
+// small static arrays
 constexpr size_t kMmLdsLimit = 150 * 1024;
-constexpr size_t kMmLdsWide = 158 * 1024;  // for the eight-wave gate/up kernel (the token map is all it has besides)
 constexpr size_t kMmGateUpImageLimit = kMmLdsLimit - kMmGateUpStripBytes;
 constexpr size_t kMmQ6DownLdsLimit = kMmLdsLimit - kGbWaves * 32 * kQ6StripStride;
-constexpr uint32_t kMaxGridY = 65535;  // token tiles per launch: grid rows that a device is sure to take
-constexpr uint32_t kMmMinToks = 16;  // below this the matrix-core path re-reads the weights too often to pay
-
-template <int kStride, bool kDigits>
-static uint32_t tile_tokens_that_fit(size_t limit, uint32_t nb) {
-    uint32_t toks = kMmToks;
-    while (toks > 0 && TileImage<kStride, kDigits>::bytes(nb, toks) > limit) toks--;
-    return toks;
-}
-static uint32_t gate_up_tile_tokens(uint32_t nb_in) { return tile_tokens_that_fit<kGbStride128, true>(kMmGateUpImageLimit, nb_in); }
-static uint32_t down_tile_tokens(uint32_t nb_mid, uint32_t down_quant) {
-    return down_quant == kQ6K ? tile_tokens_that_fit<kGbStride64, false>(kMmQ6DownLdsLimit, nb_mid)
-                              : tile_tokens_that_fit<kGbStride128, true>(kMmLdsLimit, nb_mid);
-}
+constexpr uint32_t kMmMinToks = 16;  // rows so long that fewer tokens fit are no batch for this kernel
 
 bool moe_mfma_supported(uint32_t nb_in, uint32_t nb_mid, uint32_t down_quant) {
-    return nb_in >= 1 && nb_mid >= 1 && gate_up_tile_tokens(nb_in) >= kMmMinToks && down_tile_tokens(nb_mid, down_quant) >= kMmMinToks;
+    return nb_in >= 1 && nb_mid >= 1 && TileImage<kGbStride128, true>::bytes(nb_in, kMmMinToks) <= kMmGateUpImageLimit &&
+           (down_quant == kQ6K ? TileImage<kGbStride64, false>::bytes(nb_mid, kMmMinToks) <= kMmQ6DownLdsLimit
+                               : TileImage<kGbStride128, true>::bytes(nb_mid, kMmMinToks) <= kMmLdsLimit);
 }
 
 void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act,
                              MoeGroups groups, float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream) {
     if (groups.n_groups == 0 || n_ff == 0) return;
-    const uint32_t toks = std::min<uint32_t>(std::max<uint32_t>(groups.max_group, 1), gate_up_tile_tokens(nb_in));
-    if (toks == 0) return;  // moe_mfma_supported said no
+    const uint32_t toks = groups.max_group;
     const size_t image = TileImage<kGbStride128, true>::bytes(nb_in, toks);
     // A wave's time is its chain of steps, and the chain is mostly instruction and LDS latency that only another wave on
     // the SIMD hides (without its fills the kernel still takes 40 of its 50 us); a grid of more workgroups than fit at once
@@ -690,29 +573,10 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     // one workgroup per compute unit, map and image made once per walk.  128 experts x top-8 at 64 tokens (126 groups):
     // four waves 1 / 2 / 3 tiles per workgroup 55.4 / 58.4 / 50.6 us (2 leaves half the units with two workgroups and
     // half with one), six waves x 2 tiles 48.8 us, eight waves x 1 (two rounds) 61.6, twelve waves 67-74.
-    const uint32_t units = groups.tiles_of(toks);
     int waves = kGbWaves;
     uint32_t tiles_per_wg = 1;
-    const bool many = units > groups.n_groups;  // groups of more than a tile
-    if (many) {
-        // Whole tiles: the image and a strip pair per wave leave one workgroup per compute unit; eight waves (two per SIMD)
-        // where they fit.  Row tiles are merged for the least of rounds * (steps + about two for the setup); a step of eight
-        // waves takes a little longer than one of four.  (Four waves at 512 tokens 220 us a call against 198; with one tile a
-        // group the rule below is ahead, 64 tokens 114 against 120.)
-        uint64_t best = ~0ull;
-        for (const int w : {8, 4}) {
-            if (w == 8 && (toks <= 16 || 8 * 2 * kQ4FillBytes + image > kMmLdsWide)) continue;  // no such kernel below 17 tokens
-            const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
-            for (uint32_t t = 1; t <= tiles && t <= 8; t++) {
-                const uint64_t wgs = static_cast<uint64_t>(units) * ((tiles + t - 1) / t);
-                const uint64_t cost = (wgs + 255) / 256 * (t * nb_in + 2) * (w == 8 ? 9 : 8);
-                if (cost < best) best = cost, waves = w, tiles_per_wg = t;
-            }
-        }
-    }
     for (const int w : {6, 4}) {
-        if (many) break;
-        if (w != kGbWaves && (toks > 16 || static_cast<size_t>(w) * 2 * kQ4FillBytes + image > kMmLdsLimit)) continue;
+        if (w != kGbWaves && static_cast<size_t>(w) * 2 * kQ4FillBytes + image > kMmLdsLimit) continue;
         const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
         const uint32_t t = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * groups.n_groups + 255) / 256);
         if (t >= 1 && t <= 3 && t <= tiles && static_cast<uint64_t>((tiles + t - 1) / t) * groups.n_groups <= 256 &&
@@ -725,28 +589,16 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     const size_t lds = static_cast<size_t>(waves) * 2 * kQ4FillBytes + image;
     const uint32_t rows_per_wg = 32 * waves, row_tiles = (n_ff + rows_per_wg - 1) / rows_per_wg;
     const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
-    // tiles of at most 8 / 16 / 32 tokens: the kernel finishes only that many results per lane
-#define RNB_LAUNCH_GUW(J, W)                                                                                          \
-    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, W == 8 ? kMmLdsWide : kMmLdsLimit)) return;             \
-    for (uint32_t u = 0; u < units; u += kMaxGridY)                                                                   \
-    hipLaunchKernelGGL((moe_gate_up_mfma_kernel<J, W>), dim3(wgs_x, std::min(units - u, kMaxGridY), 1), dim3(kWave * W), lds, \
-                       stream, gate_all, up_all, shared.gate, shared.up, shared.n_routed, act.qs, act.d, act.digits,  \
-                       groups.expert, groups.start, groups.n_groups, groups.sorted_slot, groups.sorted_token, mid,    \
-                       n_ff, nb_in, toks, tiles_per_wg, u, units)
-    if (toks > 16 && waves == 8) {
-        RNB_LAUNCH_GUW(4, 8);
-    } else if (toks > 16) {
-        RNB_LAUNCH_GUW(4, kGbWaves);
-    } else if (waves == 6) {
-        if (toks <= 8) {
-            RNB_LAUNCH_GUW(1, 6);
-        } else {
-            RNB_LAUNCH_GUW(2, 6);
-        }
-    } else if (toks <= 8) {
-        RNB_LAUNCH_GUW(1, kGbWaves);
+#define RNB_LAUNCH_GUW(W)                                                                                            \
+    if (!allow_lds<W>(moe_gate_up_mfma_kernel<W>, kMmLdsLimit)) return;                                              \
+    hipLaunchKernelGGL(moe_gate_up_mfma_kernel<W>, dim3(wgs_x, groups.n_groups), dim3(kWave * W), lds, stream,       \
+                       gate_all, up_all, shared.gate, shared.up, shared.n_routed, act.qs, act.d, act.digits,         \
+                       groups.expert, groups.start, groups.sorted_slot, groups.sorted_token, mid, n_ff, nb_in, toks, \
+                       tiles_per_wg)
+    if (waves == 6) {
+        RNB_LAUNCH_GUW(6);
     } else {
-        RNB_LAUNCH_GUW(2, kGbWaves);
+        RNB_LAUNCH_GUW(kGbWaves);
     }
 #undef RNB_LAUNCH_GUW
 }
@@ -757,38 +609,17 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
     // A workgroup's setup (group, map, image: a chain of dependent loads) costs more than a row tile's few blocks, and
     // about three workgroups fit a compute unit: row tiles are merged (up to 4 per workgroup) until the grid fits them at
     // once (cfg5's shape, 16 row tiles x 126 groups, 64 tokens: 1 / 2 / 4 / 8 tiles per workgroup 72 / 62 / 59 / 62 us)
-    // With groups of more than a tile, whose workgroups fit a compute unit in twos: the least of rounds * (steps + about six for the setup, in which
-    // the tile's intermediates are quantised).
     const uint32_t row_tiles = (n_embd + kGbRows - 1) / kGbRows;
-    const uint32_t toks = std::min<uint32_t>(std::max<uint32_t>(groups.max_group, 1), down_tile_tokens(nb_mid, down_quant));
-    if (toks == 0) return;
-    const uint32_t units = groups.tiles_of(toks);
+    const uint32_t toks = groups.max_group;
     uint32_t tiles_per_wg = 1;
-    if (units > groups.n_groups) {
-        uint64_t best = ~0ull;
-        for (uint32_t t = 1; t <= row_tiles && t <= 16; t++) {
-            const uint64_t cost = (static_cast<uint64_t>(units) * ((row_tiles + t - 1) / t) + 511) / 512 * (t * nb_mid + 6);
-            if (cost < best) best = cost, tiles_per_wg = t;
-        }
-    } else {
-        while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
-            tiles_per_wg *= 2;
-    }
+    while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
+        tiles_per_wg *= 2;
     const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
-#define RNB_LAUNCH_DMJ(Q, J, LDS)                                                                                     \
-    if (!allow_lds<static_cast<int>(Q) * 8 + J>(moe_down_mfma_kernel<Q, J>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
-    for (uint32_t u = 0; u < units; u += kMaxGridY)                                                                   \
-    hipLaunchKernelGGL((moe_down_mfma_kernel<Q, J>), dim3(wgs_x, std::min(units - u, kMaxGridY), 1), dim3(kGbThreads), LDS, \
-                       stream, down_all, shared.down, shared.n_routed, mid, groups.expert, groups.start, groups.n_groups, \
-                       groups.sorted_slot, slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks, u, units)
-#define RNB_LAUNCH_DM(Q, LDS)                                                                                         \
-    if (toks <= 8) {                                                                                                  \
-        RNB_LAUNCH_DMJ(Q, 1, LDS);                                                                                    \
-    } else if (toks <= 16) {                                                                                          \
-        RNB_LAUNCH_DMJ(Q, 2, LDS);                                                                                    \
-    } else {                                                                                                          \
-        RNB_LAUNCH_DMJ(Q, 4, LDS);                                                                                    \
-    }
+#define RNB_LAUNCH_DM(Q, LDS)                                                                                        \
+    if (!allow_lds<static_cast<int>(Q)>(moe_down_mfma_kernel<Q>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
+    hipLaunchKernelGGL(moe_down_mfma_kernel<Q>, dim3(wgs_x, groups.n_groups), dim3(kGbThreads), LDS, stream,          \
+                       down_all, shared.down, shared.n_routed, mid, groups.expert, groups.start, groups.sorted_slot, \
+                       slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks)
     if (down_quant == kQ6K) {
         RNB_LAUNCH_DM(kQ6K, (TileImage<kGbStride64, false>::bytes(nb_mid, toks)));
     } else if (down_quant == kQ5K) {
@@ -797,7 +628,6 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
         RNB_LAUNCH_DM(kQ4K, (TileImage<kGbStride128, true>::bytes(nb_mid, toks)));
     }
 #undef RNB_LAUNCH_DM
-#undef RNB_LAUNCH_DMJ
 }
 
 }  // namespace rnb
