@@ -1150,7 +1150,7 @@ static uint32_t b32_slices(uint32_t rows, uint32_t seq, uint32_t steps) {
 size_t gemm_blocks_slice_floats(uint32_t quant, uint32_t rows, uint32_t k_steps, uint32_t seq) {
     if (rows == 0 || seq == 0 || k_steps == 0) return 0;
     const uint32_t row_tiles = (rows + kGbRows - 1) / kGbRows;
-    const bool wide = quant == kQ6K ? q6_wide_tiles(row_tiles, seq) : wide_tiles(row_tiles, seq);
+    const bool wide = quant == kQ6K ? q6_wide_tiles(row_tiles, seq) : quant != kQ4K && wide_tiles(row_tiles, seq);
     const uint32_t slices = is_b32(quant) ? b32_slices(rows, seq, k_steps)
                                           : k_slices(tile_grid(rows, seq, wide), k_steps, quant != kQ4K && quant != kQ5K);  // as the launchers
     return slices > 1 ? static_cast<size_t>(slices) * seq * rows : 0;
@@ -1229,14 +1229,15 @@ static void launch_gemm_q45k(const uint8_t *w, const uint8_t *w2, ActView act, f
     if (rows == 0 || seq == 0 || nb == 0) return;
     constexpr uint32_t mats = kPair ? 2 : 1;
     const uint32_t row_tiles = mats * ((rows + kGbRows - 1) / kGbRows);
-    const bool wide = wide_tiles(row_tiles, seq);
+    const bool wide = kFifth && wide_tiles(row_tiles, seq);  // grids of that many tiles run in gemm_q4k.hip on Q4_K
     const uint32_t slices = slice_out ? k_slices(tile_grid(mats * rows, seq, wide), nb, false) : 1;
     const uint32_t nb_slice = (nb + slices - 1) / slices, nz = (nb + nb_slice - 1) / nb_slice;
     float *dst = nz > 1 ? slice_out : out;
     if (wide) {
         const dim3 grid(row_tiles, (seq + 63) / 64, nz);
-        hipLaunchKernelGGL((gemm_q45k_mfma_kernel<2, kFifth, 16, kPair>), grid, dim3(kGbThreads), 0, stream, w, w2, act.qs, act.d,
-                           act.digits, dst, rows, nb, seq, nb_slice);
+        if constexpr (kFifth)
+            hipLaunchKernelGGL((gemm_q45k_mfma_kernel<2, true, 16, false>), grid, dim3(kGbThreads), 0, stream, w, w2, act.qs, act.d,
+                               act.digits, dst, rows, nb, seq, nb_slice);
     } else {
         const dim3 grid(row_tiles, (seq + 31) / 32, nz);
 #define RNB_LAUNCH_Q45(LIVE)                                                                                           \
