@@ -559,11 +559,10 @@ int run_dense_ffn_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, 
     const size_t nb_in = n_embd / 256, mid_bytes = seq * n_ff * sizeof(float);
     RESERVE_TRY(s.ffn_mid, mid_bytes);
     const bool aligned = (reinterpret_cast<uintptr_t>(gate_dev) | reinterpret_cast<uintptr_t>(up_dev)) % 16 == 0;
-    // the paired gate/up GEMV (a pass over both matrices per group of up to four tokens) against two GEMMs and the
-    // gated quantiser, measured on 14336 x 4096 with a Q6_K down projection: 4 tokens 44.1 vs 47.6 us for the whole
-    // layer, 6 tokens 56.1 vs 59.6, 7 tokens 62.3 vs 58.7 (11008 x 4096: 8 tokens 52.6 vs 55.1)
-    const size_t pair_max = n_ff * nb_in * kQ4KBytes >= kGemmSmallBytes ? 7 : 9;
-    const bool small = seq < pair_max && aligned && gemv_q4k_gate_up_supported(static_cast<uint32_t>(nb_in));
+    // the paired gate/up GEMV (a pass over both matrices per group of up to four tokens) for what the few-token GEMM leaves to it
+    // (below): three tokens, and on matrices of less than 4 MB eight, whose rows keep the one-token call's bits there (a whole layer,
+    // this : few-token GEMM, us: 1792 x 2048 four tokens 12.6 : 14.7, eight 15.4 : 15.1; 3072 x 2048 eight 16.4 : 14.6)
+    const bool small = seq <= 8 && aligned && gemv_q4k_gate_up_supported(static_cast<uint32_t>(nb_in));
     ActView act;
     int st = RNB_HIP_OK;
     if (small && seq == 1 && reinterpret_cast<uintptr_t>(x_dev) % 16 == 0) {
