@@ -184,9 +184,9 @@ bool gemm_few_supported(uint32_t quant, const uint8_t *w, size_t rows, size_t nb
 }
 
 // Where it is ahead of the GEMV passes over up to four tokens (us, GEMV : this kernel): rows of more than 16 blocks from three
-// tokens on (4096 x 14336 Q4_K 13.2 : 10.9, Q6_K 18.0 : 16.1); shorter ones, whose bits at two to four tokens do not depend on how
-// many rows the matrix has, from four (14336 x 4096 Q4_K 13.5 : 11.6, three 11.2 : 11.5), Q6_K five (14336 x 4096 22.6 : 16.4, four 17.6
-// : 16.6).
+// tokens on (4096 x 14336 Q4_K 13.2 : 10.9, Q6_K 18.0 : 16.1); shorter ones from four (14336 x 4096 Q4_K 13.5 : 11.6, three 11.2 :
+// 11.5), Q6_K five (14336 x 4096 22.6 : 16.4, four 17.6 : 16.6).  The GEMV's rows have the bits of the one-token call, this kernel's sums
+// are in an order that depends on the matrix (slices); the same holds either side of the next line.
 // Matrices of less than 4 MB keep the GEMV up to eight tokens (Q6_K 1024 x 4096 7.4 : 8.0 at eight, Q4_K 7.5 : 6.8) and its bits.
 // Ahead of gemm_blocks.hip everywhere up to 16 tokens, and with Q6_K; 17 to 32 tokens of Q4_K and Q5_K read twice the
 // activations per row, which costs more than the slices in memory where a wave has many blocks (24 tokens, Q4_K, gemm_blocks :

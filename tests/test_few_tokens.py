@@ -43,6 +43,25 @@ def test_few_tokens_equal_the_gold_dots(rnb, oracle, quant, rows, nb, seq):
     _check(oracle, quant, w, rows, cols, seq, x, got)
 
 
+# (largest batch whose rows equal the one-token call's, shapes): under 4 MB, rows of up to 16 blocks, of more, matrices of 48 MB
+@pytest.mark.parametrize("quant,most,rows,nb", [
+    (Q4_K, 8, 1792, 16), (Q5_K, 8, 1472, 16), (Q6_K, 8, 1232, 16), (Q4_K, 8, 1500, 17),
+    (Q4_K, 3, 1824, 16), (Q4_K, 3, 29200, 1), (Q5_K, 3, 1490, 16), (Q6_K, 4, 1252, 16), (Q6_K, 4, 20000, 1),
+    (Q4_K, 2, 1720, 17), (Q5_K, 2, 1410, 17), (Q6_K, 2, 1182, 17),
+    (Q4_K, 3, 24576, 16), (Q6_K, 4, 16384, 15)])
+def test_rows_that_equal_the_one_token_call(rnb, oracle, quant, most, rows, nb):
+    cols = 256 * nb
+    print(f"equal rows quant={quant} rows={rows} blocks={nb} tokens 2 .. {most}", flush=True)
+    w = oracle.make_weights(quant, rows, cols, 71)
+    x = oracle.fill_normal(most * cols, 72, 1.0)
+    one, many = (getattr(rnb, BATCH[quant].replace("_batch", end)) for end in ("", "_batch"))
+    alone = np.stack([np.asarray(one(w, rows, cols, x[t * cols:(t + 1) * cols])).reshape(rows) for t in range(most)])
+    for seq in range(2, most + 1):
+        got = np.asarray(many(w, rows, cols, x[:seq * cols])).reshape(seq, rows)
+        assert np.array_equal(got.view(np.uint32), alone[:seq].view(np.uint32)), seq
+    rnb.release(w)
+
+
 @pytest.mark.parametrize("quant", [Q4_K, Q5_K, Q6_K])
 def test_few_tokens_blocks_of_any_codes(rnb, oracle, quant):
     """Codes, scales and mins of any value, activations at both ends of their range."""

@@ -1106,9 +1106,8 @@ def test_dense_gelu_ffn(rnb, oracle, down_quant, seq, n_ff, n_embd):
 
 @pytest.mark.parametrize("seq,down_quant", [(5, Q6_K), (6, Q4_K), (7, Q6_K), (9, Q4_K)])
 def test_dense_silu_ffn_few_tokens_large_matrices(rnb, oracle, seq, down_quant):
-    """Gate / up matrices of 16 MB and more (8192 x 4096 Q4_K) keep the fused gate/up GEMV up to six tokens (groups of
-    3 + 2 and 3 + 3) and leave it for the GEMMs from seven on: gate and up GEMMs, SiLU * up quantised as it is made, down
-    GEMM (K slices on these small grids)."""
+    """Five to nine tokens on gate / up matrices of 16 MB and more (8192 x 4096 Q4_K): gate, up and SiLU * up in one launch of
+    the few-token GEMM, which also makes the down projection."""
     n_ff, n_embd = 8192, 4096
     gate = oracle.make_weights(Q4_K, n_ff, n_embd, 340 + seq)
     up = oracle.make_weights(Q4_K, n_ff, n_embd, 341 + seq)
