@@ -765,7 +765,7 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     size_t table_words = 5 * n_slots + (token_count + 1) + n_groups + (n_groups + 1);
     const bool inline_tables = !mfma && table_words <= kMoeInlineWords;  // decode-sized: rides in a kernel argument
     const bool few = matrix_batch && !inline_tables && aligned4 && (!mfma || moe_few_pays(n_groups, max_group, sh.nb_in, sh.nb_mid)) &&
-                     moe_few_supported(sh.nb_in, sh.nb_mid, token_count, n_slots, n_ff, n_embd, down_quant);
+                     moe_few_supported(sh.nb_in, sh.nb_mid, token_count, n_slots, n_ff, n_embd);
     const uint32_t unit_tokens = moe_few_tile(n_slots, n_groups);
     std::vector<uint32_t> units;
     if (few)

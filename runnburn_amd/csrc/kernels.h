@@ -240,7 +240,7 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
 // addresses, both activations quantised with digits
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups);
 bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid);
-bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant);
+bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd);
 void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
                             float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);
 void launch_moe_few_down(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act, const MoeGroups &g,

@@ -172,10 +172,10 @@ bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid
     return max_group > kMoeMfmaMaxGroup || n_groups <= 16 || n_groups * nb_in * nb_mid >= 2000;
 }
 
-bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd, uint32_t down_quant) {
-    // 32-bit offsets into the activations; every other Q6_K block's last piece ends two bytes behind it (gemm_few.h)
-    return nb_in <= kFewMaxBlocks && nb_mid <= kFewMaxBlocks && token_count * n_embd < (size_t(1) << 32) && n_slots * n_ff < (size_t(1) << 32) &&
-           (down_quant != kQ6K || n_embd * nb_mid % 2 == 0);
+// 32-bit offsets into the activations.  (The last piece of every other Q6_K block ends two bytes behind it, gemm_few.h: inside the
+// expert's matrix, whose n_embd rows, a multiple of 256, make an even number of blocks.)
+bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd) {
+    return nb_in <= kFewMaxBlocks && nb_mid <= kFewMaxBlocks && token_count * n_embd < (size_t(1) << 32) && n_slots * n_ff < (size_t(1) << 32);
 }
 
 void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
