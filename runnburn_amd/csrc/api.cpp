@@ -130,6 +130,11 @@ int reserve_fail(hipError_t e) {
 // 2048 25.7 -> 21.0, four 38.8 -> 25.9, Q4_K 14336 x 4096 34.8 -> 27.0, eight 4096 x 4096 46 -> 31; 64 tokens (1 MB each way) 127 -> 120,
 // 256 tokens level.
 constexpr size_t kBusBytes = size_t(1) << 20;
+// A wave that finishes one row for several tokens, or one row of an importance quant, stores its results one by one, each a transfer of
+// its own on the bus, faster than the bus takes them: from 32 KB of results on they go to device memory and a copying kernel sends
+// them in lines (direct : copied, us a call: Q4_0 32768 x 256, four tokens, 79 : 56, 4096 x 4096, eight, 44.2 : 39.9, IQ2_XXS 65536 x 256, one
+// token, 63.5 : 53.9, Q3_K 16384 x 4096, two, 38.4 : 35.7; 16 KB 21.7 : 23.0).
+constexpr size_t kBusSingleBytes = size_t(32) << 10;
 int bus_copy(State &s, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
     if (bytes > kBusBytes) {
         HIP_TRY(hipMemcpyAsync(dst, src, bytes, kind, s.stream));
@@ -238,6 +243,19 @@ bool one_launch_gemv(uint32_t quant, const uint8_t *w_dev, size_t rows, size_t c
     if (seq != 1) return false;
     if (is_block32(quant)) return gemv_block32_f32_supported(r, static_cast<uint32_t>(cols / 32), x_dev);
     return gemv_kquant_f32_supported(quant, nb, x_dev, w_dev) && gemv_kquant_f32_pays(quant, r, nb);
+}
+
+// Whether the matmul of these tokens has waves that hold several rows side by side: the one-launch GEMV, the GEMMs, a K-quant's GEMV on rows
+// of up to eight blocks and on matrices of chunks (as copied : direct: Q4_K 6144 x 1024, two tokens, 24.7 : 22.7; Q6_K 24576 x 4096, four,
+// 59.2 : 52.7; Q4_K 256000 x 256, one, 75.6 : 66.2; Q8_0 8192 x 1024, eight, 42.0 : 40.7).
+bool stores_rows_in_runs(uint32_t quant, const uint8_t *w_dev, size_t rows, size_t cols, size_t seq, bool one_launch) {
+    if (one_launch) return true;
+    if (is_iq_quant(quant)) return seq >= kIqGemmMinSeq;
+    const size_t nb = cols / 256;
+    if (seq >= gemm_min_seq(quant, rows, cols) || (gemm_few_supported(quant, w_dev, rows, nb, seq) && gemm_few_pays(quant, rows, nb, seq))) return true;
+    QuantInfo qi;
+    if (is_block32(quant) || !quant_info(quant, &qi)) return false;
+    return nb <= 8 || (nb <= 16 && rows * nb * qi.bytes >= kGemmChunkBytes);
 }
 
 int run_matmul_dev(State &s, uint32_t quant, const uint8_t *w_dev, size_t rows, size_t cols, const float *x_dev,
@@ -410,15 +428,17 @@ int matmul_host(uint32_t quant, const uint8_t *w, size_t w_len, size_t rows, siz
     HIP_TRY(s.out_f32.reserve(out_bytes));
     std::memcpy(s.bounce_in.ptr, x, in_bytes);
     const float *x_dev = s.bounce_in.as<float>();
-    float *out_dev = out_bytes <= kBusBytes ? s.bounce_out.as<float>() : s.out_f32.as<float>();
-    if (in_bytes > kBusBytes || one_launch_gemv(quant, w_dev, rows, cols, x_dev, seq)) {
+    const bool one_launch = one_launch_gemv(quant, w_dev, rows, cols, x_dev, seq);
+    const bool direct = out_bytes <= kBusSingleBytes || (out_bytes <= kBusBytes && stores_rows_in_runs(quant, w_dev, rows, cols, seq, one_launch));
+    float *out_dev = direct ? s.bounce_out.as<float>() : s.out_f32.as<float>();
+    if (in_bytes > kBusBytes || one_launch) {
         BUS_TRY(s.x_f32.ptr, s.bounce_in.ptr, in_bytes, hipMemcpyHostToDevice);
         x_dev = s.x_f32.as<float>();
     }
     s.h2d_bytes += in_bytes;
     st = run_matmul_dev(s, quant, w_dev, rows, cols, x_dev, seq, out_dev);
     if (st != RNB_HIP_OK) return st;
-    if (out_dev != s.bounce_out.as<float>()) BUS_TRY(s.bounce_out.ptr, s.out_f32.ptr, out_bytes, hipMemcpyDeviceToHost);
+    if (!direct) BUS_TRY(s.bounce_out.ptr, s.out_f32.ptr, out_bytes, hipMemcpyDeviceToHost);
     HIP_TRY(hipStreamSynchronize(s.stream));
     s.d2h_bytes += out_bytes;
     std::memcpy(out, s.bounce_out.ptr, out_bytes);

@@ -1,19 +1,21 @@
-"""Calls on host arrays: up to 1 MB a way the kernels read and write the pinned buffers themselves, above it copy commands carry the
-floats.  The result is the one of the same call on device buffers, to the bit, on both sides of the limit."""
+"""Calls on host arrays: up to 1 MB a way the kernels read and write the pinned buffers themselves or a copying kernel does (results of
+waves with one row each, from 32 KB on), above it copy commands carry the floats.  The result is the one of the same call on device buffers, to the bit, on both sides of the limit."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-Q8_0, Q4_K, Q6_K = 8, 12, 14
-BATCH = {Q8_0: "q8_0_gemv_batch", Q4_K: "q4k_gemv_batch", Q6_K: "q6k_gemv_batch"}
+Q8_0, Q4_K, Q6_K, IQ2_XXS = 8, 12, 14, 16
+BATCH = {Q8_0: "q8_0_gemv_batch", Q4_K: "q4k_gemv_batch", Q6_K: "q6k_gemv_batch", IQ2_XXS: "iq2_xxs_gemv_batch"}
 
 
 @pytest.mark.parametrize("quant,rows,cols,seq", [
     (Q8_0, 3, 32, 1), (Q8_0, 5, 96, 3), (Q4_K, 1, 256, 1), (Q4_K, 7, 4352, 1),   # tails of the copying kernel; one and two launches
     (Q8_0, 2047, 160, 128), (Q8_0, 2048, 160, 128), (Q8_0, 2049, 160, 128),      # results of just under, of and just over 1 MB
     (Q4_K, 33, 4096, 64), (Q4_K, 33, 4096, 65),                                  # tokens of 1 MB and over
-    (Q6_K, 262145, 256, 1), (Q4_K, 5, 262144 + 256, 1)])                         # one token: rows and blocks past the limit
+    (Q6_K, 262145, 256, 1), (Q4_K, 5, 262144 + 256, 1),                          # one token: rows and blocks past the limit
+    (Q8_0, 4096, 96, 2), (Q8_0, 4097, 96, 2), (IQ2_XXS, 8191, 256, 1), (IQ2_XXS, 8193, 256, 1),  # results of a GEMV, 32 KB and over
+    (Q6_K, 4097, 2304, 2), (Q6_K, 4097, 2048, 2), (IQ2_XXS, 2049, 256, 5)])      # ... of longer and short rows, of a GEMM
 def test_host_arrays_equal_device_buffers(rnb, oracle, quant, rows, cols, seq):
     print(f"host call quant={quant} rows={rows} cols={cols} seq={seq}", flush=True)
     w = oracle.make_weights(quant, rows, cols, 3)
