@@ -595,9 +595,7 @@ int run_dense_ffn_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, 
     }
     st = quantize_activations(s, kQ4K, x_dev, seq, n_embd, &act);
     if (st != RNB_HIP_OK) return st;
-    // gate and up in one launch of the few-token GEMM: four tokens 36.5 us against the pair's 44 for the whole layer, three 36.4
-    // against 34.2 (rows of more than 16 blocks, which the paired GEMV does not take: 18.8 against 22.6)
-    const bool few = gemm_few_pays(kQ4K, n_ff, nb_in, seq) && (seq > 3 || nb_in > 16) && act.digits != nullptr &&
+    const bool few = gemm_few_gate_up_pays(n_ff, nb_in, seq) && act.digits != nullptr &&
                      gemm_few_supported(kQ4K, gate_dev, n_ff, nb_in, seq) && gemm_few_supported(kQ4K, up_dev, n_ff, nb_in, seq);
     if (few) {
         launch_gemm_few_gate_up(gate_dev, up_dev, act, s.ffn_mid.as<float>(), static_cast<uint32_t>(n_ff),

@@ -183,8 +183,10 @@ bool gemm_few_supported(uint32_t quant, const uint8_t *w, size_t rows, size_t nb
     return quant != kQ6K || rows * nb % 2 == 0;
 }
 
-// Where it is ahead of the GEMV passes over up to four tokens (us, GEMV : this kernel): rows of more than 16 blocks from three
-// tokens on (4096 x 14336 Q4_K 13.2 : 10.9, Q6_K 18.0 : 16.1); shorter ones from four (14336 x 4096 Q4_K 13.5 : 11.6, three 11.2 :
+namespace {
+
+// Where the kernel fits a matrix of this shape.  Ahead of the GEMV passes over up to four tokens (us, GEMV : this kernel): rows of more
+// than 16 blocks from three tokens on (4096 x 14336 Q4_K 13.2 : 10.9); shorter ones from four (14336 x 4096 Q4_K 13.5 : 11.6, three 11.2 :
 // 11.5), Q6_K five (14336 x 4096 22.6 : 16.4, four 17.6 : 16.6).  The GEMV's rows have the bits of the one-token call, this kernel's sums
 // are in an order that depends on the matrix (slices); the same holds either side of the next line.
 // Matrices of less than 4 MB keep the GEMV up to eight tokens (Q6_K 1024 x 4096 7.4 : 8.0 at eight, Q4_K 7.5 : 6.8) and its bits.
@@ -192,9 +194,8 @@ bool gemm_few_supported(uint32_t quant, const uint8_t *w, size_t rows, size_t nb
 // activations per row, which costs more than the slices in memory where a wave has many blocks (24 tokens, Q4_K, gemm_blocks :
 // this: 1024 x 14336 12.3 : 14.3, 1024 x 8192 9.9 : 10.6; 2048 x 8192 11.6 : 10.9) or the matrix is large (65536 x 4096 47 : 50, Q5_K
 // 28672 x 8192 55 : 57, 28672 x 1024 11.8 : 13.6; 28672 x 4096 Q4_K 30.1 : 28.4, Q5_K 34.0 : 33.4).
-bool gemm_few_pays(uint32_t quant, size_t rows, size_t nb, size_t seq) {
+bool few_shape(uint32_t quant, size_t rows, size_t nb, size_t seq, size_t bytes) {
     if (seq < 3 || seq > 32) return false;
-    const size_t bytes = rows * nb * (quant == kQ4K ? kQ4KBytes : quant == kQ5K ? kQ5KBytes : kQ6KBytes);
     if (bytes < (size_t(4) << 20)) {
         if (seq <= 8) return false;
     } else if (nb <= 16 && seq < (quant == kQ6K ? 5 : 4)) {
@@ -206,6 +207,47 @@ bool gemm_few_pays(uint32_t quant, size_t rows, size_t nb, size_t seq) {
     if (rows > 24576 && nb < 8) return false;
     return quant == kQ4K ? rows <= 32768 : rows * nb <= 480000;
 }
+
+// workgroups of a call over those that its rounds of `at_once` have places for
+double rounds_fill(const FewPlan &p, uint32_t rows, uint32_t at_once) {
+    const uint32_t per_wg = p.waves / p.slices * 16 * p.row_tiles, wgs = (rows + per_wg - 1) / per_wg;
+    return static_cast<double>(wgs) / ((wgs + at_once - 1) / at_once * at_once);
+}
+
+}  // namespace
+
+// One matrix (us, the other kernel : this one).  Left to kernels that cut K further: a few row tiles with a long chain of blocks each, up
+// to 512 rows (160 x 10752 Q4_K, 11 tokens 6.7 : 8.6, 337 x 15360 Q5_K, 12 10.3 : 12.1; 394 x 9728 Q4_K, 11 9.3 : 8.5), 1024 with three
+// tokens (the down projection of an FFN 7680 x 1024 Q4_K 13.1 : 14.4 for the whole layer), three tokens of Q5_K up to 2048 rows of more than
+// 32 blocks (eight matrices 0.73 - 1.0), of Q6_K any (41 matrices 0.68 - 1.11), four up to 2400 rows (0.71 - 1.06).
+// Left to gemm_blocks.hip where the last round of workgroups is nearly empty and each has much to read: two row tiles a wave over one
+// workgroup a unit (Q6_K 8268 x 12544, 13 tokens, 259 workgroups 28.5 : 36.3, Q4_K 8595 x 14592, three, 0.87) and, with 17 to 32 tokens from
+// 24 MB on, over the places of all (Q4_K 18981 x 15872 47.4 : 53.4, 17249 x 4352 21.4 : 23.5; Q5_K 9170 x 9216 23.2 : 27.8; 13824 x 5120, 84 %
+// full, 23.3 : 20.0); many short rows (19963 x 1536 11.4 : 13.4; 15330 x 1280 10.4 : 9.7).
+// Of 927 random matrices that take longer than a launch 34 are more than 3 % behind the kernels before this one (99 by few_shape alone),
+// 0.841 of their time on average.
+bool gemm_few_pays(uint32_t quant, size_t rows, size_t nb, size_t seq) {
+    const size_t bytes = rows * nb * (quant == kQ4K ? kQ4KBytes : quant == kQ5K ? kQ5KBytes : kQ6KBytes);
+    if (!few_shape(quant, rows, nb, seq, bytes)) return false;
+    if (seq <= 16 && rows <= (seq == 3 ? 1024 : 512)) return false;
+    if (seq == 3 && (quant == kQ6K || (quant == kQ5K && rows <= 2048 && nb > 32))) return false;
+    if (seq == 4 && quant == kQ6K && rows <= 2400) return false;
+    const uint32_t r = static_cast<uint32_t>(rows), b = static_cast<uint32_t>(nb);
+    const FewPlan p = few_plan(quant, r, b, static_cast<uint32_t>(seq));
+    if (p.row_tiles == 2 && bytes >= (size_t(24) << 20) && rounds_fill(p, r, 256) < 0.65) return false;
+    if (seq <= 16 || quant == kQ6K) return true;
+    if (rows > 16384 && nb < 8) return false;
+    if (bytes < (size_t(24) << 20) || (quant == kQ4K && p.row_tiles == 1)) return true;
+    const size_t stage = quant == kQ4K         ? FewLds<kQ4K, 2, 2, 1>::kStage
+                         : p.row_tiles == 1 ? FewLds<kQ5K, 2, 1, 1>::kStage
+                                            : FewLds<kQ5K, 2, 2, 1>::kStage;
+    const size_t lds = p.waves * stage + nb * 32 * sizeof(float);
+    return lds <= 160 * 1024 && rounds_fill(p, r, 256 * static_cast<uint32_t>(160 * 1024 / lds)) >= 0.75;
+}
+
+// both matrices of a gated FFN; three tokens of short rows: in the paired GEMV 34.2 us for the whole layer against 36.4, four 44 : 36.5
+// (rows of more than 16 blocks, which the paired GEMV does not take: 22.6 : 18.8)
+bool gemm_few_gate_up_pays(size_t rows, size_t nb, size_t seq) { return few_shape(kQ4K, rows, nb, seq, rows * nb * kQ4KBytes) && (seq > 3 || nb > 16); }
 
 void launch_gemm_few(const uint8_t *w, uint32_t quant, ActView act, float *out, uint32_t rows, uint32_t nb, uint32_t seq,
                      hipStream_t stream) {

@@ -164,6 +164,7 @@ void launch_gemm_digits(const uint8_t *w, uint32_t quant, ActView act, float *ou
 // Q4_K, Q5_K and Q6_K against at most 32 tokens, the K slices inside a workgroup: no workspace (act needs digits for Q4_K /
 // Q5_K); the gate_up form is mid = act(Wg a) * (Wu a) on Q4_K
 bool gemm_few_pays(uint32_t quant, size_t rows, size_t nb, size_t seq);
+bool gemm_few_gate_up_pays(size_t rows, size_t nb, size_t seq);
 bool gemm_few_supported(uint32_t quant, const uint8_t *w, size_t rows, size_t nb, size_t seq);
 void launch_gemm_few(const uint8_t *w, uint32_t quant, ActView act, float *out, uint32_t rows, uint32_t nb, uint32_t seq,
                      hipStream_t stream);

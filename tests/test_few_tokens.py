@@ -22,8 +22,10 @@ def _check(oracle, quant, w, rows, cols, seq, x, got):
     assert worst <= 2e-5 * rms, (quant, rows, cols, seq, worst / rms)
 
 
-# rows around the 16-row tile and the workgroup's rows, blocks around the eight and four slices, tokens around the two tiles
-SHAPES = [(1, 1, 9), (15, 2, 16), (16, 3, 17), (17, 5, 31), (31, 7, 32), (33, 8, 12), (64, 9, 10), (250, 17, 24), (77, 56, 13),
+# rows around the 16-row tile and the workgroup's rows, blocks around the eight and four slices, tokens around the two tiles (up to 512
+# rows with up to sixteen tokens are the GEMV's)
+SHAPES = [(529, 1, 9), (527, 2, 16), (545, 8, 12), (576, 9, 10), (513, 56, 13), (1026, 34, 3),
+          (1, 1, 9), (15, 2, 16), (16, 3, 17), (17, 5, 31), (31, 7, 32), (33, 8, 12), (64, 9, 10), (250, 17, 24), (77, 56, 13),
           (48, 64, 32), (2048, 33, 3), (4096, 16, 5),
           (4097, 8, 11), (4113, 3, 20), (7000, 9, 19),      # four slices; fewer blocks than slices
           (20481, 2, 15), (20490, 5, 27),                   # two slices; a second token tile
@@ -47,7 +49,7 @@ def test_few_tokens_equal_the_gold_dots(rnb, oracle, quant, rows, nb, seq):
 @pytest.mark.parametrize("quant,most,rows,nb", [
     (Q4_K, 8, 1792, 16), (Q5_K, 8, 1472, 16), (Q6_K, 8, 1232, 16), (Q4_K, 8, 1500, 17),
     (Q4_K, 3, 1824, 16), (Q4_K, 3, 29200, 1), (Q5_K, 3, 1490, 16), (Q6_K, 4, 1252, 16), (Q6_K, 4, 20000, 1),
-    (Q4_K, 2, 1720, 17), (Q5_K, 2, 1410, 17), (Q6_K, 2, 1182, 17),
+    (Q4_K, 2, 1720, 17), (Q5_K, 2, 1410, 17), (Q6_K, 3, 1182, 17),
     (Q4_K, 3, 24576, 16), (Q6_K, 4, 16384, 15)])
 def test_rows_that_equal_the_one_token_call(rnb, oracle, quant, most, rows, nb):
     cols = 256 * nb
@@ -86,7 +88,7 @@ def test_few_tokens_blocks_of_any_codes(rnb, oracle, quant):
 def test_few_tokens_of_a_part_of_a_resident_tensor(rnb, oracle, quant, shift):
     """At addresses that are no multiple of four the other kernels answer, and so they do for a Q6_K matrix of an odd number of
     blocks, whose last piece would end behind the tensor."""
-    rows, nb, seq = 35, 5, 14
+    rows, nb, seq = 515, 5, 14
     w = oracle.make_weights(quant, rows, 256 * nb, 8)
     x = oracle.fill_normal(seq * 256 * nb, 9, 1.0)
     parent = np.zeros(w.size + shift, np.uint8)
@@ -100,7 +102,7 @@ def test_few_tokens_of_a_part_of_a_resident_tensor(rnb, oracle, quant, shift):
 @pytest.mark.parametrize("quant,seq", [(Q4_K, 13), (Q6_K, 30)])
 def test_few_tokens_finite_from_any_neighbours(rnb, oracle, quant, seq):
     """A token's result does not depend on the others in its tile, NaN and infinities among them included."""
-    rows, nb = 300, 6
+    rows, nb = 600, 6
     w = oracle.make_weights(quant, rows, 256 * nb, 18)
     x = oracle.fill_normal(seq * 256 * nb, 19, 1.0).reshape(seq, -1)
     bad = x.copy()
