@@ -399,9 +399,12 @@ void launch_b32_plan(const uint8_t *w, const ActView &act, float *out, float *sl
 
 // Ahead of gemm_blocks.hip everywhere but on Q8_1, whose 36-byte blocks that kernel loads at 4-byte boundaries, where rows are
 // short or the last tile of 256 rows is most of them (590 x 1024 x 1414 tokens 21.8 us there against 23.8 here, 736 x 5120 x 90 17.4
-// against 18.2; 1030 x 1280 x 700 level; Q8_0 512 x 1024 x 33 15.4 against 11.0).
+// against 18.2; 1030 x 1280 x 700 level; Q8_0 512 x 1024 x 33 15.4 against 11.0), and in less than a round of workgroups on rows of a step or
+// two of the formats whose codes take longest to make, which nothing stands beside there (Q5_1 355 x 256 x 104 10.4 against 11.6, 3650 x
+// 512 x 407 16.5 against 17.6, Q5_0 5901 x 256 x 225 10.6 against 11.1; 17600 x 256 x 1170 52.7 against 43.1; Q5_0 x 512 within 2 %).
 bool gemm_b32_pays(uint32_t quant, const uint8_t *w, size_t rows, size_t cols, size_t seq) {
     if (quant == kQ8_1 && (rows <= 768 || cols <= 1024)) return false;
+    if (cols <= (quant == kQ5_1 ? 512 : quant == kQ5_0 ? 256 : 0) && rows * seq <= 2000000) return false;
     return seq > 32 && cols % 256 == 0 && reinterpret_cast<uintptr_t>(w) % 4 == 0 && cols < (size_t(1) << 23);
 }
 

@@ -24,7 +24,7 @@ def _check(oracle, quant, w, rows, cols, seq, x, got):
 # and the groups of two, three and four tiles
 @pytest.mark.parametrize("quant", [Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, Q8_1])
 @pytest.mark.parametrize("rows,steps,seq", [(1, 1, 33), (31, 2, 64), (33, 3, 65), (255, 1, 129), (257, 17, 96), (288, 5, 97), (1000, 11, 40),
-                                            (800, 6, 700), (2080, 5, 200), (4097, 2, 513), (1025, 33, 34)])
+                                            (800, 6, 700), (2080, 5, 200), (4097, 2, 513), (1025, 33, 34), (1, 3, 33), (4097, 3, 129)])
 def test_prefill_of_32_element_blocks(rnb, oracle, quant, rows, steps, seq):
     cols = 256 * steps
     print(f"32-element prefill quant={quant} rows={rows} cols={cols} seq={seq}", flush=True)
