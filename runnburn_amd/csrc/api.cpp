@@ -765,9 +765,9 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     const size_t n_groups = grp_expert.size();
     uint32_t max_group = 0;
     for (size_t g = 0; g < n_groups; g++) max_group = std::max(max_group, grp_start[g + 1] - grp_start[g]);
-    // Batches of sixteen tokens and more run on the matrix cores: moe_few.hip, or moe_mfma.hip for small calls (moe_few_pays) with at
-    // least 1.8 slots per routed expert on average (a 32-token tile costs the same whatever its number of live tokens, the
-    // integer-dot kernels cost per token; measured on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot
+    // Batches of sixteen tokens and more (a smaller one's rows are a lone token's bit for bit) run on the matrix cores: moe_few.hip, or
+    // moe_mfma.hip where moe_mfma_pays says so and there are at least 1.8 slots per routed expert on average (a 32-token tile
+    // costs the same whatever its number of live tokens, the integer-dot kernels cost per token; measured on 128 experts x top-8: 16 / 20 / 24 tokens 71.9 / 84.2 / 93.9 us on the integer-dot
     // kernels, 79.0 / 85.7 / 88.2 in moe_mfma.hip; the ratio is 1.6 / 1.8 / 1.9 there), which needs the quantiser's digits
     // (its gate/up rows arrive as 16-byte LDS-direct loads and the Q6_K down rows as dword-aligned pieces: an even base address and
     // whole 128-row tiles).  Tables of a kernel argument's size ride in one, with the integer-dot kernels, unless that ratio is met.
@@ -782,7 +782,8 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
     // grp_start[G+1] | slot_expert[n] | units
     size_t table_words = 5 * n_slots + (token_count + 1) + n_groups + (n_groups + 1);
     const bool inline_tables = !mfma && table_words <= kMoeInlineWords;  // decode-sized: rides in a kernel argument
-    const bool few = matrix_batch && !inline_tables && aligned4 && (!mfma || moe_few_pays(n_groups, max_group, sh.nb_in, sh.nb_mid)) &&
+    const bool mfma_pays = mfma && moe_mfma_pays(n_groups, max_group, n_ff, sh.nb_in, sh.nb_mid, down_quant);
+    const bool few = matrix_batch && !inline_tables && aligned4 && !mfma_pays &&
                      moe_few_supported(sh.nb_in, sh.nb_mid, token_count, n_slots, n_ff, n_embd);
     const uint32_t unit_tokens = moe_few_tile(n_slots, n_groups);
     std::vector<uint32_t> units;
@@ -885,7 +886,7 @@ int run_moe_dev(State &s, const uint8_t *gate_dev, const uint8_t *up_dev, const 
         if (int ls = check_launches(); ls != RNB_HIP_OK) return ls;
         return RNB_HIP_OK;
     }
-    if (mfma && max_group <= kMoeMfmaMaxGroup && n_groups <= 65535 && act.digits != nullptr) {
+    if (mfma_pays && act.digits != nullptr) {
         // the down kernel quantises the intermediate as it stages it
         launch_moe_gate_up_mfma(gate_dev, up_dev, shared, act, groups, s.moe_mid.as<float>(), static_cast<uint32_t>(n_ff),
                                 static_cast<uint32_t>(sh.nb_in), s.stream);

@@ -229,10 +229,10 @@ void launch_moe_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const Mo
 bool moe_down_quantises(uint32_t nb_mid);  // whether that pays (short intermediates)
 void launch_moe_down(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, ActView mid_act,
                      const float *mid_f32, MoeGroups groups, const float *slot_route, float *slot_out, uint32_t n_embd, uint32_t nb_mid, hipStream_t stream);
-// the same two steps on the matrix cores for small batches of groups of at most kMoeMfmaMaxGroup slots, up to 65535 of them (act
-// carries digits), see moe_mfma.hip
-constexpr size_t kMoeMfmaMaxGroup = 8;
+// the same two steps on the matrix cores for batches whose groups have at most kMoeMfmaMaxGroup slots (act carries digits)
+constexpr uint32_t kMoeMfmaMaxGroup = 16;
 bool moe_mfma_supported(uint32_t nb_in, uint32_t nb_mid, uint32_t down_quant);  // the groups' LDS images fit
+bool moe_mfma_pays(size_t n_groups, size_t max_group, size_t n_ff, size_t nb_in, size_t nb_mid, uint32_t down_quant);  // against moe_few.hip
 void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act,
                              MoeGroups groups, float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);
 void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint32_t down_quant, const float *mid, MoeGroups groups,
@@ -240,7 +240,6 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
 // the same two steps on the few-token GEMM's tiles (moe_few.hip): groups with units of moe_few_tile slots, weights at 4-byte
 // addresses, both activations quantised with digits
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups);
-bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid);
 bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd);
 void launch_moe_few_gate_up(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act, const MoeGroups &g,
                             float *mid, uint32_t n_ff, uint32_t nb_in, hipStream_t stream);

@@ -161,17 +161,6 @@ void launch_moe_few(const uint8_t *w, const uint8_t *w2, const uint8_t *ws, cons
 // top-2 of 1024 x 2304 at 400 72 : 66; only 8 x top-2 of 2048 x 4096 at 400 gained much (115 : 135).
 uint32_t moe_few_tile(size_t n_slots, size_t n_groups) { return n_slots <= 14 * n_groups ? 16 : 32; }
 
-// Against the integer-dot kernels of moe.hip from sixteen tokens on (a smaller batch's rows are a lone token's bit for bit), against
-// moe_mfma.hip unless every group is at most kMoeMfmaMaxGroup slots and the call small: that kernel finishes only the results of eight
-// slots and its down projection quantises the intermediates itself, one launch of 5 us less, which counts where the experts' weights
-// are read in 30 - 60 us; up to sixteen groups leave its one workgroup a unit idle.  Us a call, moe_mfma : this, Q5_K down projections:
-// 128 x top-8 of 256 x 2304 at 21 tokens 36.7 : 42.7, of 1024 x 1024 at 19 44.9 : 50.7; 512 x 3328 at 21 (2366 blocks) 92.7 : 76.1, 8 x top-2 of
-// 2048 x 1024, Q6_K, at 26 38.2 : 29.1.  780 random calls of 16 to 300 tokens (7 to 244 experts hit, rows of 3 to 18 blocks, intermediates of
-// 1 to 10): 0.25 % over the better one of the two on average, 19 of them 3 - 13 % behind moe_mfma.hip (mostly Q5_K with groups of 9 to 15).
-bool moe_few_pays(size_t n_groups, size_t max_group, size_t nb_in, size_t nb_mid) {
-    return max_group > kMoeMfmaMaxGroup || n_groups <= 16 || n_groups * nb_in * nb_mid >= 2000;
-}
-
 // 32-bit offsets into the activations.  (The last piece of every other Q6_K block ends two bytes behind it, gemm_few.h: inside the
 // expert's matrix, whose n_embd rows, a multiple of 256, make an even number of blocks.)
 bool moe_few_supported(size_t nb_in, size_t nb_mid, size_t token_count, size_t n_slots, size_t n_ff, size_t n_embd) {

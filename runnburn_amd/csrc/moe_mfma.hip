@@ -1,8 +1,8 @@
-// Gathered sparse-MoE experts on the matrix cores, for small batches whose experts have at most eight slots each (larger ones:
-// moe_few.hip, moe_few_pays): the grouped form of gemm_blocks.hip.  Slots are sorted by expert on the host (api.cpp); workgroup
+// Gathered sparse-MoE experts on the matrix cores, for batches whose experts have at most sixteen slots each where that pays
+// (moe_mfma_pays; others: moe_few.hip): the grouped form of gemm_blocks.hip.  Slots are sorted by expert on the host (api.cpp); workgroup
 // (row tiles, group): the group's quantised activations are gathered into LDS by the sorted lists, the expert's weight rows go
 // from global memory to the registers of the lane that owns the row, one int8 matrix instruction per scale group, the group's
-// scale on the vector units (see gemm_blocks.hip), which finish the results of eight tokens of the instruction's 32.  The work
+// scale on the vector units (see gemm_blocks.hip), which finish the results of eight or sixteen tokens of the instruction's 32.  The work
 // per group is the same whatever the number of live tokens, where the integer-dot kernels of moe.hip cost per token.  Padding
 // costs no LDS either: only the live tokens are staged, the matrix instruction's padding lanes read the last live token's
 // row, and the launch sizes the image for the largest group of the call, so that several workgroups share a compute
@@ -16,13 +16,13 @@
 #include "device_utils.h"
 #include "kernels.h"
 #include "mfma_blocks.h"
+#include <type_traits>
 
 namespace rnb {
 
 namespace {
 
 constexpr int kMmToks = 32;     // tokens of a matrix instruction
-constexpr int kMmResults = 4;   // results of a lane that belong to the first eight of them, kMoeMfmaMaxGroup
 constexpr int kQ4FillInstr = (32 * kQ4Pieces + kWave - 1) / kWave;  // 5 wave-wide 16-byte loads per 32 rows of a Q4_K block
 constexpr int kQ4FillBytes = kQ4FillInstr * 1024;                   // what they write: 32 x 144 bytes of rows + the tail
 constexpr int kMmGateUpStripBytes = kGbWaves * 2 * kQ4FillBytes;    // gate and up strips of the four waves
@@ -91,9 +91,9 @@ __device__ __forceinline__ void tile_stage_store(const TileStage<kThreads> &st, 
 
 // One super-block of one 32-token tile against one Q4_K / Q5_K row share: I = sum_sb sc * (codes . a) and the mins sum
 // S = sum_sb mn * bsum32 (through the digits); returns d * I - dmin * S per result in `val`.
-// Only the results of the tile's first eight tokens are finished on the vector units (result r of a lane is token
-// 8 * (r / 4) + 4 * khalf + r % 4, so they are the lane's first four); the matrix instructions always compute all 32
-// tokens, which costs nothing extra.
+// kJ = 1 or 2: only the results of the tile's first 8 kJ tokens are finished on the vector units (result r of a lane
+// is token 8 * (r / 4) + 4 * khalf + r % 4, so they are the lane's first 4 kJ results); the matrix instructions always
+// compute all 32 tokens, which costs nothing extra.
 // The matrix instruction of sub-block SB is issued before the results of sub-block SB - 1 are scaled: a wave that has
 // its SIMD to itself would otherwise sit out the instruction's latency (16 passes) eight times per block.
 #define RNB_Q45_ISSUE(SB, ROW, ACC, SC)                                                                  \
@@ -106,7 +106,7 @@ __device__ __forceinline__ void tile_stage_store(const TileStage<kThreads> &st, 
     }
 #define RNB_Q45_TAKE(ACC, SC, TOT)                                                                       \
     {                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < kMmResults; i++) {                                             \
+        _Pragma("unroll") for (int i = 0; i < 4 * kJ; i++) {                                             \
             TOT[i] += mul24(ACC[i], SC);                                                                 \
             asm volatile("" : "+v"(TOT[i])); /* keep the eight additions a chain, not a tree */          \
         }                                                                                                \
@@ -142,16 +142,16 @@ __device__ __forceinline__ void tile_ops_load(TileOps64 &o, const uint8_t *abase
     for (int sb = 0; sb < 16; sb++) o.v[sb] = *reinterpret_cast<const long *>(abase + 16 * sb);
 }
 
-template <bool kFifth>
+template <bool kFifth, int kJ>
 __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps128 &aops, const uint4 dig, int khalf,
-                                               float (&val)[kMmResults]) {
+                                               float (&val)[4 * kJ]) {
     const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const Q4KScales sc8 = unpack_q4k_scales(row.hdr.y, row.hdr.z, row.hdr.w);
-    // the scale on the results: four multiply-adds per sub-block, where folding it into the operand would take eight and a second
+    // the scale on the results: 4 kJ multiply-adds per sub-block, where folding it into the operand would take eight and a second
     // matrix instruction
-    int tot[kMmResults];
+    int tot[4 * kJ];
 #pragma unroll
-    for (int i = 0; i < kMmResults; i++) tot[i] = 0;
+    for (int i = 0; i < 4 * kJ; i++) tot[i] = 0;
     v16i acc_a, acc_b;
     int sc_a, sc_b;
     RNB_Q45_SUB_BLOCK(0, row, tot)
@@ -171,7 +171,7 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
     const v16i c0 = __builtin_amdgcn_mfma_i32_32x32x16_i8(op0, mnop, zero16, 0, 0, 0);
     const v16i c1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(op1, mnop, zero16, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < kMmResults; i++) val[i] = d * static_cast<float>(tot[i]) - dmin * static_cast<float>(c0[i] + 64 * c1[i]);
+    for (int i = 0; i < 4 * kJ; i++) val[i] = d * static_cast<float>(tot[i]) - dmin * static_cast<float>(c0[i] + 64 * c1[i]);
 }
 #undef RNB_Q45_SUB_BLOCK
 #undef RNB_Q45_TAKE
@@ -188,7 +188,7 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
     }
 #define RNB_Q6_TILE_TAKE(ACC, SC)                                                                        \
     {                                                                                                    \
-        _Pragma("unroll") for (int i = 0; i < kMmResults; i++) {                                             \
+        _Pragma("unroll") for (int i = 0; i < 4 * kJ; i++) {                                             \
             tot[i] += mul24(ACC[i], SC);                                                                 \
             asm volatile("" : "+v"(tot[i]));                                                             \
         }                                                                                                \
@@ -206,11 +206,12 @@ __device__ __forceinline__ void q45_block_tile(const Q5Row &row, const TileOps12
             RNB_Q6_TILE_TAKE(acc_a, sc_a)                                                                \
         }                                                                                                \
     }
-__device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 &aops, float (&val)[kMmResults]) {
+template <int kJ>
+__device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 &aops, float (&val)[4 * kJ]) {
     const v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int tot[kMmResults];
+    int tot[4 * kJ];
 #pragma unroll
-    for (int i = 0; i < kMmResults; i++) tot[i] = 0;
+    for (int i = 0; i < 4 * kJ; i++) tot[i] = 0;
     v16i acc_a, acc_b;
     int sc_a, sc_b;
     RNB_Q6_TILE_SUB_BLOCK(0)
@@ -231,23 +232,27 @@ __device__ __forceinline__ void q6_block_tile(const Q6Row &row, const TileOps64 
     RNB_Q6_TILE_SUB_BLOCK(15)
     RNB_Q6_TILE_TAKE(acc_b, sc_b)
 #pragma unroll
-    for (int i = 0; i < kMmResults; i++) val[i] = row.d * static_cast<float>(tot[i]);
+    for (int i = 0; i < 4 * kJ; i++) val[i] = row.d * static_cast<float>(tot[i]);
 }
 #undef RNB_Q6_TILE_SUB_BLOCK
 #undef RNB_Q6_TILE_TAKE
 #undef RNB_Q6_TILE_ISSUE
 
-// accf[r] += d_x[token of result r] * val[r]; result r of a tile is token 4 * khalf + r
-__device__ __forceinline__ void tile_scale_add(const float *dxbuf, int khalf, const float (&val)[kMmResults], float (&accf)[kMmResults]) {
-    const float4 dx4 = reinterpret_cast<const float4 *>(dxbuf)[khalf];
-    const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+// accf[r] += d_x[token of result r] * val[r]; result r of a tile is token 8 * (r / 4) + 4 * khalf + r % 4
+template <int kJ>
+__device__ __forceinline__ void tile_scale_add(const float *dxbuf, int khalf, const float (&val)[4 * kJ], float (&accf)[4 * kJ]) {
 #pragma unroll
-    for (int i = 0; i < kMmResults; i++) accf[i] += dx[i] * val[i];
+    for (int j = 0; j < kJ; j++) {
+        const float4 dx4 = reinterpret_cast<const float4 *>(dxbuf)[2 * j + khalf];
+        const float dx[4] = {dx4.x, dx4.y, dx4.z, dx4.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) accf[4 * j + i] += dx[i] * val[4 * j + i];
+    }
 }
 
 // LDS image of one tile: every 256-element block of the tile's live tokens, staged once and then only read
 //   act[nb][toks][kStride] | d_x[nb][32] | digits[nb][32] (16 bytes each; absent for Q6_K weights)
-// toks <= 8 is the number of token rows the launch made room for (the largest group of the call)
+// toks <= 16 is the number of token rows the launch made room for (the largest group of the call)
 template <int kStride, bool kDigits>
 struct TileImage {
     static __host__ __device__ size_t act_bytes(uint32_t nb, uint32_t toks) { return static_cast<size_t>(nb) * toks * kStride; }
@@ -285,7 +290,7 @@ __device__ __forceinline__ void tile_image_fill(const TileImage<kStride, kDigits
 // (consecutive lanes take consecutive 16-byte pieces of a row, see RowRoute for why; no vector registers hold the data in
 // flight), and each lane reads its row's share back from there.  Dynamic LDS: the waves' strips, then the tile image.
 // ---------------------------------------------------------------------------------------------
-template <int kW>
+template <int kJ, int kW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * kW), amdgpu_waves_per_eu(2)))
     moe_gate_up_mfma_kernel(const uint8_t *__restrict__ gate_all, const uint8_t *__restrict__ up_all,
                             const uint8_t *__restrict__ gate_shared, const uint8_t *__restrict__ up_shared, uint32_t n_routed,
@@ -368,36 +373,44 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(kWave * kW, kWave * k
     Q5Row cg, cu;
     take(cg, cu);
     __syncthreads();
-    for (uint32_t rt = 0; rt < rt_n; rt++) {
-        const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
-        float accg[kMmResults] = {}, accu[kMmResults] = {};
-        for (uint32_t b = 0; b < nb; b++) {
-            request();  // the step after this one
-            const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
-            const uint4 dig = img.dig(b)[lrow];
-            float val[kMmResults];
-            TileOps128 aops;
-            tile_ops_load(aops, abase);
-            q45_block_tile<false>(cg, aops, dig, khalf, val);
-            tile_scale_add(img.dx(b), khalf, val, accg);
-            q45_block_tile<false>(cu, aops, dig, khalf, val);
-            tile_scale_add(img.dx(b), khalf, val, accu);
-            take(cg, cu);  // (after the last step: a repeat of it, unused)
-        }
-        if (row < n_ff) {
+    // a group of at most eight slots among larger ones finishes only a lane's first four results
+    auto walk = [&](auto jtag) {
+        constexpr int kJl = decltype(jtag)::value;
+        for (uint32_t rt = 0; rt < rt_n; rt++) {
+            const uint32_t row = (rt0 + rt) * (32 * kW) + wave * 32 + lrow;
+            float accg[4 * kJl] = {}, accu[4 * kJl] = {};
+            for (uint32_t b = 0; b < nb; b++) {
+                request();  // the step after this one
+                const uint8_t *abase = img.act(b) + arow * kGbStride128 + 16 * khalf;
+                const uint4 dig = img.dig(b)[lrow];
+                float val[4 * kJl];
+                TileOps128 aops;
+                tile_ops_load(aops, abase);
+                q45_block_tile<false, kJl>(cg, aops, dig, khalf, val);
+                tile_scale_add<kJl>(img.dx(b), khalf, val, accg);
+                q45_block_tile<false, kJl>(cu, aops, dig, khalf, val);
+                tile_scale_add<kJl>(img.dx(b), khalf, val, accu);
+                take(cg, cu);  // (after the last step: a repeat of it, unused)
+            }
+            if (row < n_ff) {
 #pragma unroll
-            for (int r = 0; r < kMmResults; r++) {
-                const uint32_t slot = s_map.out_row[4 * khalf + r];
-                if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
+                for (int r = 0; r < 4 * kJl; r++) {
+                    const uint32_t slot = s_map.out_row[8 * (r >> 2) + 4 * khalf + (r & 3)];
+                    if (slot != 0xffffffffu) mid[static_cast<size_t>(slot) * n_ff + row] = act_mul<false>(accg[r], accu[r]);
+                }
             }
         }
-    }
+    };
+    if (kJ == 1 || live <= 8)  // workgroup-uniform
+        walk(std::integral_constant<int, 1>{});
+    else
+        walk(std::integral_constant<int, kJ>{});
 }
 
 // ---------------------------------------------------------------------------------------------
 // down projection of the re-quantised intermediate, scaled by the route weight.  Grid (row tiles of 128, groups).
 // ---------------------------------------------------------------------------------------------
-template <uint32_t kQuant>
+template <uint32_t kQuant, int kJ>
 __global__ void __launch_bounds__(kGbThreads, 2)
     moe_down_mfma_kernel(const uint8_t *__restrict__ down_all, const uint8_t *__restrict__ down_shared, uint32_t n_routed,
                          const float *__restrict__ mid,
@@ -490,52 +503,60 @@ __global__ void __launch_bounds__(kGbThreads, 2)
     }
     if constexpr (kSix) q6_take(c6);
     __syncthreads();
-    float accf[kMmResults] = {};
-    uint32_t rt = 0, b = 0;
-    for (uint32_t s = 0; s < steps; s++) {
-        uint32_t rtn = rt, bn = b + 1;  // the step after this one; the last step reloads its own block, unused
-        if (bn == nb) {
-            bn = 0;
-            rtn = rt + 1;
-        }
-        if (s + 1 == steps) {
-            rtn = rt;
-            bn = b;
-        }
-        Q5Row n5{};
-        float val[kMmResults];
-        if constexpr (kSix) {
-            q6_request(rtn, bn);
-            TileOps64 aops;
-            tile_ops_load(aops, img.act(b) + arow * kStride + 8 * khalf);
-            q6_block_tile(c6, aops, val);
-        } else {
-            n5 = q45_load_row<kFifth>(block_ptr(rtn, bn), khalf);
-            TileOps128 aops;
-            tile_ops_load(aops, img.act(b) + arow * kStride + 16 * khalf);
-            q45_block_tile<kFifth>(c5, aops, img.dig(b)[lrow], khalf, val);
-        }
-        tile_scale_add(img.dx(b), khalf, val, accf);
-        if constexpr (kSix) q6_take(c6);
-        c5 = n5;
-        if (b + 1 == nb) {  // the row tile is complete
-            const uint32_t row = row_of(rt);
-            if (row < n_embd) {
-#pragma unroll
-                for (int r = 0; r < kMmResults; r++) {
-                    const int t = 4 * khalf + r;
-                    const uint32_t slot = s_map.out_row[t];
-                    // fanout.rs:306-308: the expert's output times the slot's route weight
-                    if (slot != 0xffffffffu)
-                        slot_out[static_cast<size_t>(slot) * n_embd + row] = accf[r] * s_map.scale[t];
-                }
+    // a group of at most eight slots among larger ones finishes only a lane's first four results
+    auto walk = [&](auto jtag) {
+        constexpr int kJl = decltype(jtag)::value;
+        float accf[4 * kJl] = {};
+        uint32_t rt = 0, b = 0;
+        for (uint32_t s = 0; s < steps; s++) {
+            uint32_t rtn = rt, bn = b + 1;  // the step after this one; the last step reloads its own block, unused
+            if (bn == nb) {
+                bn = 0;
+                rtn = rt + 1;
             }
+            if (s + 1 == steps) {
+                rtn = rt;
+                bn = b;
+            }
+            Q5Row n5{};
+            float val[4 * kJl];
+            if constexpr (kSix) {
+                q6_request(rtn, bn);
+                TileOps64 aops;
+                tile_ops_load(aops, img.act(b) + arow * kStride + 8 * khalf);
+                q6_block_tile<kJl>(c6, aops, val);
+            } else {
+                n5 = q45_load_row<kFifth>(block_ptr(rtn, bn), khalf);
+                TileOps128 aops;
+                tile_ops_load(aops, img.act(b) + arow * kStride + 16 * khalf);
+                q45_block_tile<kFifth, kJl>(c5, aops, img.dig(b)[lrow], khalf, val);
+            }
+            tile_scale_add<kJl>(img.dx(b), khalf, val, accf);
+            if constexpr (kSix) q6_take(c6);
+            c5 = n5;
+            if (b + 1 == nb) {  // the row tile is complete
+                const uint32_t row = row_of(rt);
+                if (row < n_embd) {
 #pragma unroll
-            for (int i = 0; i < kMmResults; i++) accf[i] = 0.0f;
+                    for (int r = 0; r < 4 * kJl; r++) {
+                        const int t = 8 * (r >> 2) + 4 * khalf + (r & 3);
+                        const uint32_t slot = s_map.out_row[t];
+                        // fanout.rs:306-308: the expert's output times the slot's route weight
+                        if (slot != 0xffffffffu)
+                            slot_out[static_cast<size_t>(slot) * n_embd + row] = accf[r] * s_map.scale[t];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4 * kJl; i++) accf[i] = 0.0f;
+            }
+            rt = rtn;
+            b = bn;
         }
-        rt = rtn;
-        b = bn;
-    }
+    };
+    if (kJ == 1 || live <= 8)  // workgroup-uniform
+        walk(std::integral_constant<int, 1>{});
+    else
+        walk(std::integral_constant<int, kJ>{});
 }
 
 // raises a kernel's dynamic LDS limit above the default 64 KB, once per kernel (K is a distinct type per kernel only
@@ -553,12 +574,56 @@ bool allow_lds(K kernel, size_t bytes) {
 constexpr size_t kMmLdsLimit = 150 * 1024;
 constexpr size_t kMmGateUpImageLimit = kMmLdsLimit - kMmGateUpStripBytes;
 constexpr size_t kMmQ6DownLdsLimit = kMmLdsLimit - kGbWaves * 32 * kQ6StripStride;
-constexpr uint32_t kMmMinToks = 16;  // rows so long that fewer tokens fit are no batch for this kernel
 
 bool moe_mfma_supported(uint32_t nb_in, uint32_t nb_mid, uint32_t down_quant) {
-    return nb_in >= 1 && nb_mid >= 1 && TileImage<kGbStride128, true>::bytes(nb_in, kMmMinToks) <= kMmGateUpImageLimit &&
-           (down_quant == kQ6K ? TileImage<kGbStride64, false>::bytes(nb_mid, kMmMinToks) <= kMmQ6DownLdsLimit
-                               : TileImage<kGbStride128, true>::bytes(nb_mid, kMmMinToks) <= kMmLdsLimit);
+    return nb_in >= 1 && nb_mid >= 1 && TileImage<kGbStride128, true>::bytes(nb_in, kMoeMfmaMaxGroup) <= kMmGateUpImageLimit &&
+           (down_quant == kQ6K ? TileImage<kGbStride64, false>::bytes(nb_mid, kMoeMfmaMaxGroup) <= kMmQ6DownLdsLimit
+                               : TileImage<kGbStride128, true>::bytes(nb_mid, kMoeMfmaMaxGroup) <= kMmLdsLimit);
+}
+
+namespace {
+struct GateUpPlan {
+    uint32_t waves, tiles_per_wg, wgs;
+};
+// A wave's time is its chain of steps, and the chain is mostly instruction and LDS latency that only another wave on
+// the SIMD hides (without its fills the kernel still takes 40 of its 50 us); a grid of more workgroups than fit at once
+// runs in rounds, and a last round that is partly empty costs as much as a full one.  So: the widest workgroup (six
+// waves = 192 rows, else four = 128) for which merging up to three row tiles into one walk brings the grid down to
+// one workgroup per compute unit, map and image made once per walk.  128 experts x top-8 at 64 tokens (126 groups):
+// four waves 1 / 2 / 3 tiles per workgroup 55.4 / 58.4 / 50.6 us (2 leaves half the units with two workgroups and
+// half with one), six waves x 2 tiles 48.8 us, eight waves x 1 (two rounds) 61.6, twelve waves 67-74.
+GateUpPlan gate_up_plan(uint32_t n_groups, uint32_t max_group, uint32_t n_ff, uint32_t nb_in) {
+    const size_t image = TileImage<kGbStride128, true>::bytes(nb_in, max_group);
+    for (const uint32_t w : {6u, 4u}) {
+        if (w != kGbWaves && w * 2 * kQ4FillBytes + image > kMmLdsLimit) continue;
+        const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
+        const uint32_t t = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * n_groups + 255) / 256);
+        if (t >= 1 && t <= 3 && t <= tiles && (t > 1 || w == 4)) {
+            const uint32_t wgs = (tiles + t - 1) / t * n_groups;
+            if (wgs <= 256) return {w, t, wgs};
+        }
+    }
+    return {kGbWaves, 1, (n_ff + 32 * kGbWaves - 1) / (32 * kGbWaves) * n_groups};
+}
+}  // namespace
+
+// Against moe_few.hip (us a call, this : moe_few).  Its down projection quantises the intermediates itself, one launch of 5 us less, which
+// counts where the experts' weights are read in 30 - 60 us: small calls of more than sixteen groups (fewer leave its one workgroup a unit
+// idle) of up to eight slots, of which a lane finishes four results, Q5_K down projections: 128 x top-8 of 256 x 2304 at 21 tokens 36.7 :
+// 42.7, of 1024 x 1024 at 19 44.9 : 50.7; 512 x 3328 at 21 (2366 blocks) 92.7 : 76.1, 8 x top-2 of 2048 x 1024, Q6_K, at 26 38.2 : 29.1.  With up to
+// sixteen slots where the gate/up kernel's workgroups, all rows of them in use, fill one round, short intermediates: 128 x top-8 of 768 x
+// 2048 at 64 tokens of a uniform router (groups of up to ten) 97 : 104, Q5_K at 57 90.6 : 101.9, four waves of 256 x 2816, Q5_K, 51.3 : 58.2 (256 x
+// 1536, Q6_K, 47.9 : 41.8; 190 workgroups 78.8 : 81.0, 512 rows 66.9 : 64.2, 1536 rows 178 : 177).
+// 1040 random calls of 20 to 300 tokens (7 to 253 experts hit, rows of 3 to 18 blocks, intermediates of 1 to 10): 0.24 % over the better
+// one of the two on average, 24 of them 3 - 13 % behind this kernel (mostly Q5_K, 170 to 238 workgroups), 8 of them 3 - 9 % behind
+// moe_few.hip.
+bool moe_mfma_pays(size_t n_groups, size_t max_group, size_t n_ff, size_t nb_in, size_t nb_mid, uint32_t down_quant) {
+    if (max_group > kMoeMfmaMaxGroup || n_groups <= 16 || n_groups > 65535) return false;
+    if (max_group <= 8 && n_groups * nb_in * nb_mid < 2000) return true;
+    if (nb_mid > 3) return false;
+    const GateUpPlan p = gate_up_plan(static_cast<uint32_t>(n_groups), static_cast<uint32_t>(max_group), static_cast<uint32_t>(n_ff),
+                                      static_cast<uint32_t>(nb_in));
+    return n_ff % (32 * p.waves) == 0 && p.wgs <= 256 && p.wgs >= 240 && (p.waves == 6 || down_quant == kQ5K);
 }
 
 void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, const MoeShared &shared, ActView act,
@@ -566,39 +631,25 @@ void launch_moe_gate_up_mfma(const uint8_t *gate_all, const uint8_t *up_all, con
     if (groups.n_groups == 0 || n_ff == 0) return;
     const uint32_t toks = groups.max_group;
     const size_t image = TileImage<kGbStride128, true>::bytes(nb_in, toks);
-    // A wave's time is its chain of steps, and the chain is mostly instruction and LDS latency that only another wave on
-    // the SIMD hides (without its fills the kernel still takes 40 of its 50 us); a grid of more workgroups than fit at once
-    // runs in rounds, and a last round that is partly empty costs as much as a full one.  So: the widest workgroup (six
-    // waves = 192 rows, else four = 128) for which merging up to three row tiles into one walk brings the grid down to
-    // one workgroup per compute unit, map and image made once per walk.  128 experts x top-8 at 64 tokens (126 groups):
-    // four waves 1 / 2 / 3 tiles per workgroup 55.4 / 58.4 / 50.6 us (2 leaves half the units with two workgroups and
-    // half with one), six waves x 2 tiles 48.8 us, eight waves x 1 (two rounds) 61.6, twelve waves 67-74.
-    int waves = kGbWaves;
-    uint32_t tiles_per_wg = 1;
-    for (const int w : {6, 4}) {
-        if (w != kGbWaves && static_cast<size_t>(w) * 2 * kQ4FillBytes + image > kMmLdsLimit) continue;
-        const uint32_t tiles = (n_ff + 32 * w - 1) / (32 * w);
-        const uint32_t t = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * groups.n_groups + 255) / 256);
-        if (t >= 1 && t <= 3 && t <= tiles && static_cast<uint64_t>((tiles + t - 1) / t) * groups.n_groups <= 256 &&
-            (t > 1 || w == 4)) {
-            waves = w;
-            tiles_per_wg = t;
-            break;
-        }
-    }
+    const GateUpPlan plan = gate_up_plan(groups.n_groups, toks, n_ff, nb_in);
+    const uint32_t waves = plan.waves, tiles_per_wg = plan.tiles_per_wg;
     const size_t lds = static_cast<size_t>(waves) * 2 * kQ4FillBytes + image;
     const uint32_t rows_per_wg = 32 * waves, row_tiles = (n_ff + rows_per_wg - 1) / rows_per_wg;
     const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
-#define RNB_LAUNCH_GUW(W)                                                                                            \
-    if (!allow_lds<W>(moe_gate_up_mfma_kernel<W>, kMmLdsLimit)) return;                                              \
-    hipLaunchKernelGGL(moe_gate_up_mfma_kernel<W>, dim3(wgs_x, groups.n_groups), dim3(kWave * W), lds, stream,       \
+#define RNB_LAUNCH_GUW(J, W)                                                                                         \
+    if (!allow_lds<J * 16 + W>(moe_gate_up_mfma_kernel<J, W>, kMmLdsLimit)) return;                                  \
+    hipLaunchKernelGGL((moe_gate_up_mfma_kernel<J, W>), dim3(wgs_x, groups.n_groups), dim3(kWave * W), lds, stream,  \
                        gate_all, up_all, shared.gate, shared.up, shared.n_routed, act.qs, act.d, act.digits,         \
                        groups.expert, groups.start, groups.sorted_slot, groups.sorted_token, mid, n_ff, nb_in, toks, \
                        tiles_per_wg)
-    if (waves == 6) {
-        RNB_LAUNCH_GUW(6);
+    if (waves == 6 && toks <= 8) {
+        RNB_LAUNCH_GUW(1, 6);
+    } else if (waves == 6) {
+        RNB_LAUNCH_GUW(2, 6);
+    } else if (toks <= 8) {
+        RNB_LAUNCH_GUW(1, kGbWaves);
     } else {
-        RNB_LAUNCH_GUW(kGbWaves);
+        RNB_LAUNCH_GUW(2, kGbWaves);
     }
 #undef RNB_LAUNCH_GUW
 }
@@ -615,11 +666,17 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
     while (tiles_per_wg < 4 && static_cast<uint64_t>((row_tiles + tiles_per_wg - 1) / tiles_per_wg) * groups.n_groups > 768)
         tiles_per_wg *= 2;
     const uint32_t wgs_x = (row_tiles + tiles_per_wg - 1) / tiles_per_wg;
-#define RNB_LAUNCH_DM(Q, LDS)                                                                                        \
-    if (!allow_lds<static_cast<int>(Q)>(moe_down_mfma_kernel<Q>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
-    hipLaunchKernelGGL(moe_down_mfma_kernel<Q>, dim3(wgs_x, groups.n_groups), dim3(kGbThreads), LDS, stream,          \
+#define RNB_LAUNCH_DMJ(Q, J, LDS)                                                                                     \
+    if (!allow_lds<static_cast<int>(Q) * 8 + J>(moe_down_mfma_kernel<Q, J>, Q == kQ6K ? kMmQ6DownLdsLimit : kMmLdsLimit)) return; \
+    hipLaunchKernelGGL((moe_down_mfma_kernel<Q, J>), dim3(wgs_x, groups.n_groups), dim3(kGbThreads), LDS, stream,     \
                        down_all, shared.down, shared.n_routed, mid, groups.expert, groups.start, groups.sorted_slot, \
                        slot_route, slot_out, n_embd, nb_mid, tiles_per_wg, toks)
+#define RNB_LAUNCH_DM(Q, LDS)                                                                                        \
+    if (toks <= 8) {                                                                                                  \
+        RNB_LAUNCH_DMJ(Q, 1, LDS);                                                                                    \
+    } else {                                                                                                          \
+        RNB_LAUNCH_DMJ(Q, 2, LDS);                                                                                    \
+    }
     if (down_quant == kQ6K) {
         RNB_LAUNCH_DM(kQ6K, (TileImage<kGbStride64, false>::bytes(nb_mid, toks)));
     } else if (down_quant == kQ5K) {
@@ -628,6 +685,7 @@ void launch_moe_down_mfma(const uint8_t *down_all, const MoeShared &shared, uint
         RNB_LAUNCH_DM(kQ4K, (TileImage<kGbStride128, true>::bytes(nb_mid, toks)));
     }
 #undef RNB_LAUNCH_DM
+#undef RNB_LAUNCH_DMJ
 }
 
 }  // namespace rnb

@@ -1,6 +1,7 @@
 """Routed experts of a batch on the matrix cores: on the few-token GEMM's tiles (moe_few.hip: groups of every size around the 16- and
-32-slot tiles, row tiles with remainders, few and many workgroups, a shared expert) and, small calls of groups of up to eight slots, in
-moe_mfma.hip.  Against the oracle; outputs outside the plain per-row tolerance must be whole re-quantisation flips (oracle/flips.py)."""
+32-slot tiles, row tiles with remainders, few and many workgroups, a shared expert) and in moe_mfma.hip (groups of up to eight and up
+to sixteen slots).  Against the oracle; outputs outside the plain per-row tolerance must be whole re-quantisation flips
+(oracle/flips.py)."""
 import numpy as np
 import pytest
 
@@ -70,4 +71,18 @@ def test_moe_tiles_of_few_tokens(rnb, oracle, tokens, groups, n_ff, n_embd, shar
     (18, [1, 2, 3, 2] * 27, 256, 4352, Q5_K),
 ])
 def test_moe_small_groups(rnb, oracle, tokens, groups, n_ff, n_embd, down_quant):
+    _check(rnb, oracle, tokens, groups, n_ff, n_embd, False, down_quant)
+
+
+# groups of up to sixteen slots whose gate/up workgroups fill one round, 240 to 256 of them with all rows in use
+@pytest.mark.parametrize("tokens,groups,n_ff,n_embd,down_quant", [
+    (16, [16, 1, 9, 8, 2, 3] * 20, 768, 512, Q4_K),           # six waves, two row tiles a workgroup, the least groups
+    (19, [9, 12, 1, 5] * 32, 768, 768, Q5_K),                 # ... the most
+    (16, [1, 2, 3, 9] * 31, 768, 256, Q6_K),
+    (16, [16, 7, 15, 2] * 31, 256, 1280, Q5_K),               # four waves, a row tile a workgroup
+    (24, [16, 3] * 31, 512, 512, Q5_K),                       # ... four row tiles a group
+    (17, [10, 1, 3, 2] * 30, 256, 4352, Q5_K),                # four row tiles a workgroup in the down kernel, two in its last
+    (17, [17, 1, 9, 8, 2, 3] * 20, 768, 512, Q6_K),           # a slot too many
+])
+def test_moe_groups_of_up_to_sixteen(rnb, oracle, tokens, groups, n_ff, n_embd, down_quant):
     _check(rnb, oracle, tokens, groups, n_ff, n_embd, False, down_quant)
